@@ -18,7 +18,7 @@
 //   scatter  re-reads each block in chunks, sorts a chunk by tile in LDS and
 //            writes each tile's run of it to the tile's region (consecutive
 //            lanes, consecutive addresses)
-//   accum    per tile, one workgroup per chunk of up to kAccumChunk of the
+//   accum    per tile, one workgroup per chunk of up to 2^17 of the
 //            tile's records: counts in LDS, then one add per cell (an
 //            atomic one where chunks share the tile)
 // A tile is kBinTileCells consecutive cells (dimension 0 fastest), whose
@@ -70,57 +70,99 @@ __global__ void __launch_bounds__(kBinBlock)
 }
 
 // column scan: for tile t, hist[b][t] becomes the records of tiles t in
-// blocks before b (exclusive), total[t] the tile's records
-__global__ void __launch_bounds__(kBinBlock)
+// blocks before b (exclusive), total[t] the tile's records.  A workgroup
+// takes kScanTiles neighbouring tiles (whole lines of a row) and splits the
+// blocks among kScanParts groups of lanes: their sums, then the running
+// sums from each part's start.  (A lane per tile walked all blocks one
+// after another: 90 us for 4096 tiles of 1024 blocks, now 10.)
+constexpr int kScanTiles = 32, kScanParts = 32;
+
+__global__ void __launch_bounds__(kScanTiles * kScanParts)
     bin_colscan_kernel(unsigned *hist, int nblocks, int ntiles, unsigned *total)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ unsigned part[kScanParts][kScanTiles];
+    const int tx = (int)threadIdx.x & (kScanTiles - 1), ty = (int)threadIdx.x / kScanTiles;
+    const int t = (int)blockIdx.x * kScanTiles + tx;
+    const int per = (nblocks + kScanParts - 1) / kScanParts;
+    const int b0 = ty * per, b1 = min(nblocks, b0 + per);
+    unsigned *col = hist + t; // (read and written for t < ntiles only)
+    unsigned sum = 0;
+    if (t < ntiles)
+        for (int b = b0; b < b1; b += kBinUnroll) {
+            unsigned v[kBinUnroll];
+#pragma unroll
+            for (int j = 0; j < kBinUnroll; ++j)
+                v[j] = b + j < b1 ? col[(size_t)(b + j) * (size_t)ntiles] : 0u;
+#pragma unroll
+            for (int j = 0; j < kBinUnroll; ++j)
+                sum += v[j];
+        }
+    part[ty][tx] = sum;
+    __syncthreads();
+    unsigned run = 0;
+    for (int k = 0; k < kScanParts; ++k) {
+        const unsigned v = part[k][tx];
+        run += k < ty ? v : 0u;
+    }
     if (t >= ntiles)
         return;
-    unsigned run = 0;
-    for (int b0 = 0; b0 < nblocks; b0 += kBinUnroll) {
+    if (ty == kScanParts - 1)
+        total[t] = run + sum;
+    for (int b = b0; b < b1; b += kBinUnroll) {
         unsigned v[kBinUnroll];
 #pragma unroll
         for (int j = 0; j < kBinUnroll; ++j)
-            v[j] = b0 + j < nblocks ? hist[(size_t)(b0 + j) * (size_t)ntiles + t] : 0u;
+            v[j] = b + j < b1 ? col[(size_t)(b + j) * (size_t)ntiles] : 0u;
 #pragma unroll
         for (int j = 0; j < kBinUnroll; ++j)
-            if (b0 + j < nblocks) {
-                hist[(size_t)(b0 + j) * (size_t)ntiles + t] = run;
+            if (b + j < b1) {
+                col[(size_t)(b + j) * (size_t)ntiles] = run;
                 run += v[j];
             }
     }
-    total[t] = run;
 }
 
-// exclusive scan of the tile totals into start[0..ntiles] (one workgroup)
-__global__ void __launch_bounds__(1024) bin_tilescan_kernel(const unsigned *total, int ntiles,
-                                                           unsigned *start)
+// exclusive scans over the tiles (one workgroup): of their records, into
+// start[0..ntiles], and of their accumulation chunks of `chunk` records,
+// into cstart[0..ntiles]
+__global__ void __launch_bounds__(1024)
+    bin_tilescan_kernel(const unsigned *total, int ntiles, unsigned chunk, unsigned *start,
+                        unsigned *cstart)
 {
-    __shared__ unsigned part[1024];
+    __shared__ unsigned part[1024], cpart[1024];
+    const int tid = (int)threadIdx.x;
     const int per = (ntiles + (int)blockDim.x - 1) / (int)blockDim.x;
-    const int t0 = threadIdx.x * per;
-    unsigned s = 0;
+    const int t0 = tid * per;
+    unsigned s = 0, c = 0;
     for (int k = 0; k < per; ++k)
-        if (t0 + k < ntiles)
+        if (t0 + k < ntiles) {
             s += total[t0 + k];
-    part[threadIdx.x] = s;
+            c += (total[t0 + k] + chunk - 1) / chunk;
+        }
+    part[tid] = s;
+    cpart[tid] = c;
     __syncthreads();
     // Hillis-Steele inclusive scan of the per-thread sums
     for (int off = 1; off < (int)blockDim.x; off <<= 1) {
-        const unsigned v = threadIdx.x >= (unsigned)off ? part[threadIdx.x - off] : 0u;
+        const unsigned v = tid >= off ? part[tid - off] : 0u;
+        const unsigned w = tid >= off ? cpart[tid - off] : 0u;
         __syncthreads();
-        part[threadIdx.x] += v;
+        part[tid] += v;
+        cpart[tid] += w;
         __syncthreads();
     }
-    unsigned run = threadIdx.x ? part[threadIdx.x - 1] : 0u;
+    unsigned run = tid ? part[tid - 1] : 0u, crun = tid ? cpart[tid - 1] : 0u;
     for (int k = 0; k < per; ++k)
         if (t0 + k < ntiles) {
             start[t0 + k] = run;
+            cstart[t0 + k] = crun;
             run += total[t0 + k];
+            crun += (total[t0 + k] + chunk - 1) / chunk;
         }
-    if (threadIdx.x == blockDim.x - 1)
-        start[ntiles] = part[threadIdx.x];
+    if (tid == (int)blockDim.x - 1) {
+        start[ntiles] = part[tid];
+        cstart[ntiles] = cpart[tid];
+    }
 }
 
 // Each block writes its records to their tiles' regions: the k-th record of
@@ -243,18 +285,9 @@ __device__ __forceinline__ unsigned tile_word(unsigned c)
 // Tiles take very different shares of the records (the tetrahedron's
 // lowest slices hold thousands of occupied cells, its highest a few), and
 // one workgroup per tile left the device waiting on the largest.  So a tile
-// is accumulated in chunks of at most kAccumChunk records, a workgroup
-// each: chunks[t] per tile, then their exclusive scan gives tile t's work
-// items cstart[t] .. cstart[t + 1].
-constexpr unsigned kAccumChunk = 1u << 17;
-
-__global__ void __launch_bounds__(kBinBlock)
-    bin_chunks_kernel(const unsigned *start, int ntiles, unsigned *chunks)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < ntiles)
-        chunks[t] = (start[t + 1] - start[t] + kAccumChunk - 1) / kAccumChunk;
-}
+// is accumulated in chunks of at most `chunk` records (bin_accum_chunk), a
+// workgroup each: the scan of their numbers gives tile t's work items
+// cstart[t] .. cstart[t + 1].
 
 // work item w: chunk w - cstart[t] of the tile t whose items hold w.  The
 // chunk's counts go to LDS, then each cell's count into the buffer: a plain
@@ -263,11 +296,12 @@ __global__ void __launch_bounds__(kBinBlock)
 template <typename CT>
 __global__ void __launch_bounds__(1024)
     bin_accum_kernel(const unsigned *sorted, const unsigned *start, const unsigned *cstart,
-                     int ntiles, int tile_bits, unsigned long long cells, CT *buf)
+                     int ntiles, int tile_bits, unsigned long long cells, unsigned chunk,
+                     const unsigned *skip, CT *buf)
 {
     extern __shared__ unsigned cnt[];
     const unsigned w = blockIdx.x;
-    if (w >= cstart[ntiles])
+    if (w >= cstart[ntiles] || (skip && *skip))
         return; // past the last work item (uniform across the workgroup)
     // the tile: the last t with cstart[t] <= w (tiles without records have
     // no items, so their cstart equals the next tile's)
@@ -282,8 +316,8 @@ __global__ void __launch_bounds__(1024)
     const int t = lo;
     const unsigned k = w - cstart[t];
     const bool shared = cstart[t + 1] - cstart[t] > 1;
-    const unsigned s0 = start[t] + k * kAccumChunk;
-    const unsigned s1 = min(start[t + 1], s0 + kAccumChunk);
+    const unsigned s0 = start[t] + k * chunk;
+    const unsigned s1 = min(start[t + 1], s0 + chunk);
     const unsigned tile = 1u << tile_bits;
     const unsigned long long c0 = (unsigned long long)t << tile_bits;
     const unsigned long long left = cells - c0;
@@ -448,13 +482,13 @@ __global__ void __launch_bounds__(1024)
     bin_accum_colour_kernel(const unsigned *sorted, const PR *pay_sorted,
                             unsigned long long stride, int nr, const unsigned *start,
                             const unsigned *cstart, int ntiles, unsigned long long cells,
-                            CT *buf)
+                            unsigned chunk, const unsigned *skip, CT *buf)
 {
     extern __shared__ unsigned long long lds64[];
     double *col = reinterpret_cast<double *>(lds64);                 // [nr][kColourTile]
     unsigned *cnt = reinterpret_cast<unsigned *>(col + 4 * kColourTile); // [kColourTile]
     const unsigned w = blockIdx.x;
-    if (w >= cstart[ntiles])
+    if (w >= cstart[ntiles] || (skip && *skip))
         return;
     int lo = 0, hi = ntiles - 1;
     while (lo < hi) {
@@ -467,8 +501,8 @@ __global__ void __launch_bounds__(1024)
     const int t = lo;
     const unsigned k = w - cstart[t];
     const bool shared = cstart[t + 1] - cstart[t] > 1;
-    const unsigned s0 = start[t] + k * kAccumChunk;
-    const unsigned s1 = min(start[t + 1], s0 + kAccumChunk);
+    const unsigned s0 = start[t] + k * chunk;
+    const unsigned s1 = min(start[t + 1], s0 + chunk);
     const unsigned long long c0 = (unsigned long long)t * kColourTile;
     const unsigned long long left = cells - c0;
     const unsigned ncell = left < (unsigned long long)kColourTile ? (unsigned)left : kColourTile;
@@ -521,29 +555,54 @@ int grid_for(unsigned long long n, int block)
 
 } // namespace
 
+// records of a histogram and scatter block: 2^18, less for renders of few
+// records, so that they spread over the device (about 512 blocks)
+static unsigned long long bin_block_records(unsigned long long records)
+{
+    unsigned long long per = 1ull << 13;
+    while (per < kBinRecordsPerBlock && per * 512 < records)
+        per <<= 1;
+    return per;
+}
+
+// records of an accumulation chunk: 2^17, less for renders of few records
+static unsigned bin_accum_chunk(unsigned long long records)
+{
+    unsigned chunk = 1u << 12;
+    while (chunk < (1u << 17) && (unsigned long long)chunk * 1024 < records)
+        chunk <<= 1;
+    return chunk;
+}
+
 size_t bin_scratch_hist_words(unsigned long long records, int ntiles)
 {
-    const unsigned long long blocks = (records + kBinRecordsPerBlock - 1) / kBinRecordsPerBlock;
-    return (size_t)std::max<unsigned long long>(blocks, 1) * (size_t)ntiles;
+    // (a render of fewer records may take more of its smaller blocks: at
+    // most 512 while they are smaller than 2^18)
+    const unsigned long long blocks =
+        std::max<unsigned long long>(512, (records + kBinRecordsPerBlock - 1) / kBinRecordsPerBlock);
+    return (size_t)blocks * (size_t)ntiles;
 }
 
 int launch_bin_accumulate(const BinScratch &b, unsigned long long n_records,
                           unsigned long long cells, void *buf, int word_bytes, int r,
-                          int real_bytes, hipStream_t s)
+                          int real_bytes, hipStream_t s, const unsigned *skip)
 {
     const int tile_bits = r > 0 ? kBinTileBitsColour : kBinTileBits;
     const int ntiles = (int)((cells + (1ull << tile_bits) - 1) >> tile_bits);
     if (ntiles > kBinMaxTiles || n_records > 0xFFFFFFFFull || r < 0 || r > 4 ||
         (r > 0 && (real_bytes != 4 && real_bytes != 8)))
         return (int)hipErrorInvalidValue;
-    const unsigned long long per = kBinRecordsPerBlock;
+    const unsigned long long per = bin_block_records(n_records);
+    const unsigned chunk = bin_accum_chunk(n_records);
     const int nblocks = (int)std::max<unsigned long long>(1, (n_records + per - 1) / per);
     const size_t hist_lds = sizeof(unsigned) * (size_t)ntiles;
     hipLaunchKernelGGL(bin_hist_kernel, dim3(nblocks), dim3(kBinBlock), hist_lds, s, b.rec,
                        n_records, per, tile_bits, ntiles, b.hist);
-    hipLaunchKernelGGL(bin_colscan_kernel, dim3((ntiles + kBinBlock - 1) / kBinBlock),
-                       dim3(kBinBlock), 0, s, b.hist, nblocks, ntiles, b.total);
-    hipLaunchKernelGGL(bin_tilescan_kernel, dim3(1), dim3(1024), 0, s, b.total, ntiles, b.start);
+    hipLaunchKernelGGL(bin_colscan_kernel, dim3((ntiles + kScanTiles - 1) / kScanTiles),
+                       dim3(kScanTiles * kScanParts), 0, s, b.hist, nblocks, ntiles, b.total);
+    unsigned *cstart = b.total + ntiles;
+    hipLaunchKernelGGL(bin_tilescan_kernel, dim3(1), dim3(1024), 0, s, b.total, ntiles, chunk,
+                       b.start, cstart);
     const unsigned long long stride = b.capacity;
     if (r == 0) {
         if (ntiles <= 4096)
@@ -571,23 +630,18 @@ int launch_bin_accumulate(const BinScratch &b, unsigned long long n_records,
                                (const float *)b.pay, n_records, per, tile_bits, ntiles, b.hist,
                                b.start, b.sorted, (float *)b.pay_sorted, stride, r);
     }
-    // accumulation work items: per tile, chunks of at most kAccumChunk
-    // records (at most ntiles + n_records / kAccumChunk items in all)
-    unsigned *chunks = b.total, *cstart = b.total + ntiles + 1;
-    hipLaunchKernelGGL(bin_chunks_kernel, dim3((ntiles + kBinBlock - 1) / kBinBlock),
-                       dim3(kBinBlock), 0, s, b.start, ntiles, chunks);
-    hipLaunchKernelGGL(bin_tilescan_kernel, dim3(1), dim3(1024), 0, s, chunks, ntiles, cstart);
-    const unsigned items = (unsigned)((unsigned long long)ntiles + n_records / kAccumChunk);
+    // accumulation work items (at most ntiles + n_records / chunk in all)
+    const unsigned items = (unsigned)((unsigned long long)ntiles + n_records / chunk);
     if (r == 0) {
         const size_t tile_lds = sizeof(unsigned) << kBinTileBits;
         if (word_bytes == 8)
             hipLaunchKernelGGL((bin_accum_kernel<unsigned long long>), dim3(items), dim3(1024),
                                tile_lds, s, b.sorted, b.start, cstart, ntiles, tile_bits, cells,
-                               (unsigned long long *)buf);
+                               chunk, skip, (unsigned long long *)buf);
         else
             hipLaunchKernelGGL((bin_accum_kernel<unsigned>), dim3(items), dim3(1024), tile_lds,
                                s, b.sorted, b.start, cstart, ntiles, tile_bits, cells,
-                               (unsigned *)buf);
+                               chunk, skip, (unsigned *)buf);
         return (int)hipGetLastError();
     }
     // colour: 8-byte words hold u64 counts and f64 sums, 4-byte words u32
@@ -596,17 +650,17 @@ int launch_bin_accumulate(const BinScratch &b, unsigned long long n_records,
         hipLaunchKernelGGL((bin_accum_colour_kernel<unsigned long long, double, double>),
                            dim3(items), dim3(1024), accum_colour_lds(), s, b.sorted,
                            (const double *)b.pay_sorted, stride, r, b.start, cstart, ntiles,
-                           cells, (unsigned long long *)buf);
+                           cells, chunk, skip, (unsigned long long *)buf);
     else if (word_bytes == 8)
         hipLaunchKernelGGL((bin_accum_colour_kernel<unsigned long long, double, float>),
                            dim3(items), dim3(1024), accum_colour_lds(), s, b.sorted,
                            (const float *)b.pay_sorted, stride, r, b.start, cstart, ntiles,
-                           cells, (unsigned long long *)buf);
+                           cells, chunk, skip, (unsigned long long *)buf);
     else
         hipLaunchKernelGGL((bin_accum_colour_kernel<unsigned, float, float>), dim3(items),
                            dim3(1024), accum_colour_lds(), s, b.sorted,
                            (const float *)b.pay_sorted, stride, r, b.start, cstart, ntiles,
-                           cells, (unsigned *)buf);
+                           cells, chunk, skip, (unsigned *)buf);
     return (int)hipGetLastError();
 }
 

@@ -109,6 +109,17 @@ struct Stream {
     }
 };
 
+// Pointers into device memory.  A pointer read from memory (the kernels'
+// arguments) is a generic one to the compiler: its stores are FLAT
+// instructions, which count as LDS traffic too, so that the next wait for
+// an LDS or scalar read waits for the store to reach memory.  These are
+// plain global ones.
+template <typename T> using global_ptr = T __attribute__((address_space(1))) *;
+template <typename T> __device__ __forceinline__ global_ptr<T> as_global(T *p)
+{
+    return (global_ptr<T>)p;
+}
+
 // randNum (flame_rng.hpp:67-87): top 53 bits over 2^53 in double, top 24
 // bits over 2^24 in float; both exact
 __device__ __forceinline__ double rand_from_word(uint64_t w, double)

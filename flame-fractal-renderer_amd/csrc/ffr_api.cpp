@@ -96,6 +96,14 @@ struct ffr_renderer {
     bool chain_diag = false;    // ... and that matrix is diagonal
     size_t chain_lds = 0;       // its LDS bytes
     int chain_per_cu = 0;       // FFR_CHAIN_PER_CU: its walkers-per-CU limit (0: the build's)
+    // split walkers apply (no variation draws words, at most four colour
+    // dimensions, a rate of contraction that is known or to be expected);
+    // the iterations a segment runs before its first, doubled when too many
+    // segments of a render entered with another state than the walker's
+    bool split_ok = false;
+    int split_warm = 0;
+    bool last_split = false;
+    uint64_t last_split_segments = 0;
     size_t lds_bytes = 0;
     // buffer
     void *dbuf = nullptr;
@@ -151,6 +159,8 @@ struct ffr_renderer {
     // FFR_BINNED overrides.  Its records, walker states and per-pass
     // arguments are allocated on the first binned render and kept.
     int bin_pref = -1;
+    // split walkers: -1 chosen per render, 0 off (FFR_SPLIT)
+    int split_pref = -1;
     BinScratch bin;
     size_t bin_pay_bytes = 0; // bytes of bin.pay (and of bin.pay_sorted)
     // a colour flame whose renders made at least kBinColourAtomics global
@@ -191,6 +201,75 @@ static int pick_variation_set(const uint32_t ts[4])
             basic = false;
     }
     return linear_only ? 0 : (basic ? 1 : 2);
+}
+
+// Split walkers: how many iterations two trajectories of the flame that draw
+// the same words take to become equal bit for bit.  A map that shrinks
+// distances by 2^-c on average takes (mantissa bits + a few) / c; the margin
+// of 24 covers the spread over trajectories.  For linear flames c comes from
+// the maps' largest singular values; other flames are taken to halve a
+// distance per iteration (the random flames measured shrink it faster), and
+// the device reports where that was wrong.  The colour blend keeps 1 - speed
+// of the old colour.  0: the flame does not contract enough.
+constexpr int kSplitWarmMax = 512;
+
+template <typename R> static int split_warm_iterations(const DeviceFlame<R> &d, bool linear)
+{
+    const double bits = (sizeof(R) == 8 ? 53.0 : 24.0) + 24.0;
+    const int n = d.dims;
+    double map_rate = 0.0, colour_rate = 0.0, before = 0.0;
+    for (int x = 0; x < d.nxf; ++x) {
+        const double w = (x + 1 < d.nxf ? (double)d.cw[(size_t)x] : 1.0) - before;
+        before += w;
+        const R *X = d.table.data() + d.xf0 + (size_t)x * (size_t)d.lay.stride;
+        if (d.r > 0 && X[d.lay.has_color] != (R)0) {
+            const double keep = std::fabs(1.0 - (double)X[d.lay.speed]);
+            colour_rate += w * std::min(20.0, -std::log2(std::max(keep, 1e-6)));
+        }
+        if (!linear)
+            continue;
+        double wsum = 0.0;
+        for (size_t s = 0; s < d.slot_type.size(); ++s)
+            if (d.masks[(size_t)x] >> s & 1ull)
+                wsum += (double)d.table[(size_t)(d.slot_off[s] + x * d.slot_stride[s])];
+        double m[9], mtm[9], v[3] = {1.0, 0.7, 0.4};
+        for (int i = 0; i < n; ++i)
+            for (int j = 0; j < n; ++j) {
+                m[i * n + j] = 0.0;
+                for (int k = 0; k < n; ++k)
+                    m[i * n + j] += (double)X[d.lay.postA + i * n + k] * wsum *
+                                    (double)X[d.lay.preA + k * n + j];
+            }
+        for (int i = 0; i < n; ++i)
+            for (int j = 0; j < n; ++j) {
+                mtm[i * n + j] = 0.0;
+                for (int k = 0; k < n; ++k)
+                    mtm[i * n + j] += m[k * n + i] * m[k * n + j];
+            }
+        // the largest eigenvalue by power iteration
+        double norm = 0.0;
+        for (int it = 0; it < 32; ++it) {
+            double u[3] = {0, 0, 0};
+            norm = 0.0;
+            for (int i = 0; i < n; ++i) {
+                for (int j = 0; j < n; ++j)
+                    u[i] += mtm[i * n + j] * v[j];
+                norm = std::max(norm, std::fabs(u[i]));
+            }
+            if (!(norm > 1e-300) || !std::isfinite(norm))
+                break;
+            for (int i = 0; i < n; ++i)
+                v[i] = u[i] / norm;
+        }
+        if (!std::isfinite(norm))
+            return 0;
+        map_rate += w * std::min(20.0, -0.5 * std::log2(std::max(norm, 1e-12)));
+    }
+    double rate = linear ? map_rate : 1.0;
+    if (d.r > 0)
+        rate = std::min(rate, colour_rate);
+    const double k = rate > 0.0 ? std::ceil(bits / rate) : 1e9;
+    return k <= (double)kSplitWarmMax ? std::max((int)k, 8) : 0;
 }
 
 template <typename R>
@@ -271,6 +350,14 @@ static int setup_tables(ffr_renderer *r, const DeviceFlame<R> &d)
                                     chain_build_sh(r->chain_shared, r->chain_post_id, slots));
     if (r->chain_lds > (size_t)max_lds)
         r->chain_ok = false;
+    r->split_ok = d.r <= 4 && d.nxf > 0;
+    for (int t : d.slot_type)
+        r->split_ok = r->split_ok && variation_draws(t, d.dims) == 0;
+    for (int t : d.fin_type)
+        r->split_ok = r->split_ok && variation_draws(t, d.dims) == 0;
+    if (r->split_ok)
+        r->split_warm = split_warm_iterations(d, r->vs == 0);
+    r->split_ok = r->split_ok && r->split_warm > 0;
     r->nxf = d.nxf;
     r->order = d.order;
     return FFR_OK;
@@ -361,6 +448,8 @@ int ffr_create(const char *flame_json, size_t len, const ffr_options *opt_in,
         r->bin_pref = opt.binned < 0 ? -1 : (opt.binned ? 1 : 0);
         if (const char *e = std::getenv("FFR_BINNED"))
             r->bin_pref = std::atoi(e);
+        if (const char *e = std::getenv("FFR_SPLIT"))
+            r->split_pref = std::atoi(e) ? -1 : 0;
         r->compiled_pref = opt.compiled < 0 ? -1 : (opt.compiled ? 1 : 0);
         if (const char *e = std::getenv("FFR_CHAIN_PER_CU"))
             r->chain_per_cu = std::atoi(e);
@@ -395,12 +484,14 @@ int ffr_create(const char *flame_json, size_t len, const ffr_options *opt_in,
     rp->stream = rp->own_stream;
     HIP_TRY_D(hipEventCreate(&rp->ev0));
     HIP_TRY_D(hipEventCreate(&rp->ev1));
-    HIP_TRY_D(hipMalloc(&rp->dstats, sizeof(DevStats)));
-    HIP_TRY_D(hipMalloc(&rp->dxf, sizeof(unsigned long long) * (size_t)std::max(rp->nxf, 1)));
+    HIP_TRY_D(hipMalloc(&rp->dstats, (1 + kSplitSlots) * sizeof(DevStats)));
+    HIP_TRY_D(hipMalloc(&rp->dxf, 2 * sizeof(unsigned long long) * (size_t)std::max(rp->nxf, 1)));
     HIP_TRY_D(hipMalloc(&rp->dbv_xfs, sizeof(unsigned long long) * rp->opt.bad_value_cap));
     HIP_TRY_D(hipMalloc(&rp->dbv_pts, sizeof(double) * 3 * rp->opt.bad_value_cap));
     HIP_TRY_D(hipMalloc(&rp->dhist, sizeof(unsigned long long) * 3));
-    HIP_TRY_D(hipMalloc(&rp->dargs, std::max(sizeof(WalkArgs<double>), sizeof(WalkArgs<float>))));
+    // (two: a split launch's and those of the launch behind it)
+    HIP_TRY_D(hipMalloc(&rp->dargs,
+                        2 * std::max(sizeof(WalkArgs<double>), sizeof(WalkArgs<float>))));
     // hints start empty: a tag no geometry has
     HIP_TRY_D(hipMalloc(&rp->dhot, sizeof(unsigned) * (1 + (size_t)kHotSlots)));
     HIP_TRY_D(hipMemsetAsync(rp->dhot, 0xFF, sizeof(unsigned) * (1 + (size_t)kHotSlots),
@@ -545,12 +636,14 @@ struct LaunchShape {
     int block = 0;      // lanes per workgroup, 0 chosen
     int task_rounds = 1; // walkers per lane in one workgroup task
     int bin = -1;       // binned accumulation (single renders): -1 chosen, 0 off, 1 on
+    int split = 0;      // split walkers (single renders): -1 chosen, 0 off
 };
 
 static LaunchShape renderer_shape(const ffr_renderer *r)
 {
     LaunchShape sh;
     sh.bin = r->bin_pref;
+    sh.split = r->split_pref;
     sh.cache = r->cache_pref;
     sh.cache_kb = r->cache_kb;
     sh.block = r->block_pref;
@@ -561,6 +654,8 @@ static LaunchShape renderer_shape(const ffr_renderer *r)
 struct LaunchPlan {
     bool chain = false; // one walker per wave (chain_kernel)
     bool bin = false;   // binned accumulation (walk_bin_kernel + bin_kernels)
+    int split_log2 = 0; // split walkers: log2 of the segments per walker (0: not split)
+    uint64_t split_len = 0;     // iterations per segment
     bool cache = false;
     int block = 256;
     int grid = 1;
@@ -573,6 +668,52 @@ static size_t table_lds(const ffr_renderer *r)
 {
     const int rb = r->mode == MODE_F64_U64 ? 8 : 4;
     return cache_lds_offset(r->tab.tab_reals, rb, r->nxf);
+}
+
+// Split walkers (split_kernel.inc): renders of few walkers, whose unsplit
+// launches are bound by the chain of one walker's iterations, and without
+// the LDS cell cache (off below 64 walkers per CU) by atomics on hot cells.
+// A walker is split into a power of two of segments, as many as fill the
+// device (4 waves per SIMD; measured at 2^26 samples of 1024 walkers: 65536
+// lanes 3.9 ms, 131072 2.9, 262144 2.6, 524288 2.6) while a segment keeps 16
+// iterations (2^20 samples: 8 iterations 0.29-0.33 ms, 16 0.26-0.29, 64
+// 0.33, 256 0.72).  Kernel time of one render, unsplit then split:
+//   256^2 colour flame, 1024 walkers x 1024, FP32            8.8 -> 0.22 ms
+//   1024^2 colour flame, 1024 walkers x 65536, FP32        145   -> 2.6 ms
+//   Sierpinski 1024^2, 1024 x 65536, FP64 (wave per walker)  4.8 -> 1.1 ms
+//   3-D linear flame, 1892 walkers x 1024, FP32              5.4 -> 0.26 ms
+// The smallest of the renders tried, 1400 walkers x 1024 of a triangle, goes
+// from 0.30 to 0.20 ms.
+static void split_plan(const ffr_renderer *r, uint64_t walkers, uint64_t batch,
+                       const LaunchShape &sh, bool chain, LaunchPlan &p)
+{
+    const int ncol = r->spec.color_dims;
+    if (sh.split >= 0 || !r->split_ok || sh.cache >= 0 || sh.block > 0 || sh.bin >= 0)
+        return;
+    if (!chain && (r->compiled_pref > 0 || walkers >= (uint64_t)r->cu_count * 64u))
+        return;
+    if (r->cells >= (ncol > 0 ? (1ull << 25) : (1ull << 28)))
+        return;
+    // (float colour sums of 4-byte words keep the per-sample float adds of
+    // the unsplit kernels: added in double per tile they come out closer to
+    // the true sums, but elsewhere than the float build's own)
+    if (ncol > 0 && r->word_bytes == 4)
+        return;
+    const uint64_t lanes = (uint64_t)r->cu_count * 1024u;
+    int log2s = 0;
+    while (log2s < kSplitMaxLog2 && (walkers << (log2s + 1)) <= lanes &&
+           (batch >> (log2s + 1)) >= 16)
+        ++log2s;
+    if (log2s == 0)
+        return;
+    // (an even length: the segments' words then start alike in a block)
+    const uint64_t len = (((batch + (1ull << log2s) - 1) >> log2s) + 1) & ~1ull;
+    const uint64_t per_group = (uint64_t)kSplitBlock >> log2s; // walkers per workgroup
+    const uint64_t groups = (walkers + per_group - 1) / per_group;
+    if (len > kBinPassRecords / kSplitBlock || groups * kSplitBlock > kBinPassRecords / len)
+        return;
+    p.split_log2 = log2s;
+    p.split_len = len;
 }
 
 // Accumulation through the LDS cell cache needs cell indices below 2^32,
@@ -600,6 +741,19 @@ static LaunchPlan plan_launch(const ffr_renderer *r, uint64_t walkers, uint64_t 
     // or when asked for
     const uint64_t tw_bin = (uint64_t)kBinWalkBlock;
     const int ncol = r->spec.color_dims;
+    if (base_lds == 0)
+        split_plan(r, walkers, batch, sh, chain, p);
+    if (p.split_log2) {
+        p.chain = chain; // (the launch behind it)
+        p.block = kSplitBlock;
+        p.task_walkers = (uint64_t)kSplitBlock >> p.split_log2;
+        p.grid = (int)((walkers + p.task_walkers - 1) / p.task_walkers);
+        const int rb = r->mode == MODE_F64_U64 ? 8 : 4;
+        p.lds = split_lds(base, rb, r->spec.dims, ncol > 0 ? 4 : 0);
+        if (p.lds <= r->max_lds)
+            return p;
+        p = LaunchPlan();
+    }
     const bool bin_ok = base_lds == 0 && ncol <= 4 &&
                         r->cells < (ncol > 0 ? (1ull << 25) : (1ull << 28)) &&
                         (walkers + tw_bin - 1) / tw_bin * tw_bin <= kBinPassRecords;
@@ -715,6 +869,18 @@ static void walk_args(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchPlan
 
 static int launch_walk_any(int mode, int dims, const WalkLaunch &L)
 {
+    if (L.split)
+        switch (mode) {
+        case MODE_F64_U64:
+            return dims == 1 ? launch_split_f64u64_d1(L) : dims == 2 ? launch_split_f64u64_d2(L)
+                                                                      : launch_split_f64u64_d3(L);
+        case MODE_F32_U32:
+            return dims == 1 ? launch_split_f32u32_d1(L) : dims == 2 ? launch_split_f32u32_d2(L)
+                                                                      : launch_split_f32u32_d3(L);
+        default:
+            return dims == 1 ? launch_split_f32u64_d1(L) : dims == 2 ? launch_split_f32u64_d2(L)
+                                                                      : launch_split_f32u64_d3(L);
+        }
     switch (mode) {
     case MODE_F64_U64:
         return dims == 1 ? launch_walk_f64u64_d1(L) : dims == 2 ? launch_walk_f64u64_d2(L)
@@ -857,7 +1023,7 @@ template <typename R>
 static int choose_cache(ffr_renderer *r, const DeviceFlame<R> &d, LaunchPlan &p,
                         uint64_t walker0, uint64_t walkers, uint64_t batch, uint64_t samples)
 {
-    if (r->cache_pref >= 0 || !p.cache || p.chain || p.bin)
+    if (r->cache_pref >= 0 || !p.cache || p.chain || p.bin || p.split_log2)
         return FFR_OK;
     LaunchShape sh = renderer_shape(r);
     sh.cache = 0;
@@ -898,7 +1064,7 @@ static int prepare_compiled(ffr_renderer *r, const DeviceFlame<R> &d, const Laun
                             uint64_t samples)
 {
     r->rtc_fn = nullptr;
-    if (!r->compiled_pref || p.chain || p.bin)
+    if (!r->compiled_pref || p.chain || p.bin || p.split_log2)
         return FFR_OK;
     const int key = (p.cache ? 1 : 0) | (p.block << 1);
     const auto known = r->compiled_choice.find(key);
@@ -987,6 +1153,48 @@ static hipError_t ensure_device(void **p, size_t &have, size_t bytes)
     return e;
 }
 
+// the scratch of binned accumulation for `cap` records: grown as needed and
+// kept to ffr_destroy
+static hipError_t ensure_bin_scratch(ffr_renderer *r, uint64_t cap, int real_bytes)
+{
+    const int ncol = r->spec.color_dims;
+    const int tile_bits = ncol > 0 ? kBinTileBitsColour : kBinTileBits;
+    const size_t ntiles = (size_t)((r->cells + (1ull << tile_bits) - 1) >> tile_bits);
+    hipError_t e = hipSuccess;
+    size_t have_rec = (size_t)r->bin.capacity * 4, have_sorted = have_rec;
+    if (have_rec < cap * 4) {
+        e = ensure_device((void **)&r->bin.rec, have_rec, (size_t)cap * 4);
+        if (e == hipSuccess)
+            e = ensure_device((void **)&r->bin.sorted, have_sorted, (size_t)cap * 4);
+        r->bin.capacity = e == hipSuccess ? cap : 0;
+    }
+    // colour flames: the records' colours, component i at i * capacity
+    if (e == hipSuccess && ncol > 0) {
+        const size_t need = (size_t)ncol * (size_t)r->bin.capacity * (size_t)real_bytes;
+        size_t have_sorted_pay = r->bin_pay_bytes;
+        e = ensure_device(&r->bin.pay, r->bin_pay_bytes, need);
+        if (e == hipSuccess)
+            e = ensure_device(&r->bin.pay_sorted, have_sorted_pay, need);
+        if (e != hipSuccess)
+            r->bin_pay_bytes = 0;
+    }
+    size_t hist_bytes = r->bin_hist_words * 4;
+    if (e == hipSuccess)
+        e = ensure_device((void **)&r->bin.hist, hist_bytes,
+                          bin_scratch_hist_words(cap, (int)ntiles) * 4);
+    r->bin_hist_words = hist_bytes / 4;
+    // per tile: records, then the first accumulation work item; the regions
+    size_t tile_bytes = r->bin_tiles * 4;
+    if (e == hipSuccess && tile_bytes < 2 * (ntiles + 1) * 4) {
+        size_t t2 = tile_bytes;
+        e = ensure_device((void **)&r->bin.total, tile_bytes, 2 * (ntiles + 1) * 4);
+        if (e == hipSuccess)
+            e = ensure_device((void **)&r->bin.start, t2, 2 * (ntiles + 1) * 4);
+    }
+    r->bin_tiles = e == hipSuccess ? std::max(r->bin_tiles, 2 * (ntiles + 1)) : 0;
+    return e;
+}
+
 // Binned accumulation of one render: passes of `span` iterations of every
 // walker (the walkers' points and stream positions carry over in wstate),
 // each pass writing at most kBinPassRecords records, sorted by tile and
@@ -1009,41 +1217,7 @@ static int launch_binned(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchP
     const uint64_t npass = (batch + span - 1) / span;
     const uint64_t cap = slots * span;
     const int ncol = r->spec.color_dims; // colour components of each record
-    const int tile_bits = ncol > 0 ? kBinTileBitsColour : kBinTileBits;
-    const size_t ntiles = (size_t)((r->cells + (1ull << tile_bits) - 1) >> tile_bits);
-    hipError_t e = hipSuccess;
-    size_t have_rec = (size_t)r->bin.capacity * 4, have_sorted = have_rec;
-    if (have_rec < cap * 4) {
-        e = ensure_device((void **)&r->bin.rec, have_rec, (size_t)cap * 4);
-        if (e == hipSuccess)
-            e = ensure_device((void **)&r->bin.sorted, have_sorted, (size_t)cap * 4);
-        r->bin.capacity = e == hipSuccess ? cap : 0;
-    }
-    // colour flames: the records' colours, component i at i * capacity
-    if (e == hipSuccess && ncol > 0) {
-        const size_t need = (size_t)ncol * (size_t)r->bin.capacity * sizeof(R);
-        size_t have_sorted_pay = r->bin_pay_bytes;
-        e = ensure_device(&r->bin.pay, r->bin_pay_bytes, need);
-        if (e == hipSuccess)
-            e = ensure_device(&r->bin.pay_sorted, have_sorted_pay, need);
-        if (e != hipSuccess)
-            r->bin_pay_bytes = 0;
-    }
-    size_t hist_bytes = r->bin_hist_words * 4;
-    if (e == hipSuccess)
-        e = ensure_device((void **)&r->bin.hist, hist_bytes,
-                          bin_scratch_hist_words(cap, (int)ntiles) * 4);
-    r->bin_hist_words = hist_bytes / 4;
-    // per tile: records and (after the scatter) accumulation chunks, then
-    // the chunks' first work items (2 (ntiles + 1) words); the regions
-    size_t tile_bytes = r->bin_tiles * 4;
-    if (e == hipSuccess && tile_bytes < 2 * (ntiles + 1) * 4) {
-        size_t t2 = tile_bytes;
-        e = ensure_device((void **)&r->bin.total, tile_bytes, 2 * (ntiles + 1) * 4);
-        if (e == hipSuccess)
-            e = ensure_device((void **)&r->bin.start, t2, 2 * (ntiles + 1) * 4);
-    }
-    r->bin_tiles = e == hipSuccess ? std::max(r->bin_tiles, 2 * (ntiles + 1)) : 0;
+    hipError_t e = ensure_bin_scratch(r, cap, (int)sizeof(R));
     if (e == hipSuccess && npass > 1)
         e = ensure_device(&r->wstate, r->wstate_bytes, (size_t)slots * sizeof(WalkerState<R>));
     size_t args_bytes = r->dargs_bin_n * sizeof(WalkArgs<R>);
@@ -1158,11 +1332,85 @@ static int launch_binned(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchP
     return 0;
 }
 
+// records of a split render
+static uint64_t split_records(const LaunchPlan &p)
+{
+    return (uint64_t)p.grid * kSplitBlock * p.split_len;
+}
+
+// A split render: the split walkers write their records, which are binned
+// into the buffer; behind them the unsplit kernel of plan `fb`, which runs
+// only when the split failed (and then the records are not added).
+template <typename R>
+static int launch_split_render(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchPlan &p,
+                               const LaunchPlan &fb, uint64_t walker0, uint64_t walkers,
+                               uint64_t batch, uint64_t last)
+{
+    WalkArgs<R> a[2];
+    walk_args(r, d, fb, walker0, walkers, batch, last, a[0]);
+    a[0].split_main = r->dstats;
+    a[0].split_xf = r->dxf + r->nxf;
+    walk_args(r, d, p, walker0, walkers, batch, last, a[1]);
+    a[1].xf_count = r->dxf + r->nxf;
+    a[1].split_main = r->dstats;
+    a[1].split_len = p.split_len;
+    a[1].split_log2 = p.split_log2;
+    a[1].split_warm = r->split_warm;
+    a[1].rec = r->bin.rec;
+    a[1].pay = r->bin.pay;
+    a[1].pay_stride = r->bin.capacity;
+    r->hargs.resize(sizeof a);
+    std::memcpy(r->hargs.data(), a, sizeof a);
+    hipError_t e = hipMemcpyAsync(r->dargs, r->hargs.data(), sizeof a, hipMemcpyHostToDevice,
+                                  r->stream);
+    if (e != hipSuccess)
+        return (int)e;
+    WalkLaunch L;
+    L.nc = r->spec.color_dims;
+    L.vs = r->vs;
+    L.split = true;
+    L.grid = p.grid;
+    L.block = p.block;
+    L.lds = p.lds;
+    L.stream = r->stream;
+    L.args = (const unsigned char *)r->dargs + sizeof a[0];
+    int rc = launch_walk_any(r->mode, r->spec.dims, L);
+    if (rc)
+        return rc;
+    rc = launch_bin_accumulate(r->bin, split_records(p), r->cells, r->dbuf, (int)r->word_bytes,
+                               r->spec.color_dims, (int)sizeof(R), r->stream,
+                               &r->dstats->split_fail);
+    if (rc)
+        return rc;
+    return launch_table_kernel(r, fb, (int)d.slot_type.size());
+}
+
 static int launch(ffr_renderer *r, uint64_t samples)
 {
     uint64_t batch, walkers, last;
     split_samples(r, samples, batch, walkers, last);
     LaunchPlan p = plan_launch(r, walkers, batch, renderer_shape(r));
+    LaunchPlan fb;
+    r->last_split = false;
+    if (p.split_log2) {
+        // (its scratch may be allocated here, so not while the stream is
+        // captured; without the memory for it the walkers run unsplit)
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        const bool captured = hipStreamIsCapturing(r->stream, &cap) != hipSuccess ||
+                              cap != hipStreamCaptureStatusNone;
+        LaunchShape sh = renderer_shape(r);
+        sh.split = 0;
+        if (!captured &&
+            ensure_bin_scratch(r, split_records(p), r->mode == MODE_F64_U64 ? 8 : 4) == hipSuccess) {
+            r->last_split = true;
+            r->last_split_segments = walkers << p.split_log2;
+            sh.bin = 0;
+            fb = plan_launch(r, walkers, batch, sh);
+        } else {
+            (void)hipGetLastError();
+            p = plan_launch(r, walkers, batch, sh);
+        }
+    }
     // (the cache and compiled-kernel probes run first: the reset after them
     // clears what they counted)
     int rc = r->mode == MODE_F64_U64
@@ -1184,7 +1432,7 @@ static int launch(ffr_renderer *r, uint64_t samples)
     rc = launch_reset_stats(r->dstats, r->dxf, r->nxf, r->stream);
     if (rc)
         return fail(FFR_E_DEVICE, std::string("stats reset: ") + hipGetErrorString((hipError_t)rc));
-    if (p.bin) {
+    if (p.bin || r->last_split) {
         static std::once_flag prepared;
         static int prep_rc = 0;
         std::call_once(prepared, [] { prep_rc = prepare_bin_kernels(); });
@@ -1193,7 +1441,11 @@ static int launch(ffr_renderer *r, uint64_t samples)
                                           hipGetErrorString((hipError_t)prep_rc));
     }
     HIP_TRY(hipEventRecord(r->ev0, r->stream));
-    if (p.bin)
+    if (r->last_split)
+        rc = r->mode == MODE_F64_U64
+                 ? launch_split_render(r, r->f64, p, fb, r->next_walker, walkers, batch, last)
+                 : launch_split_render(r, r->f32, p, fb, r->next_walker, walkers, batch, last);
+    else if (p.bin)
         rc = r->mode == MODE_F64_U64
                  ? launch_binned(r, r->f64, p, r->next_walker, walkers, batch, last, samples)
                  : launch_binned(r, r->f32, p, r->next_walker, walkers, batch, last, samples);
@@ -1235,6 +1487,17 @@ static int finish(ffr_renderer *r, ffr_stats *out)
         for (int i = 0; i < r->spec.dims; ++i) {
             r->pmin[i] = std::min(r->pmin[i], st.pmin[i]);
             r->pmax[i] = std::max(r->pmax[i], st.pmax[i]);
+        }
+        if (r->last_split) {
+            // seams that did not join, or a bad value: unsplit from now on;
+            // many segments run twice: a longer run-up
+            if (st.split_fail)
+                r->split_ok = false;
+            else if (st.split_again * 256ull > r->last_split_segments)
+                r->split_warm *= 2;
+            if (r->split_warm > kSplitWarmMax)
+                r->split_ok = false;
+            r->last_split = false;
         }
         r->last_bad = st.n_bad;
         r->last_atomics = st.atomics;

@@ -5,21 +5,26 @@
 
 namespace ffr {
 
+// (a renderer's statistics blocks: the render's, and a split launch's
+// kSplitSlots behind it; the render's selection counters and the split's)
 __global__ void reset_stats_kernel(DevStats *st, unsigned long long *xf_count, int nxf)
 {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) {
-        st->s_iter = 0;
-        st->s_plot = 0;
-        st->n_bad = 0;
-        st->atomics = 0;
-        st->flush_atomics = 0;
+    const int t = threadIdx.x;
+    if (t <= kSplitSlots) {
+        DevStats *s = st + t;
+        s->s_iter = 0;
+        s->s_plot = 0;
+        s->n_bad = 0;
+        s->atomics = 0;
+        s->flush_atomics = 0;
+        s->split_fail = 0;
+        s->split_again = 0;
         for (int i = 0; i < 3; ++i) {
-            st->pmin[i] = (double)INFINITY;
-            st->pmax[i] = -(double)INFINITY;
+            s->pmin[i] = (double)INFINITY;
+            s->pmax[i] = -(double)INFINITY;
         }
     }
-    for (int k = t; k < nxf; k += gridDim.x * blockDim.x)
+    for (int k = t; k < 2 * nxf; k += blockDim.x)
         xf_count[k] = 0;
 }
 

@@ -5,6 +5,8 @@
 
 namespace ffr {
 
+// zero a renderer's statistics blocks (the render's, then kSplitSlots of a
+// split launch) and selection counters (nxf of the render, nxf of the split)
 int launch_reset_stats(DevStats *st, unsigned long long *xf_count, int nxf, hipStream_t s);
 // reset n renderers' statistics (device array e) and nq queue counters
 int launch_reset_many(const ResetEntry *e, int n, unsigned *queues, int nq, hipStream_t s);
@@ -46,8 +48,8 @@ struct BinScratch {
     unsigned *rec = nullptr;     // records of one pass (cell index or kEmptyKey)
     unsigned *sorted = nullptr;  // the same records grouped by tile
     unsigned *hist = nullptr;    // per block of records, per tile: count, then offset
-    unsigned *total = nullptr;   // per tile: records; then accumulation chunks and
-                                 // their first work items (2 (ntiles + 1) words)
+    unsigned *total = nullptr;   // per tile: records, then the first of its accumulation
+                                 // work items (2 ntiles + 1 words)
     unsigned *start = nullptr;   // per tile: first slot of its region (ntiles + 1)
     unsigned long long capacity = 0; // records rec and sorted hold
     // colour flames: each record's colour, component i at i * capacity
@@ -60,9 +62,10 @@ size_t bin_scratch_hist_words(unsigned long long records, int ntiles);
 // buffer (cells count words of word_bytes, no colour words)
 // (colour flames: r colour words per cell, the records' colours in b.pay as
 // reals of real_bytes; tile_bits kBinTileBitsColour)
+// skip (a device word, may be nullptr): add nothing when it is not 0
 int launch_bin_accumulate(const BinScratch &b, unsigned long long n_records,
                           unsigned long long cells, void *buf, int word_bytes, int r,
-                          int real_bytes, hipStream_t s);
+                          int real_bytes, hipStream_t s, const unsigned *skip = nullptr);
 // set the accumulate kernel's LDS limit (outside any stream capture)
 int prepare_bin_kernels();
 
@@ -77,10 +80,14 @@ int add_cells_staged_noalloc(void *dst, const void *src, unsigned long long byte
                              int word_bytes, hipStream_t s);
 
 // walker launches, one entry per precision mode and dimension count
+// (and the split walkers', split_kernel.inc)
 #define FFR_DECL_WALK(mode)                             \
     int launch_walk_##mode##_d1(const WalkLaunch &L); \
     int launch_walk_##mode##_d2(const WalkLaunch &L); \
-    int launch_walk_##mode##_d3(const WalkLaunch &L);
+    int launch_walk_##mode##_d3(const WalkLaunch &L); \
+    int launch_split_##mode##_d1(const WalkLaunch &L); \
+    int launch_split_##mode##_d2(const WalkLaunch &L); \
+    int launch_split_##mode##_d3(const WalkLaunch &L);
 FFR_DECL_WALK(f64u64)
 FFR_DECL_WALK(f32u32)
 FFR_DECL_WALK(f32u64)

@@ -17,6 +17,11 @@ struct DevStats {
     unsigned long long flush_atomics; // of those, the LDS cell-cache flushes
     double pmin[3];
     double pmax[3];
+    // split walkers (split_kernel.inc): set when the segments did not join
+    // up or a bad value was met, so that the render runs unsplit instead;
+    // and the segments that ran again from their neighbour's end
+    unsigned split_fail;
+    unsigned split_again;
 };
 
 constexpr int kMaxSlots = 64;     // variation slots per flame
@@ -70,6 +75,16 @@ template <typename R> struct WalkDyn {
     // at (R *)pay + i * pay_stride + k
     void *pay;
     uint64_t pay_stride;
+    // split walkers (split_kernel.inc): the render's statistics block, which
+    // holds the verdict; the split launch's own blocks follow it (kSplitSlots)
+    // and split_xf has its selection counters.  A kernel launched behind the split
+    // one with split_main set (and split_len 0) runs only if the split
+    // failed, else it adds the split's statistics to the render's.
+    DevStats *split_main;
+    unsigned long long *split_xf;
+    uint64_t split_len; // iterations per segment
+    int split_log2;     // log2 of the segments per walker
+    int split_warm;     // iterations a segment runs before its first
 };
 
 template <typename R> struct WalkArgs : WalkDyn<R> {
@@ -108,6 +123,15 @@ template <int D> struct XformLay {
 
 // lanes per workgroup (= walkers per task) of the binned walker kernel
 constexpr int kBinWalkBlock = 256;
+
+// lanes per workgroup of the split walker kernel, and the most segments a
+// walker is split into (2^kSplitMaxLog2: one workgroup)
+constexpr int kSplitBlock = 256;
+constexpr int kSplitMaxLog2 = 8;
+// its statistics blocks, taken by the workgroups in turn: on one block the
+// waves' atomics (and their retries) queue on a few addresses, 80 us of a
+// 210 us launch of 1024 waves
+constexpr int kSplitSlots = 32;
 
 // a walker between two passes of binned accumulation
 template <typename R> struct WalkerState {
@@ -204,6 +228,7 @@ struct WalkLaunch {
     bool chain_shared = false;        // one pre-affine matrix and weight for all
     bool chain_diag = false;          // ... and that matrix diagonal
     bool bin = false;                 // binned accumulation (walk_bin_kernel)
+    bool split = false;               // split walkers (split_kernel)
 };
 #endif // __HIPCC_RTC__
 
@@ -241,6 +266,13 @@ __host__ __device__ inline size_t cache_lds_offset(int tab_reals, int real_bytes
 __host__ __device__ inline size_t chain_stage_offset(int tab_reals, int real_bytes, int nxf)
 {
     return (cache_lds_offset(tab_reals, real_bytes, nxf) + 15u) & ~(size_t)15u;
+}
+
+// LDS of the split walker kernel: the flame table, masks and counters, then the lanes' end states
+__host__ __device__ inline size_t split_lds(size_t table_lds, int real_bytes, int d, int nc)
+{
+    return ((table_lds + 15u) & ~(size_t)15u) +
+           (size_t)kSplitBlock * (size_t)(d + nc) * (size_t)real_bytes;
 }
 
 // bytes of one cell-cache entry: key, count and the colour words

@@ -60,7 +60,14 @@ typedef struct ffr_options {
      * once a renderer renders again after its renders have asked for 2^28
      * samples in all, by a timed probe of the launch with and without it
      * per walker count; 0 off; 1 on where the flame allows it), the LDS the
-     * cache may take in KiB (0: 144), lanes per workgroup (0: chosen) */
+     * cache may take in KiB (0: 144), lanes per workgroup (0: chosen).
+     * With cell_cache and binned -1 and block 0, renders of few walkers
+     * (under 64 per CU) of a flame whose variations draw no random words,
+     * of at most 2^28 samples, split each walker's iterations over many
+     * lanes (not colour flames with 4-byte words).  The result is the
+     * unsplit one; scratch memory is allocated as for binned accumulation,
+     * and without it, or while the stream is captured, the walkers run
+     * unsplit. */
     int32_t cell_cache;
     int32_t cache_kib;
     int32_t block;
@@ -103,14 +110,16 @@ typedef struct ffr_stats {
     double kernel_ms;         /* device time of the last render's kernel (HIP events)  */
     uint64_t atomics;         /* global atomic adds of the last render on the buffer:
                                  one per word of a cell update that missed the LDS
-                                 cell cache or flushed it (no reference counterpart)  */
+                                 cell cache or flushed it (no reference counterpart);
+                                 0 when its walkers ran split                         */
     uint64_t flush_atomics;   /* of those, the LDS cell-cache flushes                   */
-    uint32_t wave_per_walker; /* 1: the last render ran one walker per wavefront (few
-                                 walkers of a linear flame, up to four colour
-                                 dimensions), 0: one per lane                         */
+    uint32_t wave_per_walker; /* 1: the last render gave each walker a wavefront or
+                                 more (few walkers of a linear flame, up to four
+                                 colour dimensions), 0: a lane, or split lanes        */
     uint32_t cache_slots;     /* LDS cell-cache slots per workgroup of the last render
                                  (0: no cache)                                        */
-    uint32_t binned;          /* 1: the last render used binned accumulation          */
+    uint32_t binned;          /* 1: the last render used binned accumulation behind
+                                 unsplit walkers                                      */
     uint32_t compiled;        /* 1: the last render ran the flame's compiled kernel    */
 } ffr_stats;
 
