@@ -488,7 +488,7 @@ int ffr_create(const char *flame_json, size_t len, const ffr_options *opt_in,
     HIP_TRY_D(hipMalloc(&rp->dxf, 2 * sizeof(unsigned long long) * (size_t)std::max(rp->nxf, 1)));
     HIP_TRY_D(hipMalloc(&rp->dbv_xfs, sizeof(unsigned long long) * rp->opt.bad_value_cap));
     HIP_TRY_D(hipMalloc(&rp->dbv_pts, sizeof(double) * 3 * rp->opt.bad_value_cap));
-    HIP_TRY_D(hipMalloc(&rp->dhist, sizeof(unsigned long long) * 3));
+    HIP_TRY_D(hipMalloc(&rp->dhist, sizeof(unsigned long long) * (kHistWords + kToneLut)));
     // (two: a split launch's and those of the launch behind it)
     HIP_TRY_D(hipMalloc(&rp->dargs,
                         2 * std::max(sizeof(WalkArgs<double>), sizeof(WalkArgs<float>))));
@@ -2003,8 +2003,36 @@ int render_image(ffr_renderer *r, int mode, double gamma, int bits, void *dst, s
         return fail(FFR_E_SIZE, "ffr_render_image: expected " + std::to_string(need) +
                                     " bytes of pixels");
     HIP_TRY(hipSetDevice(r->device));
-    HIP_TRY((hipError_t)launch_hist_stats(r->dbuf, r->cells, (int)r->cell_words,
-                                          (int)r->word_bytes, r->dhist, r->stream));
+    // the pixel kernel takes the bounds from device memory (and writes
+    // nothing when the histogram is empty), so one wait covers both passes
+    const bool pixels = dst && !(mode == FFR_IMG_COLOR && r->spec.color_dims != 3);
+    if (pixels) {
+        void *out = dst;
+        if (to_host) {
+            if (r->dimg_bytes < need) {
+                HIP_TRY(hipFree(r->dimg));
+                r->dimg = nullptr;
+                r->dimg_bytes = 0;
+                HIP_TRY(hipMalloc(&r->dimg, need));
+                r->dimg_bytes = need;
+            }
+            out = r->dimg;
+        }
+        HIP_TRY((hipError_t)launch_hist_bounds(r->dbuf, r->cells, (int)r->cell_words,
+                                               (int)r->word_bytes, r->dhist, r->stream));
+        // num_t gp = 1.0 / arg_gamma (ffr_img.cpp:240): a double division, then num_t
+        const double gp = f32 ? (double)(float)(1.0 / (double)(float)gamma) : 1.0 / gamma;
+        if (info)
+            HIP_TRY(hipEventRecord(r->ev0, r->stream));
+        HIP_TRY((hipError_t)launch_tonemap(r->dbuf, r->cells, (int)r->cell_words,
+                                           (int)r->word_bytes, mode, r->dhist, gp,
+                                           mode == FFR_IMG_MONO ? 8 : bits, out, r->stream));
+        if (info)
+            HIP_TRY(hipEventRecord(r->ev1, r->stream));
+    } else {
+        HIP_TRY((hipError_t)launch_hist_stats(r->dbuf, r->cells, (int)r->cell_words,
+                                              (int)r->word_bytes, r->dhist, r->stream));
+    }
     unsigned long long h[3];
     HIP_TRY(hipMemcpyAsync(h, r->dhist, sizeof h, hipMemcpyDeviceToHost, r->stream));
     HIP_TRY(hipStreamSynchronize(r->stream));
@@ -2029,31 +2057,13 @@ int render_image(ffr_renderer *r, int mode, double gamma, int bits, void *dst, s
         return fail(FFR_E_UNSUPPORTED, "buffer must use 3 color dimensions");
     if (!dst)
         return FFR_OK;
-    void *out = dst;
-    if (to_host) {
-        if (r->dimg_bytes < need) {
-            HIP_TRY(hipFree(r->dimg));
-            r->dimg = nullptr;
-            r->dimg_bytes = 0;
-            HIP_TRY(hipMalloc(&r->dimg, need));
-            r->dimg_bytes = need;
-        }
-        out = r->dimg;
-    }
-    // num_t gp = 1.0 / arg_gamma (ffr_img.cpp:240): a double division, then num_t
-    const double gp = f32 ? (double)(float)(1.0 / (double)(float)gamma) : 1.0 / gamma;
-    HIP_TRY(hipEventRecord(r->ev0, r->stream));
-    HIP_TRY((hipError_t)launch_tonemap(r->dbuf, r->cells, (int)r->cell_words,
-                                       (int)r->word_bytes, mode, mx, gp,
-                                       mode == FFR_IMG_MONO ? 8 : bits, out, r->stream));
-    HIP_TRY(hipEventRecord(r->ev1, r->stream));
     if (to_host)
-        HIP_TRY(hipMemcpyAsync(dst, r->dimg, need, hipMemcpyDeviceToHost, r->stream));
-    HIP_TRY(hipStreamSynchronize(r->stream));
-    float ms = 0.f;
-    HIP_TRY(hipEventElapsedTime(&ms, r->ev0, r->ev1));
-    if (info)
+        HIP_TRY(hipMemcpy(dst, r->dimg, need, hipMemcpyDeviceToHost));
+    if (info) {
+        float ms = 0.f;
+        HIP_TRY(hipEventElapsedTime(&ms, r->ev0, r->ev1));
         info->kernel_ms = (double)ms;
+    }
     return FFR_OK;
 }
 

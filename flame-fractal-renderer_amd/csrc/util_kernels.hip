@@ -77,18 +77,35 @@ constexpr int kReduceBlock = 256;
 constexpr int kReduceWaves = kReduceBlock / 64;
 constexpr int kReduceGrid = 512;
 
+// Sum, min and max of the counts, one set per workgroup (kHistGrid of them,
+// padded with a neutral set each lane of a short grid writes): no counter
+// to clear before and no atomics.  A cell's count is 8 of its 32 bytes, so
+// every line of the buffer is read; eight loads of a lane are in flight.
+constexpr int kHistLoads = 8;
+
 template <typename CT>
-__global__ void hist_stats_kernel(const CT *buf, unsigned long long cells, int cw,
-                                  unsigned long long *out /* sum, min, max */)
+__global__ void __launch_bounds__(kReduceBlock)
+    hist_stats_kernel(const CT *buf, unsigned long long cells, int cw,
+                      unsigned long long *part /* [3][kHistGrid]: sums, mins, maxs */)
 {
     unsigned long long sum = 0, mn = ~0ull, mx = 0;
-#pragma unroll 4
-    for (unsigned long long c = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
-         c < cells; c += (unsigned long long)gridDim.x * blockDim.x) {
-        unsigned long long v = (unsigned long long)buf[c * (unsigned long long)cw];
-        sum += v;
-        mn = v < mn ? v : mn;
-        mx = v > mx ? v : mx;
+    const unsigned long long step = (unsigned long long)gridDim.x * kReduceBlock;
+    for (unsigned long long c0 = (unsigned long long)blockIdx.x * kReduceBlock + threadIdx.x;
+         c0 < cells; c0 += step * kHistLoads) {
+        CT v[kHistLoads];
+#pragma unroll
+        for (int j = 0; j < kHistLoads; ++j) {
+            const unsigned long long c = c0 + (unsigned long long)j * step;
+            v[j] = buf[(c < cells ? c : c0) * (unsigned long long)cw];
+        }
+#pragma unroll
+        for (int j = 0; j < kHistLoads; ++j) {
+            const unsigned long long w = (unsigned long long)v[j];
+            // (past the end, the first cell again: no new bound)
+            sum += c0 + (unsigned long long)j * step < cells ? w : 0ull;
+            mn = w < mn ? w : mn;
+            mx = w > mx ? w : mx;
+        }
     }
     for (int off = 32; off > 0; off >>= 1) {
         sum += __shfl_xor(sum, off, 64);
@@ -97,8 +114,6 @@ __global__ void hist_stats_kernel(const CT *buf, unsigned long long cells, int c
         mn = a < mn ? a : mn;
         mx = b > mx ? b : mx;
     }
-    // one set of atomics per workgroup: atomics on one address serialise
-    // (about 80 M/s), so per-wave atomics over a 4K buffer took milliseconds
     __shared__ unsigned long long ps[kReduceWaves], pn[kReduceWaves], px[kReduceWaves];
     const int w = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) {
@@ -108,15 +123,70 @@ __global__ void hist_stats_kernel(const CT *buf, unsigned long long cells, int c
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int i = 1; i < (int)(blockDim.x >> 6); ++i) {
+        for (int i = 1; i < kReduceWaves; ++i) {
             sum += ps[i];
             mn = pn[i] < mn ? pn[i] : mn;
             mx = px[i] > mx ? px[i] : mx;
         }
-        atomicAdd(&out[0], sum);
-        atomicMin(&out[1], mn);
-        atomicMax(&out[2], mx);
+        for (int g = (int)blockIdx.x; g < kHistGrid; g += (int)gridDim.x) {
+            const bool own = g == (int)blockIdx.x;
+            part[g] = own ? sum : 0;
+            part[kHistGrid + g] = own ? mn : ~0ull;
+            part[2 * kHistGrid + g] = own ? mx : 0;
+        }
     }
+}
+
+// the largest count of all workgroups, in every lane of the calling
+// workgroup of kReduceBlock lanes; with `out`, lane 0 also leaves sum, min
+// and max there
+__device__ unsigned long long hist_reduce(const unsigned long long *part,
+                                          unsigned long long *out)
+{
+    __shared__ unsigned long long ps[kReduceWaves], pn[kReduceWaves], px[kReduceWaves];
+    unsigned long long sum = 0, mn = ~0ull, mx = 0;
+    for (int g = (int)threadIdx.x; g < kHistGrid; g += kReduceBlock) {
+        const unsigned long long b = part[2 * kHistGrid + g];
+        mx = b > mx ? b : mx;
+        if (out) {
+            sum += part[g];
+            const unsigned long long a = part[kHistGrid + g];
+            mn = a < mn ? a : mn;
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned long long b = __shfl_xor(mx, off, 64);
+        mx = b > mx ? b : mx;
+        if (out) {
+            sum += __shfl_xor(sum, off, 64);
+            const unsigned long long a = __shfl_xor(mn, off, 64);
+            mn = a < mn ? a : mn;
+        }
+    }
+    if ((threadIdx.x & 63) == 0) {
+        ps[threadIdx.x >> 6] = sum;
+        pn[threadIdx.x >> 6] = mn;
+        px[threadIdx.x >> 6] = mx;
+    }
+    __syncthreads();
+    for (int i = 0; i < kReduceWaves; ++i)
+        mx = px[i] > mx ? px[i] : mx;
+    if (out && threadIdx.x == 0) {
+        for (int i = 1; i < kReduceWaves; ++i) {
+            sum += ps[i];
+            mn = pn[i] < mn ? pn[i] : mn;
+        }
+        out[0] = sum;
+        out[1] = mn;
+        out[2] = mx;
+    }
+    return mx;
+}
+
+__global__ void __launch_bounds__(kReduceBlock)
+    hist_reduce_kernel(const unsigned long long *part, unsigned long long *out)
+{
+    (void)hist_reduce(part, out);
 }
 
 // L1 distance of two normalised count histograms with the same cells:
@@ -175,17 +245,45 @@ __device__ inline float img_log(float x) { return (float)log((double)x); }
 __device__ inline double img_pow(double x, double y) { return pow(x, y); }
 __device__ inline float img_pow(float x, float y) { return (float)pow((double)x, (double)y); }
 
-template <typename CT, typename CR, typename N, typename P>
-__global__ void tonemap_kernel(const CT *buf, unsigned long long cells, int cw, int mode,
-                               N maxc, N gp, N scale, P *out)
+// pow(log(1 + h) / max, gp) of every count h below `lut_n` and up to the
+// largest: most cells of an image hold one of few counts, and the two
+// functions in double cost more than the cell's trip through memory (a
+// 3840x2160 colour image: 51 us evaluating them per cell, ~250 double
+// instructions each).  The bounds pass's results are reduced here too, so
+// that the host need not wait for them in between.
+template <typename N>
+__global__ void __launch_bounds__(kReduceBlock)
+    tonemap_lut_kernel(unsigned long long *hist, N gp, unsigned lut_n, N *lut)
 {
-    const N max = img_log((N)1 + maxc);
+    const unsigned long long maxc = hist_reduce(hist + 3, blockIdx.x == 0 ? hist : nullptr);
+    const unsigned h = blockIdx.x * kReduceBlock + threadIdx.x;
+    if (maxc == 0 || h >= lut_n || h > maxc)
+        return;
+    lut[h] = img_pow(img_log((N)1 + (N)h) / img_log((N)1 + (N)maxc), gp);
+}
+
+template <typename CT, typename CR, typename N, typename P>
+__global__ void __launch_bounds__(kReduceBlock)
+    tonemap_kernel(const CT *buf, unsigned long long cells, int cw, int mode,
+                   const unsigned long long *hist, N gp, N scale, unsigned lut_n, const N *lut,
+                   P *out)
+{
+    const unsigned long long maxc = hist[2];
+    if (maxc == 0)
+        return; // (the host reports the empty histogram)
+    const N max = img_log((N)1 + (N)maxc);
     // an empty cell is 0 in every mode while gp > 0: log(1) / max = 0 and
     // pow(0, gp) = 0 in gray; in colour the sums over a zero count give
     // NaN or infinity, whose conversion leaves 0
     const bool empty_is_zero = gp > (N)0;
-    for (unsigned long long c = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
-         c < cells; c += (unsigned long long)gridDim.x * blockDim.x) {
+    auto level = [&](CT h) {
+        return h < (CT)lut_n ? lut[h] : img_pow(img_log((N)1 + (N)h) / max, gp);
+    };
+    // from the buffer's end backwards: its last part, which the bounds pass
+    // read last, is still in the last-level cache
+    for (unsigned long long k = (unsigned long long)blockIdx.x * kReduceBlock + threadIdx.x;
+         k < cells; k += (unsigned long long)gridDim.x * kReduceBlock) {
+        const unsigned long long c = cells - 1 - k;
         const CT *cell = buf + c * (unsigned long long)cw;
         const CT h = cell[0];
         if (mode == 0) {
@@ -195,13 +293,13 @@ __global__ void tonemap_kernel(const CT *buf, unsigned long long cells, int cw, 
         if (mode == 1) {
             N v = (N)0;
             if (h != 0 || !empty_is_zero)
-                v = img_pow(img_log((N)1 + (N)h) / max, gp);
+                v = level(h);
             out[c] = (P)host_i32(v * scale);
             continue;
         }
         P px[3] = {0, 0, 0};
         if (h != 0) {
-            const N ll = img_pow(img_log((N)1 + (N)h) / max, gp);
+            const N ll = level(h);
             const N hn = (N)h;
             const CR *col = reinterpret_cast<const CR *>(cell + 1);
             for (int i = 0; i < 3; ++i)
@@ -233,13 +331,6 @@ __global__ void scatter_atomics_kernel(CT *buf, unsigned long long cells, int cw
         for (int i = 0; i < cw - 1; ++i)
             unsafeAtomicAdd(&col[i], (CR)0.5);
     }
-}
-
-__global__ void hist_stats_init_kernel(unsigned long long *out)
-{
-    out[0] = 0;
-    out[1] = ~0ull;
-    out[2] = 0;
 }
 
 __global__ void fill_zero_kernel(unsigned int *p, unsigned long long n)
@@ -285,18 +376,27 @@ int launch_add_cells(void *dst, const void *src, unsigned long long words, int c
     return (int)hipGetLastError();
 }
 
+int launch_hist_bounds(const void *buf, unsigned long long cells, int cw, int word_bytes,
+                       unsigned long long *out, hipStream_t s)
+{
+    const int grid = std::min(grid_for(cells, kReduceBlock), kHistGrid);
+    if (word_bytes == 8)
+        hipLaunchKernelGGL((hist_stats_kernel<unsigned long long>), dim3(grid),
+                           dim3(kReduceBlock), 0, s, (const unsigned long long *)buf, cells, cw,
+                           out + 3);
+    else
+        hipLaunchKernelGGL((hist_stats_kernel<unsigned int>), dim3(grid), dim3(kReduceBlock), 0,
+                           s, (const unsigned int *)buf, cells, cw, out + 3);
+    return (int)hipGetLastError();
+}
+
 int launch_hist_stats(const void *buf, unsigned long long cells, int cw, int word_bytes,
                       unsigned long long *out, hipStream_t s)
 {
-    hipLaunchKernelGGL(hist_stats_init_kernel, dim3(1), dim3(1), 0, s, out);
-    const int block = kReduceBlock;
-    const int grid = std::min(grid_for(cells, block), kReduceGrid);
-    if (word_bytes == 8)
-        hipLaunchKernelGGL((hist_stats_kernel<unsigned long long>), dim3(grid), dim3(block), 0,
-                           s, (const unsigned long long *)buf, cells, cw, out);
-    else
-        hipLaunchKernelGGL((hist_stats_kernel<unsigned int>), dim3(grid), dim3(block), 0, s,
-                           (const unsigned int *)buf, cells, cw, out);
+    const int rc = launch_hist_bounds(buf, cells, cw, word_bytes, out, s);
+    if (rc)
+        return rc;
+    hipLaunchKernelGGL(hist_reduce_kernel, dim3(1), dim3(kReduceBlock), 0, s, out + 3, out);
     return (int)hipGetLastError();
 }
 
@@ -324,38 +424,42 @@ int launch_l1_counts(const void *a, int cwa, int wba, const void *b, int cwb, in
     return (int)hipGetLastError();
 }
 
-int launch_tonemap(const void *buf, unsigned long long cells, int cw, int word_bytes, int mode,
-                   unsigned long long maxc, double gp, int bits, void *out, hipStream_t s)
+template <typename CT, typename CR>
+static void launch_tonemap_words(const void *buf, unsigned long long cells, int cw, int mode,
+                                 unsigned long long *hist, CR gp, int bits, CR scale, void *out,
+                                 hipStream_t s)
 {
+    // a table of at most a quarter of the cells (mono takes none)
+    const unsigned lut_n =
+        mode == 0 ? 0u : (unsigned)std::min<unsigned long long>(kToneLut, cells / 4);
+    CR *lut = reinterpret_cast<CR *>(hist + kHistWords);
+    hipLaunchKernelGGL((tonemap_lut_kernel<CR>),
+                       dim3(std::max(1u, (lut_n + kReduceBlock - 1) / kReduceBlock)),
+                       dim3(kReduceBlock), 0, s, hist, gp, lut_n, lut);
     // 2048 workgroups of 256 (eight waves per SIMD); each lane takes about
     // 16 cells of a 3840 x 2160 buffer, so the max above is taken rarely
-    const int block = 256;
-    const int grid = std::min(grid_for(cells, block), 2048);
-    using U8 = unsigned long long;
-    using U4 = unsigned int;
-    if (word_bytes == 8) {
-        // the default build: num_t = double, 64-bit words
-        const double scale = (bits == 8 ? 256.0 : 65536.0) * (1.0 - 1.0 / 4503599627370496.0);
-        if (bits == 8)
-            hipLaunchKernelGGL((tonemap_kernel<U8, double, double, unsigned char>), dim3(grid),
-                               dim3(block), 0, s, (const U8 *)buf, cells, cw, mode, (double)maxc, gp,
-                               scale, (unsigned char *)out);
-        else
-            hipLaunchKernelGGL((tonemap_kernel<U8, double, double, unsigned short>), dim3(grid),
-                               dim3(block), 0, s, (const U8 *)buf, cells, cw, mode, (double)maxc, gp,
-                               scale, (unsigned short *)out);
-    } else {
-        // the float build: num_t = float, 32-bit words
-        const float scale = (bits == 8 ? 256.0f : 65536.0f) * (1.0f - 1.0f / 8388608.0f);
-        if (bits == 8)
-            hipLaunchKernelGGL((tonemap_kernel<U4, float, float, unsigned char>), dim3(grid),
-                               dim3(block), 0, s, (const U4 *)buf, cells, cw, mode, (float)maxc,
-                               (float)gp, scale, (unsigned char *)out);
-        else
-            hipLaunchKernelGGL((tonemap_kernel<U4, float, float, unsigned short>), dim3(grid),
-                               dim3(block), 0, s, (const U4 *)buf, cells, cw, mode, (float)maxc,
-                               (float)gp, scale, (unsigned short *)out);
-    }
+    const int grid = std::min(grid_for(cells, kReduceBlock), 2048);
+    if (bits == 8)
+        hipLaunchKernelGGL((tonemap_kernel<CT, CR, CR, unsigned char>), dim3(grid),
+                           dim3(kReduceBlock), 0, s, (const CT *)buf, cells, cw, mode, hist, gp,
+                           scale, lut_n, lut, (unsigned char *)out);
+    else
+        hipLaunchKernelGGL((tonemap_kernel<CT, CR, CR, unsigned short>), dim3(grid),
+                           dim3(kReduceBlock), 0, s, (const CT *)buf, cells, cw, mode, hist, gp,
+                           scale, lut_n, lut, (unsigned short *)out);
+}
+
+int launch_tonemap(const void *buf, unsigned long long cells, int cw, int word_bytes, int mode,
+                   unsigned long long *hist, double gp, int bits, void *out, hipStream_t s)
+{
+    if (word_bytes == 8) // the default build: num_t = double, 64-bit words
+        launch_tonemap_words<unsigned long long, double>(
+            buf, cells, cw, mode, hist, gp, bits,
+            (bits == 8 ? 256.0 : 65536.0) * (1.0 - 1.0 / 4503599627370496.0), out, s);
+    else // the float build: num_t = float, 32-bit words
+        launch_tonemap_words<unsigned, float>(
+            buf, cells, cw, mode, hist, (float)gp, bits,
+            (bits == 8 ? 256.0f : 65536.0f) * (1.0f - 1.0f / 8388608.0f), out, s);
     return (int)hipGetLastError();
 }
 

@@ -12,6 +12,15 @@ int launch_reset_stats(DevStats *st, unsigned long long *xf_count, int nxf, hipS
 int launch_reset_many(const ResetEntry *e, int n, unsigned *queues, int nq, hipStream_t s);
 int launch_add_cells(void *dst, const void *src, unsigned long long words, int cw,
                      int word_bytes, hipStream_t s);
+// sum, min and max of the counts into out[0..2]; out has kHistWords words,
+// the rest is scratch.  launch_hist_bounds leaves only the scratch, which
+// launch_tonemap reduces into out[0..2].
+constexpr int kHistGrid = 1024;
+constexpr int kHistWords = 3 + 3 * kHistGrid;
+// the tone table of an image follows them: kToneLut reals
+constexpr unsigned kToneLut = 1u << 16;
+int launch_hist_bounds(const void *buf, unsigned long long cells, int cw, int word_bytes,
+                       unsigned long long *out, hipStream_t s);
 int launch_hist_stats(const void *buf, unsigned long long cells, int cw, int word_bytes,
                       unsigned long long *out, hipStream_t s);
 // L1 distance of two normalised count histograms (word bytes 4 or 8 each)
@@ -19,10 +28,11 @@ int launch_l1_counts(const void *a, int cwa, int wba, const void *b, int cwb, in
                      unsigned long long cells, double inv_a, double inv_b, double *out,
                      hipStream_t s);
 // the ffr-img image of a 2-D buffer: mode 0 mono, 1 gray, 2 colour (r = 3);
-// maxc = the largest count, gp = 1 / gamma in num_t; bits 8 or 16 (mono
+// hist: what launch_hist_bounds left of the buffer (nothing is written when
+// its largest count is 0), gp = 1 / gamma in num_t; bits 8 or 16 (mono
 // always writes 8-bit pixels)
 int launch_tonemap(const void *buf, unsigned long long cells, int cw, int word_bytes, int mode,
-                   unsigned long long maxc, double gp, int bits, void *out, hipStream_t s);
+                   unsigned long long *hist, double gp, int bits, void *out, hipStream_t s);
 // `updates` cell updates scattered uniformly over `cells` cells of cw words
 // (a count add and cw - 1 colour adds each, as the walker kernel's misses)
 int launch_scatter_atomics(void *buf, unsigned long long cells, int cw, int word_bytes,
