@@ -28,6 +28,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 namespace ffr {
 
@@ -353,57 +354,110 @@ __global__ void __launch_bounds__(1024)
     }
 }
 
-// Colour flames: the scatter also moves each record's colour.  The chunk's
-// keys are sorted in LDS; then, one colour component at a time, the chunk's
-// values are read in order (coalesced), placed in LDS where their keys went
-// and written out in tile order.  (Gathered from HBM through the keys'
-// places in the chunk instead, the reads fetched about ten times the
-// colours' bytes.)
-constexpr size_t scatter_pay_lds(int ntiles, int per, int real_bytes)
+// Workgroup barriers that order the LDS only: loads and stores of device
+// memory stay in flight across them.
+__device__ __forceinline__ void lds_barrier()
 {
-    return sizeof(unsigned) * (2 * (size_t)ntiles + (size_t)kScatterLanes * (size_t)per) +
-           (size_t)real_bytes * (size_t)kScatterLanes * (size_t)per;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <int PER, typename PR>
+// Colour flames: the scatter also moves each record's colour.  The walker
+// leaves keys and colour components in arrays of their own; here a chunk's
+// records are read once, put into tile order in LDS as whole records of NW
+// words (key, colour, padding to 16 bytes) and written out as such, so that
+// a tile's run of a chunk (8 records of 16 bytes for 1024 tiles) is one
+// piece of memory.  The next chunk's records are read while this one is
+// written.  (Moved one component at a time through LDS, with 4-byte runs
+// and a barrier on every component's reads, a pass of 2^28 three-colour FP32
+// records took 3.83 ms; now 2.67.)
+constexpr size_t scatter_pay_lds(int ntiles, int per, int nw)
+{
+    return sizeof(unsigned) * ((size_t)nw * (size_t)kScatterLanes * (size_t)per +
+                               2 * (size_t)ntiles + 16);
+}
+
+// words of a colour record as the kernels below are built: the key and up
+// to three reals, or four, to whole 16 bytes
+constexpr int colour_record_words(int r, int real_bytes)
+{
+    return ((1 + (r <= 3 ? 3 : 4) * (real_bytes / 4)) + 3) / 4 * 4;
+}
+static_assert(colour_record_words(1, 4) == 4 && colour_record_words(4, 4) == 8 &&
+                  colour_record_words(1, 8) == 8 && colour_record_words(4, 8) == 12,
+              "the record sizes the colour kernels are built for");
+
+template <typename PR> __device__ __forceinline__ void put_real(unsigned *w, PR v);
+template <> __device__ __forceinline__ void put_real(unsigned *w, float v)
+{
+    w[0] = __float_as_uint(v);
+}
+template <> __device__ __forceinline__ void put_real(unsigned *w, double v)
+{
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    w[0] = (unsigned)b;
+    w[1] = (unsigned)(b >> 32);
+}
+template <typename PR> __device__ __forceinline__ double get_real(const unsigned *w);
+template <> __device__ __forceinline__ double get_real<float>(const unsigned *w)
+{
+    return (double)__uint_as_float(w[0]);
+}
+template <> __device__ __forceinline__ double get_real<double>(const unsigned *w)
+{
+    return __longlong_as_double((long long)(((unsigned long long)w[1] << 32) | w[0]));
+}
+
+template <int PER, int NW, typename PR>
 __global__ void __launch_bounds__(kScatterLanes)
     bin_scatter_pay_kernel(const unsigned *rec, const PR *pay, unsigned long long n,
                            unsigned long long per_block, int tile_bits, int ntiles,
-                           const unsigned *hist, const unsigned *start, unsigned *sorted,
-                           PR *pay_sorted, unsigned long long stride, int nr)
+                           const unsigned *hist, const unsigned *start, uint4 *sorted,
+                           unsigned long long stride, int nr)
 {
-    extern __shared__ unsigned lds[];
-    unsigned *cur = lds;                          // [ntiles] next slot of each tile
-    unsigned *off = cur + ntiles;                 // [ntiles] chunk counts, then ends
-    unsigned *stage = off + ntiles;               // [chunk] keys in tile order
-    // [chunk] one colour component in tile order (8-byte aligned: the
-    // arrays before it are even numbers of words)
-    PR *pl = reinterpret_cast<PR *>(stage + kScatterLanes * PER);
-    unsigned *wsum = stage;                       // [16] wave sums of the scan
+    constexpr int kReal = (int)sizeof(PR) / 4;
+    constexpr int NR = (NW - 1) / kReal < 4 ? (NW - 1) / kReal : 4; // reals a record can hold
+    constexpr int kChunk = kScatterLanes * PER;
+    extern __shared__ uint4 stage[];                // [NW / 4][kChunk] records in tile order
+    unsigned *cur = reinterpret_cast<unsigned *>(stage + NW / 4 * kChunk); // [ntiles] next slots
+    unsigned *off = cur + ntiles;                   // [ntiles] chunk counts, then run starts
+    unsigned *wsum = off + ntiles;                  // [16] wave sums of the scan
     const int tid = (int)threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const unsigned *row = hist + (size_t)blockIdx.x * (size_t)ntiles;
-    for (int t = tid; t < ntiles; t += kScatterLanes)
+    for (int t = tid; t < ntiles; t += kScatterLanes) {
         cur[t] = start[t] + row[t];
+        off[t] = 0;
+    }
     const unsigned long long b0 = (unsigned long long)blockIdx.x * per_block;
     const unsigned long long b1 = b0 + per_block < n ? b0 + per_block : n;
-    constexpr unsigned long long chunk = (unsigned long long)kScatterLanes * PER;
     const int per_t = (ntiles + kScatterLanes - 1) / kScatterLanes;
-    for (unsigned long long c0 = b0; c0 < b1; c0 += chunk) {
-        for (int t = tid; t < ntiles; t += kScatterLanes)
-            off[t] = 0;
-        __syncthreads();
-        unsigned c[PER];
+    unsigned c[PER];
+    PR v[PER][NR];
+    auto load = [&](unsigned long long c0) {
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
             const unsigned long long i = c0 + (unsigned long long)k * kScatterLanes + tid;
             c[k] = i < b1 ? rec[i] : kBinEmpty;
+#pragma unroll
+            for (int j = 0; j < NR; ++j)
+                if (j < nr)
+                    v[k][j] = pay[(unsigned long long)j * stride + (i < b1 ? i : b0)];
         }
+    };
+    if (b0 < b1)
+        load(b0);
+    lds_barrier();
+    for (unsigned long long c0 = b0; c0 < b1; c0 += kChunk) {
+        // each record's rank in its tile's run of the chunk
+        unsigned at[PER];
 #pragma unroll
         for (int k = 0; k < PER; ++k)
-            if (c[k] != kBinEmpty)
-                atomicAdd(&off[c[k] >> tile_bits], 1u);
-        __syncthreads();
+            at[k] = c[k] != kBinEmpty ? atomicAdd(&off[c[k] >> tile_bits], 1u) : 0u;
+        lds_barrier();
+        // exclusive scan of the chunk's tile counts (per lane, per wave,
+        // across the sixteen waves)
         const int t0 = tid * per_t;
         unsigned mine = 0;
         for (int j = 0; j < per_t; ++j)
@@ -418,7 +472,7 @@ __global__ void __launch_bounds__(kScatterLanes)
         }
         if (lane == 63)
             wsum[wave] = incl;
-        __syncthreads();
+        lds_barrier();
         unsigned before = 0, total = 0;
         for (int w = 0; w < kScatterLanes / 64; ++w) {
             const unsigned ws = wsum[w];
@@ -428,45 +482,52 @@ __global__ void __launch_bounds__(kScatterLanes)
         unsigned run = before + incl - mine;
         for (int j = 0; j < per_t; ++j)
             if (t0 + j < ntiles) {
-                const unsigned v = off[t0 + j];
+                const unsigned m = off[t0 + j];
                 off[t0 + j] = run;
-                run += v;
+                run += m;
             }
-        __syncthreads();
-        // each record's place in the chunk's tile order (kBinEmpty: none)
-        unsigned at[PER];
+        lds_barrier();
 #pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            at[k] = kBinEmpty;
+        for (int k = 0; k < PER; ++k)
             if (c[k] != kBinEmpty) {
-                at[k] = atomicAdd(&off[c[k] >> tile_bits], 1u);
-                stage[at[k]] = c[k];
-            }
-        }
-        __syncthreads();
-        for (unsigned i = (unsigned)tid; i < total; i += kScatterLanes) {
-            const unsigned r = stage[i];
-            const unsigned t = r >> tile_bits;
-            sorted[cur[t] + (i - (t ? off[t - 1] : 0u))] = r;
-        }
-        for (int j = 0; j < nr; ++j) {
-            const PR *src = pay + (unsigned long long)j * stride + c0;
+                unsigned w[NW];
 #pragma unroll
-            for (int k = 0; k < PER; ++k)
-                if (at[k] != kBinEmpty)
-                    pl[at[k]] = src[(unsigned)(k * kScatterLanes + tid)];
-            __syncthreads();
-            PR *dst = pay_sorted + (unsigned long long)j * stride;
-            for (unsigned i = (unsigned)tid; i < total; i += kScatterLanes) {
-                const unsigned t = stage[i] >> tile_bits;
-                dst[cur[t] + (i - (t ? off[t - 1] : 0u))] = pl[i];
+                for (int j = 0; j < NW; ++j)
+                    w[j] = 0;
+                w[0] = c[k];
+#pragma unroll
+                for (int j = 0; j < NR; ++j)
+                    if (j < nr)
+                        put_real<PR>(w + 1 + j * kReal, v[k][j]);
+                const unsigned pos = off[c[k] >> tile_bits] + at[k];
+#pragma unroll
+                for (int q = 0; q < NW / 4; ++q)
+                    stage[q * kChunk + pos] =
+                        make_uint4(w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]);
             }
-            __syncthreads();
+        if (c0 + kChunk < b1)
+            load(c0 + kChunk);
+        lds_barrier();
+        for (unsigned i = (unsigned)tid; i < total; i += kScatterLanes) {
+            const uint4 first = stage[i];
+            const unsigned t = first.x >> tile_bits;
+            uint4 *dst = sorted + (size_t)(cur[t] + (i - off[t])) * (NW / 4);
+            dst[0] = first;
+#pragma unroll
+            for (int q = 1; q < NW / 4; ++q)
+                dst[q] = stage[q * kChunk + i];
         }
-        __syncthreads();
+        lds_barrier();
+        // (the run of tile t ends where the next one's starts)
+        for (int j = 0; j < per_t; ++j)
+            if (t0 + j < ntiles) {
+                const unsigned end = t0 + j + 1 < ntiles ? off[t0 + j + 1] : total;
+                cur[t0 + j] += end - off[t0 + j];
+            }
+        lds_barrier();
         for (int t = tid; t < ntiles; t += kScatterLanes)
-            cur[t] += off[t] - (t ? off[t - 1] : 0u);
-        __syncthreads();
+            off[t] = 0;
+        lds_barrier();
     }
 }
 
@@ -474,16 +535,20 @@ __global__ void __launch_bounds__(kScatterLanes)
 // sums of the records' colours), then one add per word of each occupied
 // cell: plain where the tile has one chunk, atomic where chunks share it.
 // Colour sums come out in another order than the atomic path's per-sample
-// adds, equal to the rounding of that order.
+// adds, equal to the rounding of that order.  Several records of a lane are
+// in flight (one at a time, 2.36 ms per 2^28 three-colour FP32 records;
+// now 1.44).
 constexpr int kColourTile = 1 << kBinTileBitsColour;
+constexpr int kColourUnroll = 4;
 
-template <typename CT, typename CR, typename PR>
+template <typename CT, typename CR, typename PR, int NW>
 __global__ void __launch_bounds__(1024)
-    bin_accum_colour_kernel(const unsigned *sorted, const PR *pay_sorted,
-                            unsigned long long stride, int nr, const unsigned *start,
+    bin_accum_colour_kernel(const uint4 *sorted, int nr, const unsigned *start,
                             const unsigned *cstart, int ntiles, unsigned long long cells,
                             unsigned chunk, const unsigned *skip, CT *buf)
 {
+    constexpr int kReal = (int)sizeof(PR) / 4;
+    constexpr int NR = (NW - 1) / kReal < 4 ? (NW - 1) / kReal : 4;
     extern __shared__ unsigned long long lds64[];
     double *col = reinterpret_cast<double *>(lds64);                 // [nr][kColourTile]
     unsigned *cnt = reinterpret_cast<unsigned *>(col + 4 * kColourTile); // [kColourTile]
@@ -514,28 +579,48 @@ __global__ void __launch_bounds__(1024)
     }
     __syncthreads();
     constexpr unsigned mask = kColourTile - 1;
-    for (unsigned i = s0 + threadIdx.x; i < s1; i += blockDim.x) {
-        const unsigned cw = tile_word(sorted[i] & mask);
-        atomicAdd(&cnt[cw], 1u);
-        for (int j = 0; j < nr; ++j)
-            atomicAdd(&col[j * kColourTile + cw],
-                      (double)pay_sorted[(unsigned long long)j * stride + i]);
+    for (unsigned i0 = s0 + threadIdx.x; i0 < s1; i0 += blockDim.x * kColourUnroll) {
+        unsigned v[kColourUnroll][NW];
+#pragma unroll
+        for (int u = 0; u < kColourUnroll; ++u) {
+            const unsigned i = i0 + (unsigned)u * blockDim.x;
+            const uint4 *src = sorted + (size_t)(i < s1 ? i : i0) * (NW / 4);
+#pragma unroll
+            for (int q = 0; q < NW / 4; ++q) {
+                const uint4 x = src[q];
+                v[u][4 * q] = x.x;
+                v[u][4 * q + 1] = x.y;
+                v[u][4 * q + 2] = x.z;
+                v[u][4 * q + 3] = x.w;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kColourUnroll; ++u) {
+            if (i0 + (unsigned)u * blockDim.x >= s1)
+                break;
+            const unsigned cw = tile_word(v[u][0] & mask);
+            atomicAdd(&cnt[cw], 1u);
+#pragma unroll
+            for (int j = 0; j < NR; ++j)
+                if (j < nr)
+                    atomicAdd(&col[j * kColourTile + cw], get_real<PR>(&v[u][1 + j * kReal]));
+        }
     }
     __syncthreads();
     const int words = 1 + nr;
     for (unsigned i = threadIdx.x; i < ncell; i += blockDim.x) {
         const unsigned cw = tile_word(i);
-        const unsigned v = cnt[cw];
-        if (!v)
+        const unsigned n = cnt[cw];
+        if (!n)
             continue;
         CT *cell = buf + (c0 + i) * (unsigned long long)words;
         CR *colour = reinterpret_cast<CR *>(cell + 1);
         if (shared) {
-            atomicAdd(cell, (CT)v);
+            atomicAdd(cell, (CT)n);
             for (int j = 0; j < nr; ++j)
                 unsafeAtomicAdd(&colour[j], (CR)col[j * kColourTile + cw]);
         } else {
-            *cell += (CT)v;
+            *cell += (CT)n;
             for (int j = 0; j < nr; ++j)
                 colour[j] += (CR)col[j * kColourTile + cw];
         }
@@ -545,6 +630,84 @@ __global__ void __launch_bounds__(1024)
 constexpr size_t accum_colour_lds()
 {
     return sizeof(double) * 4 * kColourTile + sizeof(unsigned) * kColourTile;
+}
+
+// the scatter's records a lane per chunk, by record words and tiles: what
+// the LDS holds
+constexpr int kScatterTiles = 3072; // tiles beside the larger chunks
+constexpr int scatter_per(int nw, bool many) { return nw == 4 ? (many ? 4 : 8) : nw == 8 ? (many ? 2 : 4) : (many ? 1 : 2); }
+
+// the colour kernels of a record size: scatter, then (with the work items
+// known) accumulation
+template <typename PR, int NW>
+void launch_scatter_pay(const BinScratch &b, unsigned long long n, unsigned long long per,
+                        int nblocks, int tile_bits, int ntiles, int r, hipStream_t s)
+{
+    auto go = [&](auto kern, int per_lane) {
+        hipLaunchKernelGGL(kern, dim3(nblocks), dim3(kScatterLanes),
+                           scatter_pay_lds(ntiles, per_lane, NW), s, b.rec, (const PR *)b.pay, n,
+                           per, tile_bits, ntiles, b.hist, b.start, (uint4 *)b.pay_sorted,
+                           b.capacity, r);
+    };
+    if (ntiles <= kScatterTiles)
+        go(bin_scatter_pay_kernel<scatter_per(NW, false), NW, PR>, scatter_per(NW, false));
+    else
+        go(bin_scatter_pay_kernel<scatter_per(NW, true), NW, PR>, scatter_per(NW, true));
+}
+
+template <typename PR, int NW>
+void launch_accum_colour(const BinScratch &b, unsigned items, int r, const unsigned *cstart,
+                         int ntiles, unsigned long long cells, unsigned chunk,
+                         const unsigned *skip, void *buf, int word_bytes, hipStream_t s)
+{
+    // 8-byte words hold u64 counts and f64 sums, 4-byte words u32 and f32
+    // (the float build); the records' colours are the walker's reals
+    if (word_bytes == 8)
+        hipLaunchKernelGGL((bin_accum_colour_kernel<unsigned long long, double, PR, NW>),
+                           dim3(items), dim3(1024), accum_colour_lds(), s,
+                           (const uint4 *)b.pay_sorted, r, b.start, cstart, ntiles, cells, chunk,
+                           skip, (unsigned long long *)buf);
+    else
+        hipLaunchKernelGGL((bin_accum_colour_kernel<unsigned, float, PR, NW>), dim3(items),
+                           dim3(1024), accum_colour_lds(), s, (const uint4 *)b.pay_sorted, r,
+                           b.start, cstart, ntiles, cells, chunk, skip, (unsigned *)buf);
+}
+
+// f(a walker's real, the record's words) for a flame of r colours
+template <typename F> void with_colour_record(int r, int real_bytes, F &&f)
+{
+    if (real_bytes == 8) {
+        if (r <= 3)
+            f(double(), std::integral_constant<int, colour_record_words(3, 8)>());
+        else
+            f(double(), std::integral_constant<int, colour_record_words(4, 8)>());
+    } else {
+        if (r <= 3)
+            f(float(), std::integral_constant<int, colour_record_words(3, 4)>());
+        else
+            f(float(), std::integral_constant<int, colour_record_words(4, 4)>());
+    }
+}
+
+template <typename PR, int NW> hipError_t prepare_colour()
+{
+    auto limit = [](const void *k, size_t bytes) {
+        return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    };
+    static_assert(scatter_pay_lds(kScatterTiles, scatter_per(NW, false), NW) <= 160 * 1024, "scatter chunk beyond the LDS");
+    static_assert(scatter_pay_lds(kBinMaxTiles, scatter_per(NW, true), NW) <= 160 * 1024, "scatter chunk beyond the LDS");
+    hipError_t e = limit((const void *)bin_scatter_pay_kernel<scatter_per(NW, false), NW, PR>,
+                         scatter_pay_lds(kScatterTiles, scatter_per(NW, false), NW));
+    if (e == hipSuccess)
+        e = limit((const void *)bin_scatter_pay_kernel<scatter_per(NW, true), NW, PR>,
+                  scatter_pay_lds(kBinMaxTiles, scatter_per(NW, true), NW));
+    if (e == hipSuccess)
+        e = limit((const void *)bin_accum_colour_kernel<unsigned long long, double, PR, NW>,
+                  accum_colour_lds());
+    if (e == hipSuccess)
+        e = limit((const void *)bin_accum_colour_kernel<unsigned, float, PR, NW>,
+                  accum_colour_lds());
+    return e;
 }
 
 int grid_for(unsigned long long n, int block)
@@ -603,7 +766,6 @@ int launch_bin_accumulate(const BinScratch &b, unsigned long long n_records,
     unsigned *cstart = b.total + ntiles;
     hipLaunchKernelGGL(bin_tilescan_kernel, dim3(1), dim3(1024), 0, s, b.total, ntiles, chunk,
                        b.start, cstart);
-    const unsigned long long stride = b.capacity;
     if (r == 0) {
         if (ntiles <= 4096)
             hipLaunchKernelGGL(bin_scatter_kernel<32>, dim3(nblocks), dim3(kScatterLanes),
@@ -613,22 +775,11 @@ int launch_bin_accumulate(const BinScratch &b, unsigned long long n_records,
             hipLaunchKernelGGL(bin_scatter_kernel<16>, dim3(nblocks), dim3(kScatterLanes),
                                scatter_lds(ntiles, 16), s, b.rec, n_records, per, tile_bits,
                                ntiles, b.hist, b.start, b.sorted);
-    } else if (real_bytes == 8) {
-        hipLaunchKernelGGL((bin_scatter_pay_kernel<8, double>), dim3(nblocks),
-                           dim3(kScatterLanes), scatter_pay_lds(ntiles, 8, 8), s, b.rec,
-                           (const double *)b.pay, n_records, per, tile_bits, ntiles, b.hist,
-                           b.start, b.sorted, (double *)b.pay_sorted, stride, r);
     } else {
-        if (ntiles <= 4096)
-            hipLaunchKernelGGL((bin_scatter_pay_kernel<16, float>), dim3(nblocks),
-                               dim3(kScatterLanes), scatter_pay_lds(ntiles, 16, 4), s, b.rec,
-                               (const float *)b.pay, n_records, per, tile_bits, ntiles, b.hist,
-                               b.start, b.sorted, (float *)b.pay_sorted, stride, r);
-        else
-            hipLaunchKernelGGL((bin_scatter_pay_kernel<8, float>), dim3(nblocks),
-                               dim3(kScatterLanes), scatter_pay_lds(ntiles, 8, 4), s, b.rec,
-                               (const float *)b.pay, n_records, per, tile_bits, ntiles, b.hist,
-                               b.start, b.sorted, (float *)b.pay_sorted, stride, r);
+        with_colour_record(r, real_bytes, [&](auto real, auto words) {
+            launch_scatter_pay<decltype(real), decltype(words)::value>(b, n_records, per, nblocks,
+                                                                       tile_bits, ntiles, r, s);
+        });
     }
     // accumulation work items (at most ntiles + n_records / chunk in all)
     const unsigned items = (unsigned)((unsigned long long)ntiles + n_records / chunk);
@@ -644,25 +795,14 @@ int launch_bin_accumulate(const BinScratch &b, unsigned long long n_records,
                                chunk, skip, (unsigned *)buf);
         return (int)hipGetLastError();
     }
-    // colour: 8-byte words hold u64 counts and f64 sums, 4-byte words u32
-    // and f32 (the float build); the records' colours are the walker's reals
-    if (word_bytes == 8 && real_bytes == 8)
-        hipLaunchKernelGGL((bin_accum_colour_kernel<unsigned long long, double, double>),
-                           dim3(items), dim3(1024), accum_colour_lds(), s, b.sorted,
-                           (const double *)b.pay_sorted, stride, r, b.start, cstart, ntiles,
-                           cells, chunk, skip, (unsigned long long *)buf);
-    else if (word_bytes == 8)
-        hipLaunchKernelGGL((bin_accum_colour_kernel<unsigned long long, double, float>),
-                           dim3(items), dim3(1024), accum_colour_lds(), s, b.sorted,
-                           (const float *)b.pay_sorted, stride, r, b.start, cstart, ntiles,
-                           cells, chunk, skip, (unsigned long long *)buf);
-    else
-        hipLaunchKernelGGL((bin_accum_colour_kernel<unsigned, float, float>), dim3(items),
-                           dim3(1024), accum_colour_lds(), s, b.sorted,
-                           (const float *)b.pay_sorted, stride, r, b.start, cstart, ntiles,
-                           cells, chunk, skip, (unsigned *)buf);
+    with_colour_record(r, real_bytes, [&](auto real, auto words) {
+        launch_accum_colour<decltype(real), decltype(words)::value>(
+            b, items, r, cstart, ntiles, cells, chunk, skip, buf, word_bytes, s);
+    });
     return (int)hipGetLastError();
 }
+
+int colour_record_bytes(int r, int real_bytes) { return 4 * colour_record_words(r, real_bytes); }
 
 int prepare_bin_kernels()
 {
@@ -676,9 +816,6 @@ int prepare_bin_kernels()
     // the scatter kernel: chunks of 32 records a lane up to 4096 tiles, of
     // 16 up to 8192
     static_assert(scatter_lds(4096, 32) <= 160 * 1024, "scatter chunk beyond the LDS");
-    static_assert(scatter_pay_lds(4096, 16, 4) <= 160 * 1024, "scatter chunk beyond the LDS");
-    static_assert(scatter_pay_lds(kBinMaxTiles, 8, 4) <= 160 * 1024, "scatter chunk beyond the LDS");
-    static_assert(scatter_pay_lds(kBinMaxTiles, 8, 8) <= 160 * 1024, "scatter chunk beyond the LDS");
     static_assert(accum_colour_lds() <= 160 * 1024, "colour tile beyond the LDS");
     static_assert(scatter_lds(kBinMaxTiles, 16) <= 160 * 1024, "scatter chunk beyond the LDS");
     if (e == hipSuccess)
@@ -689,29 +826,14 @@ int prepare_bin_kernels()
         e = hipFuncSetAttribute((const void *)bin_scatter_kernel<16>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)scatter_lds(kBinMaxTiles, 16));
-    // colour flames: f32 colours in chunks of 16 records a lane up to 4096
-    // tiles, of 8 up to 8192; f64 colours in chunks of 8; the accumulation's
-    // tile of counts and four f64 sums
     if (e == hipSuccess)
-        e = hipFuncSetAttribute((const void *)bin_scatter_pay_kernel<16, float>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)scatter_pay_lds(4096, 16, 4));
+        e = prepare_colour<float, 4>();
     if (e == hipSuccess)
-        e = hipFuncSetAttribute((const void *)bin_scatter_pay_kernel<8, float>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)scatter_pay_lds(kBinMaxTiles, 8, 4));
+        e = prepare_colour<float, 8>();
     if (e == hipSuccess)
-        e = hipFuncSetAttribute((const void *)bin_scatter_pay_kernel<8, double>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)scatter_pay_lds(kBinMaxTiles, 8, 8));
-    const void *acc[] = {
-        (const void *)bin_accum_colour_kernel<unsigned long long, double, double>,
-        (const void *)bin_accum_colour_kernel<unsigned long long, double, float>,
-        (const void *)bin_accum_colour_kernel<unsigned, float, float>};
-    for (const void *k : acc)
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)accum_colour_lds());
+        e = prepare_colour<double, 8>();
+    if (e == hipSuccess)
+        e = prepare_colour<double, 12>();
     return (int)e;
 }
 

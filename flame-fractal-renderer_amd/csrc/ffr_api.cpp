@@ -162,7 +162,8 @@ struct ffr_renderer {
     // split walkers: -1 chosen per render, 0 off (FFR_SPLIT)
     int split_pref = -1;
     BinScratch bin;
-    size_t bin_pay_bytes = 0; // bytes of bin.pay (and of bin.pay_sorted)
+    size_t bin_pay_bytes = 0;    // bytes of bin.pay
+    size_t bin_sorted_bytes = 0; // bytes of bin.pay_sorted
     // a colour flame whose renders made at least kBinColourAtomics global
     // atomic adds per sample: its later single renders take binned
     // accumulation (binned -1)
@@ -1164,19 +1165,19 @@ static hipError_t ensure_bin_scratch(ffr_renderer *r, uint64_t cap, int real_byt
     size_t have_rec = (size_t)r->bin.capacity * 4, have_sorted = have_rec;
     if (have_rec < cap * 4) {
         e = ensure_device((void **)&r->bin.rec, have_rec, (size_t)cap * 4);
-        if (e == hipSuccess)
+        if (e == hipSuccess && ncol == 0)
             e = ensure_device((void **)&r->bin.sorted, have_sorted, (size_t)cap * 4);
         r->bin.capacity = e == hipSuccess ? cap : 0;
     }
-    // colour flames: the records' colours, component i at i * capacity
+    // colour flames: the records' colours, component i at i * capacity, and
+    // the whole records in tile order
     if (e == hipSuccess && ncol > 0) {
         const size_t need = (size_t)ncol * (size_t)r->bin.capacity * (size_t)real_bytes;
-        size_t have_sorted_pay = r->bin_pay_bytes;
         e = ensure_device(&r->bin.pay, r->bin_pay_bytes, need);
         if (e == hipSuccess)
-            e = ensure_device(&r->bin.pay_sorted, have_sorted_pay, need);
-        if (e != hipSuccess)
-            r->bin_pay_bytes = 0;
+            e = ensure_device(&r->bin.pay_sorted, r->bin_sorted_bytes,
+                              (size_t)r->bin.capacity *
+                                  (size_t)colour_record_bytes(ncol, real_bytes));
     }
     size_t hist_bytes = r->bin_hist_words * 4;
     if (e == hipSuccess)

@@ -56,17 +56,19 @@ constexpr unsigned long long kBinRecordsPerBlock = 1ull << 18;
 constexpr unsigned long long kBinPassRecords = 1ull << 28;
 struct BinScratch {
     unsigned *rec = nullptr;     // records of one pass (cell index or kEmptyKey)
-    unsigned *sorted = nullptr;  // the same records grouped by tile
+    unsigned *sorted = nullptr;  // the same records grouped by tile (no colour)
     unsigned *hist = nullptr;    // per block of records, per tile: count, then offset
     unsigned *total = nullptr;   // per tile: records, then the first of its accumulation
                                  // work items (2 ntiles + 1 words)
     unsigned *start = nullptr;   // per tile: first slot of its region (ntiles + 1)
     unsigned long long capacity = 0; // records rec and sorted hold
     // colour flames: each record's colour, component i at i * capacity
-    // reals (float or double, as the walker's), and the same grouped by tile
+    // reals (float or double, as the walker's), and the records grouped by
+    // tile, whole ones of colour_record_bytes (`sorted` is not used)
     void *pay = nullptr;
     void *pay_sorted = nullptr;
 };
+int colour_record_bytes(int r, int real_bytes);
 size_t bin_scratch_hist_words(unsigned long long records, int ntiles);
 // sort the n_records records of b.rec by tile and add the counts into the
 // buffer (cells count words of word_bytes, no colour words)
