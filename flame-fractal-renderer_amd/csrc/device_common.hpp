@@ -68,9 +68,9 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t
 
 struct Stream {
     uint32_t k0, k1, w0, w1;
-    uint64_t n;       // index of the next word
-    uint64_t cache;   // word cache_n, when loaded with its even partner
-    uint64_t cache_n;
+    uint64_t n;     // index of the next word
+    uint64_t cache; // word n, when `have` (loaded with its even partner)
+    bool have;
 
     __device__ __forceinline__ void init(uint64_t seed, uint64_t walker)
     {
@@ -79,16 +79,23 @@ struct Stream {
         k1 = __builtin_amdgcn_readfirstlane((uint32_t)(seed >> 32));
         w0 = (uint32_t)walker;
         w1 = (uint32_t)(walker >> 32);
-        n = 0;
         cache = 0;
-        cache_n = ~0ull;
+        seek(0);
+    }
+
+    // the next word is word `at`
+    __device__ __forceinline__ void seek(uint64_t at)
+    {
+        n = at;
+        have = false;
     }
 
     __device__ __forceinline__ uint64_t next()
     {
         uint64_t w;
-        if (n == cache_n) {
+        if (have) {
             w = cache;
+            have = false;
         } else {
             uint64_t blk = n >> 1;
             uint32_t o0, o1, o2, o3;
@@ -96,13 +103,10 @@ struct Stream {
                           o2, o3);
             uint64_t lo = (uint64_t)o0 | ((uint64_t)o1 << 32);
             uint64_t hi = (uint64_t)o2 | ((uint64_t)o3 << 32);
-            if (n & 1) {
-                w = hi;
-            } else {
-                w = lo;
-                cache = hi;
-                cache_n = n + 1;
-            }
+            const bool odd = (n & 1) != 0;
+            w = odd ? hi : lo;
+            cache = hi;
+            have = !odd;
         }
         ++n;
         return w;
@@ -118,6 +122,16 @@ template <typename T> using global_ptr = T __attribute__((address_space(1))) *;
 template <typename T> __device__ __forceinline__ global_ptr<T> as_global(T *p)
 {
     return (global_ptr<T>)p;
+}
+
+// a float add to global memory without a result (relaxed, any order)
+__device__ __forceinline__ void global_add(global_ptr<float> p, float v)
+{
+    (void)__builtin_amdgcn_global_atomic_fadd_f32(p, v);
+}
+__device__ __forceinline__ void global_add(global_ptr<double> p, double v)
+{
+    (void)__builtin_amdgcn_global_atomic_fadd_f64(p, v);
 }
 
 // randNum (flame_rng.hpp:67-87): top 53 bits over 2^53 in double, top 24
@@ -201,8 +215,8 @@ template <> struct Consts<float> {
 
 template <typename R> __device__ __forceinline__ bool bad_value(R v)
 {
-    // utils/flame.hpp:26-29
-    return m_fabs(v) > Consts<R>::bad || v != v;
+    // utils/flame.hpp:26-29: beyond the limit, or NaN
+    return !(m_fabs(v) <= Consts<R>::bad);
 }
 
 } // namespace ffr

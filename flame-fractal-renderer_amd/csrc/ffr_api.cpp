@@ -190,6 +190,14 @@ struct ffr_renderer {
     uint64_t samples_asked = 0;
 };
 
+// the colour registers of the renderer's walker kernels (the build for three
+// is for 2-D flames)
+static int walk_nc(const ffr_renderer *r)
+{
+    const int nc = nc_class(r->spec.color_dims, r->vs);
+    return nc == 3 && r->spec.dims != 2 ? 4 : nc;
+}
+
 static int pick_variation_set(const uint32_t ts[4])
 {
     bool linear_only = true, basic = true;
@@ -299,6 +307,14 @@ static int setup_tables(ffr_renderer *r, const DeviceFlame<R> &d)
                                            " bytes exceeds the " + std::to_string(max_lds) +
                                            "-byte LDS of a workgroup");
     r->vs = pick_variation_set(d.type_set);
+    // the basic set's kernels add a zero times the mapped point where a list
+    // is short: the point is finite as long as the pre-affines cannot
+    // overflow from a point within the bad-value limit
+    if (r->vs == 1)
+        for (const XformSpec &x : r->spec.xforms)
+            for (int i = 0; i < 9; ++i)
+                if (std::fabs(x.preA[i]) > 1e15 || std::fabs(x.preb[i % 3]) > 1e15)
+                    r->vs = 2;
     r->chain_ok = r->vs == 0 /* linear only, final xform included */ && d.r <= 4 &&
                   d.slot_type.size() <= (size_t)kChainSlots;
     // every xform's post-affine is exactly the identity (entries 1.0 and
@@ -620,10 +636,7 @@ static void fill_args(ffr_renderer *r, const DeviceFlame<R> &d, WalkArgs<R> &a)
     a.bt0 = d.bt0;
     a.bt_stride = d.bt_stride;
     a.bt_nvmax = d.bt_nvmax;
-    a.bt_union = 0;
-    if (d.bt0 >= 0)
-        for (int x = 0; x < d.nxf; ++x)
-            a.bt_union |= (int)d.table[(size_t)(d.bt0 + x * d.bt_stride + 1)];
+    a.bt_union = d.bt_union;
     for (size_t j = 0; j < d.fin_type.size(); ++j) {
         a.fin_type[j] = d.fin_type[j];
         a.fin_off[j] = d.fin_off[j];
@@ -895,14 +908,6 @@ static int launch_walk_any(int mode, int dims, const WalkLaunch &L)
     }
 }
 
-// the colour-register class the walker kernel is built for (launch_walk)
-static int nc_class(int r, bool cache)
-{
-    if (cache && r <= 4)
-        return r == 0 ? 0 : 4;
-    return r == 0 ? 0 : (r <= 4 ? 4 : 128);
-}
-
 static int launch_walk_any(int mode, int dims, const WalkLaunch &L);
 
 // the table-driven walker kernel for a plan, its arguments at r->dargs
@@ -1086,7 +1091,7 @@ static int prepare_compiled(ffr_renderer *r, const DeviceFlame<R> &d, const Laun
     RtcKernel k;
     k.mode = r->mode;
     k.dims = r->spec.dims;
-    k.nc = nc_class(r->spec.color_dims, p.cache);
+    k.nc = walk_nc(r);
     k.vs = r->vs;
     k.cache = p.cache;
     k.block_max = p.cache ? cache_block_max(r->mode == MODE_F64_U64, r->vs) : 256;
@@ -1268,7 +1273,7 @@ static int launch_binned(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchP
             RtcKernel k;
             k.mode = r->mode;
             k.dims = r->spec.dims;
-            k.nc = ncol;
+            k.nc = walk_nc(r);
             k.vs = r->vs;
             k.block_max = kBinWalkBlock;
             k.bin = true;

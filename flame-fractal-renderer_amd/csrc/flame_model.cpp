@@ -464,7 +464,7 @@ XformLayout xform_layout(int dims, int color_dims)
     L.has_pre = o; o += 1;
     L.has_post = o; o += 1;
     L.color = o; o += color_dims;
-    L.stride = (o + 1) & ~1;
+    L.stride = (o + 3) & ~3; // (records begin on 16 bytes)
     return L;
 }
 
@@ -901,8 +901,8 @@ template <typename R> DeviceFlame<R> compile_flame(const FlameSpec &spec)
     // table layout
     d.lay = xform_layout(dims, r);
     std::vector<R> &T = d.table;
-    auto align2 = [](size_t n) { return (n + 1) & ~(size_t)1; };
-    T.assign(align2((size_t)d.nxf), (R)0);
+    auto align4 = [](size_t n) { return (n + 3) & ~(size_t)3; };
+    T.assign(align4((size_t)d.nxf), (R)0);
     for (int k = 0; k < d.nxf; ++k)
         T[(size_t)k] = d.cw[(size_t)k];
     auto put_xform = [&](const XformSpec &x) {
@@ -925,6 +925,11 @@ template <typename R> DeviceFlame<R> compile_flame(const FlameSpec &spec)
         if (hc)
             for (int i = 0; i < r; ++i)
                 X[d.lay.color + i] = (R)x.color[(size_t)i];
+        // 2-D records have no use for has_post (both affines always apply):
+        // its place holds the speed of the colour blend, 0 without a colour
+        // (the colour fields are then 0 too, so the blend keeps the colour)
+        if (dims == 2)
+            X[d.lay.has_post] = hc ? X[d.lay.speed] : (R)0;
         return base;
     };
     d.xf0 = (int)T.size();
@@ -1004,26 +1009,26 @@ template <typename R> DeviceFlame<R> compile_flame(const FlameSpec &spec)
                 basic = basic && code_of(v->type) >= 0;
         }
         if (basic) {
+            // at least three terms (linear of weight 0, which adds a zero,
+            // pads the shorter lists), whole 16 bytes
             d.bt_nvmax = nvmax;
-            d.bt_stride = 2 + 2 * nvmax;
+            d.bt_stride = (int)align4(2 * (size_t)std::max(nvmax, 3));
+            T.resize(align4(T.size()), (R)0);
             d.bt0 = (int)T.size();
             T.resize(T.size() + (size_t)(d.bt_stride * d.nxf), (R)0);
             for (int k = 0; k < d.nxf; ++k) {
                 R *B = T.data() + d.bt0 + (size_t)(k * d.bt_stride);
-                int mask = 0;
                 const auto &L = lists[(size_t)k];
-                B[0] = (R)(int)L.size();
                 for (size_t j = 0; j < L.size(); ++j) {
                     const int c = code_of(L[j]->type);
-                    mask |= 1 << c;
-                    B[2 + 2 * j] = (R)c;
-                    B[3 + 2 * j] = (R)L[j]->weight;
+                    d.bt_union |= 1 << c;
+                    B[2 * j] = basic_code_real<R>(c);
+                    B[2 * j + 1] = (R)L[j]->weight;
                 }
-                B[1] = (R)mask;
             }
         }
     }
-    T.resize(align2(T.size()), (R)0);
+    T.resize(align4(T.size()), (R)0);
     if (ns > 64)
         throw JsonError("flame has " + std::to_string(ns) +
                         " variation slots after merging the xforms' variation orders "

@@ -85,6 +85,18 @@ struct XformLayout {
 };
 XformLayout xform_layout(int dims, int color_dims);
 
+// A basic variation's code (0..5) as a real: values that the device compares
+// with inline constants
+template <typename R> constexpr R basic_code_real(int code)
+{
+    return code == 1   ? (R)1
+           : code == 2 ? (R)2
+           : code == 3 ? (R)4
+           : code == 4 ? (R)-1
+           : code == 5 ? (R)-2
+                       : (R)0;
+}
+
 template <typename R> struct DeviceFlame {
     int dims = 2, r = 0;
     int nxf = 0, n_ids = 0;
@@ -107,9 +119,11 @@ template <typename R> struct DeviceFlame {
     std::vector<int> fin_type, fin_off;
     // per-xform variation lists for 2-D flames whose variations are all of
     // the basic six (linear, sinusoidal, spherical, swirl, horseshoe,
-    // polar; codes 0..5): [count, code mask, (code, weight) x bt_nvmax]
-    // per xform in JSON order, at table offset bt0 (-1: not built)
-    int bt0 = -1, bt_stride = 0, bt_nvmax = 0;
+    // polar; codes 0..5): (code as a real, weight) pairs per xform in JSON
+    // order, at least three (padded with linear of weight 0), at table
+    // offset bt0 (-1: not built); bt_union: bit k set when some list holds
+    // code k
+    int bt0 = -1, bt_stride = 0, bt_nvmax = 0, bt_union = 0;
     uint32_t type_set[4] = {0, 0, 0, 0}; // bitset of variation types present
     int max_draws = 0;
 };

@@ -171,7 +171,7 @@ std::string flame_source(const WalkArgs<R> &a, const std::vector<R> &cw, const R
          "    extern __shared__ __align__(16) unsigned char smem[];\n";
     if (k.bin)
         s << "    ffr::walk_bin_tasks<" << bin_types(k.mode) << ", " << k.dims << ", "
-          << (k.nc > 0 ? 4 : 0) << ", " << k.vs << ">(*args, smem);\n}\n";
+          << k.nc << ", " << k.vs << ">(*args, smem);\n}\n";
     else
         s << "    ffr::walk_tasks<" << mode_types(k.mode) << ", " << k.dims << ", " << k.nc << ", "
           << k.vs << ", " << (k.cache ? "true" : "false") << ">(*args, smem);\n}\n";

@@ -81,8 +81,8 @@ template <typename R> __device__ __forceinline__ R dev_norm2sq(const R *x, int n
 // once per iteration: linear, sinusoidal, spherical, swirl, horseshoe,
 // polar (codes 0..5).  Each output is the expression calc2d / var_eval
 // evaluate for it (variations.hpp:169-208, 509-555), with the squared norm
-// and its root shared.  `need` has bit k set when some lane of the wave
-// uses code k; the others are left untouched.
+// and its root shared.  `need` has bit k set when the flame uses code k; the
+// others keep no particular value (no lane selects them).
 // 1.0 / x as the reference writes it for spherical and horseshoe: with
 // num_t = float that is a double division whose quotient is then rounded to
 // float.  Double rounding of a quotient is innocuous when the wide format
@@ -97,6 +97,12 @@ __device__ __forceinline__ void basic6(unsigned need, const R *t, R (&o)[6][2])
     const R EPS = Consts<R>::eps;
     const R x = t[0], y = t[1];
     const R n2sq = x * x + y * y;
+    // (defined without an instruction: a zero would be moved into each)
+#pragma unroll
+    for (int k = 1; k < 6; ++k) {
+        asm volatile("" : "=v"(o[k][0]));
+        asm volatile("" : "=v"(o[k][1]));
+    }
     o[0][0] = x;
     o[0][1] = y;
     if (need & 2u) {

@@ -119,6 +119,9 @@ template <int D> struct XformLay {
     static constexpr int preA = 0, preb = D * D, postA = D * D + D, postb = 2 * D * D + D,
                          speed = 2 * D * D + 2 * D, has_color = speed + 1, has_pre = speed + 2,
                          has_post = speed + 3, color = speed + 4;
+    // 2-D records: the speed of the colour blend, 0 without a colour (both
+    // affines always apply, so has_post has no use there)
+    static constexpr int blend = has_post;
 };
 
 // lanes per workgroup (= walkers per task) of the binned walker kernel
@@ -205,6 +208,13 @@ __host__ __device__ constexpr int chain_build_ns(int slots)
 __host__ __device__ constexpr bool chain_build_sh(bool shared, bool post_id, int slots)
 {
     return shared && post_id && slots <= 1;
+}
+
+// the colour registers a walker kernel is built for: none; exactly three
+// (2-D flames of the basic variations, set 1); up to four; more
+constexpr int nc_class(int r, int vs)
+{
+    return r == 0 ? 0 : r == 3 && vs == 1 ? 3 : r <= 4 ? 4 : 128;
 }
 
 #ifndef __HIPCC_RTC__
