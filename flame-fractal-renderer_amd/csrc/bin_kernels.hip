@@ -23,6 +23,7 @@
 //            atomic one where chunks share the tile)
 // A tile is kBinTileCells consecutive cells (dimension 0 fastest), whose
 // u32 counts fit the LDS of one workgroup.
+#include "bin_common.hpp"
 #include "util_kernels.hpp"
 
 #include <hip/hip_runtime.h>
@@ -272,17 +273,6 @@ __global__ void __launch_bounds__(kScatterLanes)
     }
 }
 
-// The LDS word of cell c of a tile: c with its low five bits (its bank)
-// turned by a hash of the rest.  Cells that flames occupy often share their
-// low bits (the Sierpinski tetrahedron's occupied cells of a row have x
-// digits that avoid y's and z's, so a few banks held them all and the
-// counts' atomics queued on them); the hash spreads each group of 32 cells
-// over the banks, one bank each.
-__device__ __forceinline__ unsigned tile_word(unsigned c)
-{
-    return c ^ (((c >> 5) * 0x9E3779B1u) >> 27);
-}
-
 // Tiles take very different shares of the records (the tetrahedron's
 // lowest slices hold thousands of occupied cells, its highest a few), and
 // one workgroup per tile left the device waiting on the largest.  So a tile
@@ -354,15 +344,6 @@ __global__ void __launch_bounds__(1024)
     }
 }
 
-// Workgroup barriers that order the LDS only: loads and stores of device
-// memory stay in flight across them.
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // Colour flames: the scatter also moves each record's colour.  The walker
 // leaves keys and colour components in arrays of their own; here a chunk's
 // records are read once, put into tile order in LDS as whole records of NW
@@ -376,37 +357,6 @@ constexpr size_t scatter_pay_lds(int ntiles, int per, int nw)
 {
     return sizeof(unsigned) * ((size_t)nw * (size_t)kScatterLanes * (size_t)per +
                                2 * (size_t)ntiles + 16);
-}
-
-// words of a colour record as the kernels below are built: the key and up
-// to three reals, or four, to whole 16 bytes
-constexpr int colour_record_words(int r, int real_bytes)
-{
-    return ((1 + (r <= 3 ? 3 : 4) * (real_bytes / 4)) + 3) / 4 * 4;
-}
-static_assert(colour_record_words(1, 4) == 4 && colour_record_words(4, 4) == 8 &&
-                  colour_record_words(1, 8) == 8 && colour_record_words(4, 8) == 12,
-              "the record sizes the colour kernels are built for");
-
-template <typename PR> __device__ __forceinline__ void put_real(unsigned *w, PR v);
-template <> __device__ __forceinline__ void put_real(unsigned *w, float v)
-{
-    w[0] = __float_as_uint(v);
-}
-template <> __device__ __forceinline__ void put_real(unsigned *w, double v)
-{
-    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-    w[0] = (unsigned)b;
-    w[1] = (unsigned)(b >> 32);
-}
-template <typename PR> __device__ __forceinline__ double get_real(const unsigned *w);
-template <> __device__ __forceinline__ double get_real<float>(const unsigned *w)
-{
-    return (double)__uint_as_float(w[0]);
-}
-template <> __device__ __forceinline__ double get_real<double>(const unsigned *w)
-{
-    return __longlong_as_double((long long)(((unsigned long long)w[1] << 32) | w[0]));
 }
 
 template <int PER, int NW, typename PR>
@@ -678,14 +628,14 @@ template <typename F> void with_colour_record(int r, int real_bytes, F &&f)
 {
     if (real_bytes == 8) {
         if (r <= 3)
-            f(double(), std::integral_constant<int, colour_record_words(3, 8)>());
+            f(double(), std::integral_constant<int, record_words(3, 8)>());
         else
-            f(double(), std::integral_constant<int, colour_record_words(4, 8)>());
+            f(double(), std::integral_constant<int, record_words(4, 8)>());
     } else {
         if (r <= 3)
-            f(float(), std::integral_constant<int, colour_record_words(3, 4)>());
+            f(float(), std::integral_constant<int, record_words(3, 4)>());
         else
-            f(float(), std::integral_constant<int, colour_record_words(4, 4)>());
+            f(float(), std::integral_constant<int, record_words(4, 4)>());
     }
 }
 
@@ -801,8 +751,6 @@ int launch_bin_accumulate(const BinScratch &b, unsigned long long n_records,
     });
     return (int)hipGetLastError();
 }
-
-int colour_record_bytes(int r, int real_bytes) { return 4 * colour_record_words(r, real_bytes); }
 
 int prepare_bin_kernels()
 {

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cmath>
 #include <condition_variable>
@@ -76,7 +77,212 @@ struct DevTables {
     int tab_reals = 0;
 };
 
+// grow a device allocation to at least `bytes` (contents not kept)
+hipError_t ensure_device(void **p, size_t &have, size_t bytes)
+{
+    if (have >= bytes)
+        return hipSuccess;
+    (void)hipFree(*p);
+    *p = nullptr;
+    have = 0;
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess)
+        have = bytes;
+    return e;
+}
+
 } // namespace
+
+// Miss records: the memory of a renderer's launches (or a batch's: its
+// kinds run one after another)
+struct MissMemory {
+    void *rec = nullptr, *sorted = nullptr, *info = nullptr, *ctrl = nullptr, *state = nullptr;
+    size_t rec_bytes = 0, sorted_bytes = 0, info_bytes = 0, ctrl_bytes = 0, state_bytes = 0;
+
+    hipError_t ensure(int groups, int lanes, unsigned chunks, int words, int real_bytes)
+    {
+        const size_t n = (size_t)chunks * miss_chunk(words) * (size_t)words * 4;
+        const size_t pause = real_bytes == 8 ? sizeof(WalkerPause<double>)
+                                             : sizeof(WalkerPause<float>);
+        hipError_t e = ensure_device(&rec, rec_bytes, n);
+        if (e == hipSuccess)
+            e = ensure_device(&sorted, sorted_bytes, n);
+        if (e == hipSuccess)
+            e = ensure_device(&info, info_bytes, (size_t)chunks * sizeof(MissChunk));
+        if (e == hipSuccess) // (the pool's counters in front)
+            e = ensure_device(&ctrl, ctrl_bytes,
+                              sizeof(MissCtrl) + (size_t)groups * sizeof(MissCtrl));
+        if (e == hipSuccess)
+            e = ensure_device(&state, state_bytes, (size_t)groups * (size_t)lanes * pause);
+        return e;
+    }
+    void free_all()
+    {
+        for (void *p : {rec, sorted, info, ctrl, state})
+            (void)hipFree(p);
+        *this = MissMemory();
+    }
+};
+
+// ... and the tiles of its flames
+struct MissTiles {
+    void *words = nullptr, *flames = nullptr;
+    size_t words_bytes = 0, flames_bytes = 0;
+    int tiles = 0, max_tiles = 0;
+    // host copies, alive until the device's ones were made
+    std::vector<unsigned> tile_flame;
+    std::vector<MissFlame> list;
+
+    // flames (buf, cells, r filled in) in tiles of 2^tile_bits cells
+    hipError_t set(const std::vector<MissFlame> &fl, int tile_bits, hipStream_t s)
+    {
+        auto same = [](const MissFlame &x, const MissFlame &y) {
+            return x.buf == y.buf && x.cells == y.cells && x.r == y.r;
+        };
+        if (tiles && fl.size() == list.size() &&
+            std::equal(fl.begin(), fl.end(), list.begin(), same))
+            return hipSuccess; // (the device has them)
+        // copies of the last call may still read the vectors
+        hipError_t e = hipStreamSynchronize(s);
+        if (e != hipSuccess)
+            return e;
+        list = fl;
+        tile_flame.clear();
+        max_tiles = 0;
+        for (size_t i = 0; i < list.size(); ++i) {
+            MissFlame &f = list[i];
+            f.tile0 = (int)tile_flame.size();
+            f.tiles = (int)((f.cells + (1ull << tile_bits) - 1) >> tile_bits);
+            max_tiles = std::max(max_tiles, f.tiles);
+            tile_flame.insert(tile_flame.end(), (size_t)f.tiles, (unsigned)i);
+        }
+        const int n = (int)tile_flame.size();
+        tiles = 0;
+        e = ensure_device(&words, words_bytes, ((size_t)n * 5 + 2) * 4);
+        if (e == hipSuccess)
+            e = ensure_device(&flames, flames_bytes, list.size() * sizeof(MissFlame));
+        if (e == hipSuccess)
+            e = hipMemcpyAsync((unsigned *)words + (size_t)n * 4 + 2, tile_flame.data(),
+                               (size_t)n * 4, hipMemcpyHostToDevice, s);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(flames, list.data(), list.size() * sizeof(MissFlame),
+                               hipMemcpyHostToDevice, s);
+        if (e == hipSuccess)
+            tiles = n;
+        return e;
+    }
+    void free_all()
+    {
+        (void)hipFree(words);
+        (void)hipFree(flames);
+        *this = MissTiles();
+    }
+};
+
+// The rounds (walker launch, then its records binned) of a render, the chunks
+// of its records, and the chunk from which its workgroups pause.  Where
+// every sample's record fits, one round is enough; else as many as the
+// expected misses (rate) fill and two more, and a last launch finishes with
+// atomics what is left then.
+struct MissRounds {
+    unsigned chunks = 0, limit = 0;
+    int rounds = 0;
+    bool last = false;
+};
+
+// The record memory (as much again holds the sorted records); at most a
+// sixteenth of the free memory.  The batch of 24 flames (32 GB of records)
+// took 216 ms with 1 GB, 195 with 2, 189 with 4 and 185 with 8; the 4K
+// colour flame (2.4 GB) 57.7, 56.7 and 55.9 ms with 1, 2 and 4
+constexpr size_t kMissBytes = (size_t)4 << 30;
+// renders of fewer samples keep their atomics, and flames that miss little:
+// at 0.14 missed words a sample (4K colour flame) records took an FP32 render
+// from 82 to 56 ms, but an FP64 one, whose longer iterations hide the
+// atomics, from 28.3 to 30.7 ms
+constexpr uint64_t kMissMinSamples = 1ull << 24;
+constexpr double kMissWords32 = 0.05, kMissWords64 = 0.3;
+
+// rate: of the last render's samples those that missed (negative: unknown)
+static bool miss_worth(double rate, int cell_words, int real_bytes)
+{
+    return rate < 0 || rate * cell_words >= (real_bytes == 8 ? kMissWords64 : kMissWords32);
+}
+
+static MissRounds miss_rounds(const MissMemory &mem, uint64_t samples, uint64_t tasks, int groups,
+                              int lanes, int words, double rate)
+{
+    const uint64_t chunk = miss_chunk(words), chunk_bytes = chunk * (uint64_t)words * 4;
+    const uint64_t waves = ((uint64_t)lanes + 63) / 64;
+    // a wave ends each task, and each launch, with a chunk that is partly filled
+    const uint64_t all = samples / chunk + (tasks + (uint64_t)groups) * waves + 1;
+    uint64_t bytes = kMissBytes;
+    if (const char *e = std::getenv("FFR_MISS_BYTES"))
+        bytes = std::max<uint64_t>((uint64_t)std::atoll(e), 2 * chunk_bytes);
+    else if (mem.rec_bytes < std::min(bytes, all * chunk_bytes)) {
+        size_t free_b = 0, total_b = 0;
+        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess)
+            return MissRounds();
+        bytes = std::max<uint64_t>(mem.rec_bytes, std::min<uint64_t>(bytes, free_b / 16));
+    }
+    MissRounds m;
+    const uint64_t most = bytes / chunk_bytes;
+    if (all <= most) {
+        m.chunks = m.limit = (unsigned)all;
+        m.rounds = 1;
+        return m;
+    }
+    // (the next render may miss somewhat more)
+    rate = rate < 0 ? 0.75 : std::min(1.0, 0.02 + 1.3 * rate);
+    const uint64_t spare = std::min<uint64_t>(most / 2, (uint64_t)groups * waves);
+    m.chunks = (unsigned)most;
+    m.limit = (unsigned)(most - spare);
+    const double expect = (double)samples * rate / (double)chunk +
+                          0.5 * (double)tasks * (double)waves;
+    m.rounds = most ? (int)std::min(expect / ((double)m.limit - 0.25 * (double)spare) + 2.0, 4096.0)
+                    : 0;
+    m.last = true;
+    return m;
+}
+
+static MissScratch miss_scratch(const MissMemory &m, const MissTiles &t, unsigned chunks,
+                                int groups, int words, int real_bytes, int cu_count)
+{
+    MissScratch x;
+    x.rec = (unsigned *)m.rec;
+    x.sorted = (unsigned *)m.sorted;
+    x.info = (MissChunk *)m.info;
+    x.pool = (MissPool *)m.ctrl;
+    x.ctrl = (MissCtrl *)m.ctrl + 1;
+    x.state = m.state;
+    unsigned *w = (unsigned *)t.words;
+    x.count = w;
+    x.cursor = w + t.tiles;
+    x.start = w + 2 * (size_t)t.tiles;
+    x.cstart = w + 3 * (size_t)t.tiles + 1;
+    x.tile_flame = w + 4 * (size_t)t.tiles + 2;
+    x.flames = (MissFlame *)t.flames;
+    x.chunks = chunks;
+    x.groups = groups;
+    x.words = words;
+    x.real_bytes = real_bytes;
+    x.tiles = t.tiles;
+    x.max_tiles = t.max_tiles;
+    x.cu_count = cu_count;
+    return x;
+}
+
+static MissArgs miss_args(const MissScratch &x, unsigned limit)
+{
+    return MissArgs{x.rec, x.info, x.pool, x.ctrl, x.state, x.chunks, limit};
+}
+
+static int prepare_miss_once()
+{
+    static std::once_flag once;
+    static int rc = 0;
+    std::call_once(once, [] { rc = prepare_miss_kernels(); });
+    return rc;
+}
 
 struct ffr_renderer {
     ffr_options opt{};
@@ -161,6 +367,14 @@ struct ffr_renderer {
     int bin_pref = -1;
     // split walkers: -1 chosen per render, 0 off (FFR_SPLIT)
     int split_pref = -1;
+    // miss records: -1 chosen per render, 0 off (FFR_MISS); the share of the
+    // samples expected to miss the cell cache (measured by each render)
+    int miss_pref = -1;
+    MissMemory miss_memory;
+    MissTiles miss_tiles;
+    double miss_rate = -1;
+    bool last_cached = false; // the last render's misses count (a hashed cache)
+    MissRounds miss_last; // the last render's (memory and chunks)
     BinScratch bin;
     size_t bin_pay_bytes = 0;    // bytes of bin.pay
     size_t bin_sorted_bytes = 0; // bytes of bin.pay_sorted
@@ -467,6 +681,8 @@ int ffr_create(const char *flame_json, size_t len, const ffr_options *opt_in,
             r->bin_pref = std::atoi(e);
         if (const char *e = std::getenv("FFR_SPLIT"))
             r->split_pref = std::atoi(e) ? -1 : 0;
+        if (const char *e = std::getenv("FFR_MISS"))
+            r->miss_pref = std::atoi(e) ? -1 : 0;
         r->compiled_pref = opt.compiled < 0 ? -1 : (opt.compiled ? 1 : 0);
         if (const char *e = std::getenv("FFR_CHAIN_PER_CU"))
             r->chain_per_cu = std::atoi(e);
@@ -555,6 +771,8 @@ void ffr_destroy(ffr_renderer *r)
     (void)hipFree(r->bin.pay_sorted);
     (void)hipFree(r->wstate);
     (void)hipFree(r->dargs_bin);
+    r->miss_memory.free_all();
+    r->miss_tiles.free_all();
     for (int k = 0; k < 2; ++k) {
         if (r->pin[k])
             (void)hipHostFree(r->pin[k]);
@@ -910,8 +1128,9 @@ static int launch_walk_any(int mode, int dims, const WalkLaunch &L)
 
 static int launch_walk_any(int mode, int dims, const WalkLaunch &L);
 
-// the table-driven walker kernel for a plan, its arguments at r->dargs
-static int launch_table_kernel(ffr_renderer *r, const LaunchPlan &p, int nslots)
+// the table-driven walker kernel for a plan, its arguments at `dargs`
+static int launch_table_kernel(ffr_renderer *r, const LaunchPlan &p, int nslots,
+                               const void *dargs)
 {
     WalkLaunch L;
     L.nc = r->spec.color_dims;
@@ -926,14 +1145,14 @@ static int launch_table_kernel(ffr_renderer *r, const LaunchPlan &p, int nslots)
     L.block = p.block;
     L.lds = p.lds;
     L.stream = r->stream;
-    L.args = r->dargs;
+    L.args = dargs;
     return launch_walk_any(r->mode, r->spec.dims, L);
 }
 
-// the flame's compiled kernel, its arguments (the WalkDyn part) at r->dargs
-static int launch_compiled_kernel(ffr_renderer *r, const LaunchPlan &p, void *fn)
+// the flame's compiled kernel, its arguments (the WalkDyn part) at `dargs`
+static int launch_compiled_kernel(ffr_renderer *r, const LaunchPlan &p, void *fn,
+                                  const void *dargs)
 {
-    void *dargs = r->dargs;
     void *params[] = {&dargs};
     return (int)hipModuleLaunchKernel((hipFunction_t)fn, (unsigned)p.grid, 1, 1,
                                       (unsigned)p.block, 1, 1, (unsigned)p.lds, r->stream,
@@ -945,6 +1164,30 @@ static int launch_compiled_kernel(ffr_renderer *r, const LaunchPlan &p, void *fn
 // flame's kernel and probes whether it beats the table-driven one: the
 // compile (about half a second) pays off only over repeated renders.
 constexpr uint64_t kCompiledProbeSamples = 1ull << 33;
+
+// Miss records apply to a cached launch of a flame whose cells (and colour
+// sums) the binning kernels hold: not colour flames with 4-byte words, whose
+// float sums keep the per-sample float adds
+static bool miss_ok(const ffr_renderer *r)
+{
+    const int ncol = r->spec.color_dims;
+    return r->miss_pref < 0 && ncol <= 4 && !(ncol > 0 && r->word_bytes == 4) &&
+           r->cells < (ncol > 0 ? (1ull << 25) : (1ull << 28));
+}
+
+// ... and a kernel probe takes them as the last render did, where that
+// render's memory holds this launch's workgroups
+static bool miss_ready(const ffr_renderer *r, const LaunchPlan &p, int real_bytes, MissScratch &x)
+{
+    const size_t pause = real_bytes == 8 ? sizeof(WalkerPause<double>) : sizeof(WalkerPause<float>);
+    if (!r->miss_last.rounds || !p.cache || p.direct ||
+        r->miss_memory.ctrl_bytes < (size_t)(p.grid + 1) * sizeof(MissCtrl) ||
+        r->miss_memory.state_bytes < (size_t)p.grid * (size_t)p.block * pause)
+        return false;
+    x = miss_scratch(r->miss_memory, r->miss_tiles, r->miss_last.chunks, p.grid,
+                     record_words(walk_nc(r), real_bytes), real_bytes, r->cu_count);
+    return true;
+}
 
 // Time kernels for the coming render: n launch plans, each with the flame's
 // compiled kernel fns[k] or the table-driven one (nullptr), on the render's
@@ -962,10 +1205,15 @@ static int time_kernels(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchPl
     void *scratch = nullptr;
     HIP_TRY(hipMalloc(&scratch, ffr_buffer_bytes(r)));
     std::vector<std::vector<unsigned char>> h((size_t)n);
+    MissScratch miss;
     for (int k = 0; k < n; ++k) {
         WalkArgs<R> a;
         walk_args(r, d, plans[k], walker0, walkers, pb, pb, a);
         a.buf = scratch;
+        // (records of the last render's memory, which nothing bins; a
+        // workgroup that pauses ends its run there)
+        if (miss_ready(r, plans[k], (int)sizeof(R), miss))
+            a.miss = miss_args(miss, r->miss_last.limit);
         a.bv_limit = ~0ull; // the runs never stop at the bad-value limit
         h[(size_t)k].resize(sizeof a);
         std::memcpy(h[(size_t)k].data(), &a, sizeof a);
@@ -987,12 +1235,15 @@ static int time_kernels(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchPl
                 e = launch_reset_stats(r->dstats, r->dxf, r->nxf, r->stream)
                         ? hipErrorLaunchFailure
                         : hipSuccess;
+            if (e == hipSuccess && miss_ready(r, plans[k], (int)sizeof(R), miss))
+                e = (hipError_t)launch_miss_init(miss, plans[k].task_walkers, r->stream);
             if (e == hipSuccess)
                 e = hipEventRecord(r->ev0, r->stream);
             if (e == hipSuccess)
-                e = (hipError_t)(fns[k] ? launch_compiled_kernel(r, plans[k], fns[k])
+                e = (hipError_t)(fns[k] ? launch_compiled_kernel(r, plans[k], fns[k], r->dargs)
                                         : launch_table_kernel(r, plans[k],
-                                                              (int)d.slot_type.size()));
+                                                              (int)d.slot_type.size(),
+                                                              r->dargs));
             if (e == hipSuccess)
                 e = hipEventRecord(r->ev1, r->stream);
             if (e == hipSuccess)
@@ -1120,20 +1371,78 @@ template <typename R>
 static int launch_single(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchPlan &p,
                          uint64_t walker0, uint64_t walkers, uint64_t batch, uint64_t last)
 {
-    WalkArgs<R> a;
-    walk_args(r, d, p, walker0, walkers, batch, last, a);
+    WalkArgs<R> a[2];
+    walk_args(r, d, p, walker0, walkers, batch, last, a[0]);
+    // miss records (unless the cache is forced, or indexed directly, where
+    // nothing misses; their memory may be allocated here, so not while the
+    // stream is captured; without it the misses stay atomics)
+    const int words = record_words(walk_nc(r), (int)sizeof(R));
+    MissRounds m;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (p.cache && !p.direct && r->cache_pref < 0 && miss_ok(r) &&
+        miss_worth(r->miss_rate, r->cell_words, (int)sizeof(R)) &&
+        walkers * batch >= kMissMinSamples &&
+        hipStreamIsCapturing(r->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+        if (const int rc = prepare_miss_once())
+            return rc;
+        m = miss_rounds(r->miss_memory, walkers * batch,
+                        (walkers + p.task_walkers - 1) / p.task_walkers, p.grid, p.block, words,
+                        r->miss_rate);
+        hipError_t e = hipSuccess;
+        if (m.rounds)
+            e = r->miss_memory.ensure(p.grid, p.block, m.chunks, words, (int)sizeof(R));
+        if (m.rounds && e == hipSuccess) {
+            MissFlame f{};
+            f.buf = r->dbuf;
+            f.cells = r->cells;
+            f.r = r->spec.color_dims;
+            e = r->miss_tiles.set({f}, f.r > 0 ? kBinTileBitsColour : kBinTileBits, r->stream);
+        }
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            r->miss_memory.free_all();
+            m = MissRounds();
+        }
+    }
+    r->miss_last = m;
+    MissScratch x;
+    if (m.rounds) {
+        x = miss_scratch(r->miss_memory, r->miss_tiles, m.chunks, p.grid, words, (int)sizeof(R),
+                         r->cu_count);
+        a[0].miss = miss_args(x, m.limit);
+        // hints: with records, workgroups seeded alike have no atomics to
+        // queue on (the headline flame misses 3.0 instead of 3.5 %)
+        if (r->dhot && p.slots <= kHotSlots) {
+            a[0].hot = r->dhot;
+            a[0].hot_tag = 0x40000000u | ((unsigned)p.log2s << 8) | (unsigned)p.ways;
+        }
+    }
+    a[1] = a[0];
+    a[1].miss.chunks = 0;
     r->hargs.resize(sizeof a);
-    std::memcpy(r->hargs.data(), &a, sizeof a);
-    // a compiled flame's kernel reads only the launch part (WalkDyn, at the
-    // start of WalkArgs); its flame fields are constants
-    const size_t nbytes = r->rtc_fn ? sizeof(WalkDyn<R>) : sizeof a;
-    hipError_t e = hipMemcpyAsync(r->dargs, r->hargs.data(), nbytes, hipMemcpyHostToDevice,
-                                  r->stream);
+    std::memcpy(r->hargs.data(), a, sizeof a);
+    hipError_t e = hipMemcpyAsync(r->dargs, r->hargs.data(), m.last ? sizeof a : sizeof a[0],
+                                  hipMemcpyHostToDevice, r->stream);
     if (e != hipSuccess)
         return (int)e;
-    if (r->rtc_fn)
-        return launch_compiled_kernel(r, p, r->rtc_fn);
-    return launch_table_kernel(r, p, (int)d.slot_type.size());
+    // (a compiled flame's kernel reads only the launch part, WalkDyn, at the
+    // start of WalkArgs; its flame fields are constants)
+    auto walk = [&](int k) {
+        const void *args = (const unsigned char *)r->dargs + (size_t)k * sizeof a[0];
+        return r->rtc_fn ? launch_compiled_kernel(r, p, r->rtc_fn, args)
+                         : launch_table_kernel(r, p, (int)d.slot_type.size(), args);
+    };
+    if (!m.rounds)
+        return walk(0);
+    int rc = launch_miss_init(x, p.task_walkers, r->stream);
+    for (int k = 0; k < m.rounds && !rc; ++k) {
+        rc = walk(0);
+        if (!rc)
+            rc = launch_miss_round(x, (int)r->word_bytes, r->stream);
+    }
+    if (!rc && m.last)
+        rc = walk(1);
+    return rc;
 }
 
 // walkers and samples per walker of a render of `samples`
@@ -1143,20 +1452,6 @@ static void split_samples(const ffr_renderer *r, uint64_t samples, uint64_t &bat
     batch = r->opt.batch_size ? r->opt.batch_size : ffr_auto_batch(r, samples);
     walkers = (samples + batch - 1) / batch;
     last = samples - (walkers - 1) * batch;
-}
-
-// grow a device allocation to at least `bytes` (contents not kept)
-static hipError_t ensure_device(void **p, size_t &have, size_t bytes)
-{
-    if (have >= bytes)
-        return hipSuccess;
-    (void)hipFree(*p);
-    *p = nullptr;
-    have = 0;
-    hipError_t e = hipMalloc(p, bytes);
-    if (e == hipSuccess)
-        have = bytes;
-    return e;
 }
 
 // the scratch of binned accumulation for `cap` records: grown as needed and
@@ -1182,7 +1477,7 @@ static hipError_t ensure_bin_scratch(ffr_renderer *r, uint64_t cap, int real_byt
         if (e == hipSuccess)
             e = ensure_device(&r->bin.pay_sorted, r->bin_sorted_bytes,
                               (size_t)r->bin.capacity *
-                                  (size_t)colour_record_bytes(ncol, real_bytes));
+                                  (size_t)(4 * record_words(ncol, real_bytes)));
     }
     size_t hist_bytes = r->bin_hist_words * 4;
     if (e == hipSuccess)
@@ -1388,7 +1683,7 @@ static int launch_split_render(ffr_renderer *r, const DeviceFlame<R> &d, const L
                                &r->dstats->split_fail);
     if (rc)
         return rc;
-    return launch_table_kernel(r, fb, (int)d.slot_type.size());
+    return launch_table_kernel(r, fb, (int)d.slot_type.size(), r->dargs);
 }
 
 static int launch(ffr_renderer *r, uint64_t samples)
@@ -1398,6 +1693,7 @@ static int launch(ffr_renderer *r, uint64_t samples)
     LaunchPlan p = plan_launch(r, walkers, batch, renderer_shape(r));
     LaunchPlan fb;
     r->last_split = false;
+    r->last_cached = p.cache && !p.direct && !p.bin && !p.split_log2;
     if (p.split_log2) {
         // (its scratch may be allocated here, so not while the stream is
         // captured; without the memory for it the walkers run unsplit)
@@ -1506,6 +1802,9 @@ static int finish(ffr_renderer *r, ffr_stats *out)
             r->last_split = false;
         }
         r->last_bad = st.n_bad;
+        if (r->last_cached && st.s_iter)
+            r->miss_rate = (double)(st.atomics - st.flush_atomics) / (double)r->cell_words /
+                           (double)st.s_iter;
         r->last_atomics = st.atomics;
         r->last_flush_atomics = st.flush_atomics;
         // a colour flame whose samples missed the LDS cache often enough

@@ -64,11 +64,10 @@ struct BinScratch {
     unsigned long long capacity = 0; // records rec and sorted hold
     // colour flames: each record's colour, component i at i * capacity
     // reals (float or double, as the walker's), and the records grouped by
-    // tile, whole ones of colour_record_bytes (`sorted` is not used)
+    // tile, whole ones of record_words (`sorted` is not used)
     void *pay = nullptr;
     void *pay_sorted = nullptr;
 };
-int colour_record_bytes(int r, int real_bytes);
 size_t bin_scratch_hist_words(unsigned long long records, int ntiles);
 // sort the n_records records of b.rec by tile and add the counts into the
 // buffer (cells count words of word_bytes, no colour words)
@@ -80,6 +79,37 @@ int launch_bin_accumulate(const BinScratch &b, unsigned long long n_records,
                           int real_bytes, hipStream_t s, const unsigned *skip = nullptr);
 // set the accumulate kernel's LDS limit (outside any stream capture)
 int prepare_bin_kernels();
+
+// Binning of miss records (miss_kernels.hip).  A flame of a launch: its
+// buffer, and its tiles among the launch's
+struct MissFlame {
+    void *buf;
+    unsigned long long cells;
+    int tile0, tiles;
+    int r;
+    int pad;
+};
+// the device arrays of a launch's miss records
+struct MissScratch {
+    unsigned *rec = nullptr;    // [chunks][miss_chunk] records of `words` words
+    unsigned *sorted = nullptr; // as many, in tile order
+    MissChunk *info = nullptr;  // [chunks]
+    MissPool *pool = nullptr;
+    MissCtrl *ctrl = nullptr;   // [groups]
+    void *state = nullptr;      // [groups][lanes] paused walkers
+    unsigned *count = nullptr, *cursor = nullptr; // [tiles]
+    unsigned *start = nullptr, *cstart = nullptr; // [tiles + 1]
+    unsigned *tile_flame = nullptr;               // [tiles]
+    MissFlame *flames = nullptr;
+    unsigned chunks = 0;
+    int groups = 0, words = 0, real_bytes = 4, tiles = 0, max_tiles = 0, cu_count = 256;
+};
+// no chunk taken, and the workgroups' first tasks (task_walkers apart)
+int launch_miss_init(const MissScratch &x, uint64_t task_walkers, hipStream_t s);
+// bin the chunks' records into the flames' buffers
+int launch_miss_round(const MissScratch &x, int word_bytes, hipStream_t s);
+// set the kernels' LDS limits (outside any stream capture)
+int prepare_miss_kernels();
 
 // the staging memory of ffr_add_buffer_noalloc: a file-scope device array
 // of this many bytes per GPU (noalloc.hip)

@@ -13,7 +13,7 @@ struct DevStats {
     unsigned long long s_iter;
     unsigned long long s_plot;
     unsigned long long n_bad;   // bad values seen; > limit stops new walkers
-    unsigned long long atomics; // global atomic adds on the buffer (misses, flushes)
+    unsigned long long atomics; // words of misses (atomics or records) and cache flushes
     unsigned long long flush_atomics; // of those, the LDS cell-cache flushes
     double pmin[3];
     double pmax[3];
@@ -27,6 +27,73 @@ struct DevStats {
 constexpr int kMaxSlots = 64;     // variation slots per flame
 constexpr int kMaxFinalVars = 16; // variations of the final xform
 constexpr int kMaxXforms = 1024;  // xforms after removing weight 0
+
+// Miss records (miss_kernels.hip): a cached walker launch writes the cell
+// updates that miss its LDS cell cache as records instead of adding them
+// with global atomics; a pass of kernels behind it bins the records into the
+// buffers.  Each wave fills a chunk of the launch's record memory at a time
+// (miss_chunk records, of one flame) and takes the next from a counter, so
+// that the memory goes where the misses are and all workgroups run until it
+// is used up: from chunk `limit` on (a chunk per wave is then left) a
+// workgroup pauses, its lanes leave their walkers in `state`, and the next
+// launch goes on.  The last launch of a render has no chunks: it finishes
+// what is left with atomics.
+struct MissCtrl {
+    uint64_t next;   // first walker of the workgroup's next task, or the paused
+                     // task of the queue (batched launches)
+    unsigned resume; // that task was paused
+    unsigned pad;
+};
+struct MissPool {
+    unsigned next; // chunks taken (past `chunks` where the last were gone)
+    unsigned used; // chunks to bin
+};
+struct MissChunk {
+    unsigned flame, n; // its records
+};
+struct MissArgs {
+    void *rec;       // [chunks][miss_chunk] records
+    MissChunk *info; // [chunks]
+    MissPool *pool;
+    MissCtrl *ctrl;  // [workgroup]; nullptr: no miss records
+    void *state;     // [workgroup][lane] WalkerPause
+    unsigned chunks; // 0 in the last launch
+    unsigned limit;
+};
+// LDS of a workgroup (256 bytes are kept for it and the task queue): per
+// wave [chunk u32 | records in it u32]; the arguments, which are read where
+// they are used; a wave of the workgroup took a chunk past the limit
+struct MissLds {
+    unsigned long long wave[16];
+    MissArgs args;
+    unsigned full;
+};
+static_assert(sizeof(MissLds) <= 240, "more static LDS than the cell cache leaves");
+constexpr unsigned kNoChunk = 0xFFFFFFFFu;
+constexpr unsigned kMissFull = 1u << 20; // records of "no chunk": past any chunk's
+template <typename R> struct WalkerPause {
+    R p[3];
+    R c[4];
+    uint64_t n;  // stream position
+    uint64_t it; // iterations done
+    uint64_t wl; // the walker, or kNoWalker
+};
+constexpr uint64_t kNoWalker = ~0ull;
+// iterations of a lane between two looks whether to pause, and between two
+// flushes of its packed selection counts (a byte each: at most 255)
+constexpr unsigned kWalkBlock = 128;
+
+// 32-bit words of a record: the cell, and for colour flames as many reals as
+// the kernel has colour registers (nc 3 or 4), to whole 16 bytes
+__host__ __device__ constexpr int record_words(int nc, int real_bytes)
+{
+    return nc == 0 ? 1 : (1 + (nc <= 3 ? 3 : 4) * (real_bytes / 4) + 3) / 4 * 4;
+}
+// records of a chunk: 64 KB of counts' or FP32 colour records
+__host__ __device__ constexpr unsigned miss_chunk(int words) { return words == 1 ? 16384u : 4096u; }
+static_assert(record_words(1, 4) == 4 && record_words(4, 4) == 8 && record_words(1, 8) == 8 &&
+                  record_words(4, 8) == 12,
+              "the record sizes the binning kernels are built for");
 
 // The walker kernel's arguments in two parts.  WalkDyn holds what changes
 // from launch to launch: device addresses, seed and walker positions, the
@@ -85,6 +152,7 @@ template <typename R> struct WalkDyn {
     uint64_t split_len; // iterations per segment
     int split_log2;     // log2 of the segments per walker
     int split_warm;     // iterations a segment runs before its first
+    MissArgs miss;      // miss records of a single flame's launch
 };
 
 template <typename R> struct WalkArgs : WalkDyn<R> {
@@ -239,6 +307,7 @@ struct WalkLaunch {
     bool chain_diag = false;          // ... and that matrix diagonal
     bool bin = false;                 // binned accumulation (walk_bin_kernel)
     bool split = false;               // split walkers (split_kernel)
+    MissArgs miss{};                  // miss records of a batched launch
 };
 #endif // __HIPCC_RTC__
 

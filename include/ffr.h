@@ -108,10 +108,11 @@ typedef struct ffr_stats {
     double pt_min[3];         /* getPointExtremes (cumulative)                         */
     double pt_max[3];
     double kernel_ms;         /* device time of the last render's kernel (HIP events)  */
-    uint64_t atomics;         /* global atomic adds of the last render on the buffer:
-                                 one per word of a cell update that missed the LDS
-                                 cell cache or flushed it (no reference counterpart);
-                                 0 when its walkers ran split                         */
+    uint64_t atomics;         /* words of the last render's updates of the buffer past
+                                 the LDS cell cache: its flushes, and the misses, which
+                                 are global atomic adds or, in renders of 2^24 samples
+                                 or more that miss enough, records that are binned; 0
+                                 when its walkers ran split (no reference counterpart) */
     uint64_t flush_atomics;   /* of those, the LDS cell-cache flushes                   */
     uint32_t wave_per_walker; /* 1: the last render gave each walker a wavefront or
                                  more (few walkers of a linear flame, up to four

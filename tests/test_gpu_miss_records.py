@@ -1,0 +1,115 @@
+"""Cell updates past the LDS cell cache kept as records and binned: buffers,
+counts and statistics equal those of the same render with every miss an
+atomic (FFR_MISS=0) exactly, colour sums to the rounding of their order of
+addition (n additions of f64 values of one sign: under 1e-12 relative at the
+1e3..1e4 samples a cell has here).
+
+Record memory from two chunks (walkers pause every few iterations, and the
+last launch finishes with atomics) to enough for one round; one to four
+colour components and none, FP32 and FP64 walkers, 4-byte counts, three
+dimensions; renders of several flames in one launch; bad values."""
+
+import numpy as np
+import pytest
+
+import flames as TF
+from conftest import read_flame
+
+pytestmark = pytest.mark.gpu
+
+SEED = 0x5EED0021
+SAMPLES = 17_000_003  # (renders under 2^24 samples keep their atomics)
+
+
+def spread_2d(size):
+    """A count-only flame over many cells."""
+    text = read_flame("sierpinski_1024.json")
+    assert "[1024, 1024]" in text
+    return text.replace("[1024, 1024]", f"[{size}, {size}]")
+
+
+def compare(a, b):
+    wa, wb = a.read_buffer(), b.read_buffer()
+    assert np.array_equal(a.counts(wa), b.counts(wb))
+    if a.color_dims:
+        ca, cb = a.colors(wa), b.colors(wb)
+        assert np.allclose(ca, cb, rtol=1e-12, atol=1e-12 * np.abs(cb).max())
+    assert a.samples_iterated == b.samples_iterated
+    assert a.samples_plotted == b.samples_plotted
+    assert np.array_equal(a.xform_distribution(), b.xform_distribution())
+    assert a.point_extremes == b.point_extremes
+
+
+def pair(ffr, monkeypatch, text, **kw):
+    a = ffr.BufferRenderer(text, seed=SEED, **kw)
+    monkeypatch.setenv("FFR_MISS", "0")
+    b = ffr.BufferRenderer(text, seed=SEED, **kw)
+    monkeypatch.delenv("FFR_MISS")
+    return a, b
+
+
+CASES = [
+    ("c1_f32", lambda: TF.color_flame(1, size=700), dict(precision="fp32")),
+    ("c2_f64", lambda: TF.color_flame(2, size=700), dict(precision="fp64")),
+    ("c3_f32", lambda: TF.color_flame(3, size=4000), dict(precision="fp32")),
+    ("c3_f64", lambda: TF.color_flame(3, size=700), dict(precision="fp64")),
+    ("c4_f32", lambda: TF.color_flame(4, size=700), dict(precision="fp32")),
+    ("c4_f64", lambda: TF.color_flame(4, size=700), dict(precision="fp64")),
+    ("n_f64", lambda: spread_2d(3000), dict(precision="fp64")),
+    ("n_u32", lambda: spread_2d(5000), dict(precision="fp32", word=32)),
+    ("n3d_u32", TF.tetrahedron, dict(precision="fp32", word=32)),
+]
+
+
+@pytest.mark.parametrize("pool", [0, 1 << 21, 80 << 20, None])
+@pytest.mark.parametrize("name", [c[0] for c in CASES])
+def test_render(ffr_mod, monkeypatch, name, pool):
+    _, text, kw = next(c for c in CASES if c[0] == name)
+    print(f"miss records {name} pool={pool}", flush=True)
+    a, b = pair(ffr_mod, monkeypatch, text(), batch_size=900, binned=0, **kw)
+    if pool is not None:
+        monkeypatch.setenv("FFR_MISS_BYTES", str(pool))
+    for _ in range(2):
+        assert a.render(SAMPLES) and b.render(SAMPLES)
+    compare(a, b)
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("pool", [0, 40 << 20, None])
+def test_batch(ffr_mod, monkeypatch, pool):
+    print(f"miss records batch pool={pool}", flush=True)
+    flames = [
+        (TF.color_flame(3, size=200, seed=3), dict(precision="fp32")),
+        (TF.color_flame(3, size=900, seed=5), dict(precision="fp32")),
+        (TF.color_flame(2, size=333, seed=7), dict(precision="fp32")),
+        (TF.color_flame(3, size=600, seed=9), dict(precision="fp64")),
+        (spread_2d(1500), dict(precision="fp64")),
+        (spread_2d(700), dict(precision="fp64")),
+    ]
+    samples = [9_000_001, 12_000_000, 60_000, 18_000_000, 9_000_000, 17_000_011]
+    pairs = [pair(ffr_mod, monkeypatch, t, batch_size=1000, **kw) for t, kw in flames]
+    if pool is not None:
+        monkeypatch.setenv("FFR_MISS_BYTES", str(pool))
+    with ffr_mod.Batch([p[0] for p in pairs]) as batch:
+        for rep in range(3):
+            assert all(batch.render(samples))
+            for (a, b), n in zip(pairs, samples):
+                assert b.render(n)
+                compare(a, b)
+    for a, b in pairs:
+        a.close()
+        b.close()
+
+
+def test_bad_values(ffr_mod, monkeypatch):
+    """A flame that throws points beyond the bad-value threshold."""
+    print("miss records bad values", flush=True)
+    a, b = pair(ffr_mod, monkeypatch, TF.occasional_bad(size=3000), precision="fp64",
+                batch_size=900, binned=0, bad_value_limit=10 ** 9)
+    monkeypatch.setenv("FFR_MISS_BYTES", "1000000")
+    assert a.render(SAMPLES) and b.render(SAMPLES)
+    compare(a, b)
+    assert len(a.bad_values()) == len(b.bad_values()) > 0
+    a.close()
+    b.close()
