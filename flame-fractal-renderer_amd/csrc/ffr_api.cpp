@@ -10,11 +10,13 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <condition_variable>
 #include <cstdio>
 #include <deque>
+#include <map>
 #include <mutex>
 #include <thread>
 #include <unordered_map>
@@ -22,6 +24,7 @@
 #include <cstring>
 #include <limits>
 #include <memory>
+#include <system_error>
 #include <type_traits>
 #include <string>
 #include <vector>
@@ -284,7 +287,119 @@ static int prepare_miss_once()
     return rc;
 }
 
+// Pinned chunks through which large host copies go.  The runtime's own copy
+// of pageable memory stages through one thread, whose memcpy (and the page
+// faults of a new destination) bound it: adding a buffer of 66 MB to another
+// and reading it took 7.5 to 9.1 ms.  Here several threads copy chunks while
+// the link moves others: 1.9 ms for 66 MB either way (8 threads of 2 MB
+// chunks; 2.3 with 6 or 12 of 1 MB, 3.2 of 0.5 MB).  One per device, shared by its
+// renderers and given back with the last of them; a copy that finds it in
+// use takes the runtime's.
+struct HostStage {
+    static constexpr int kThreads = 8, kSlots = 2;
+    static constexpr size_t kChunk = (size_t)2 << 20;
+    static constexpr size_t kMinBytes = (size_t)8 << 20; // (smaller: the threads' start)
+    std::mutex busy;
+    bool ready = false;
+    char *pin = nullptr;
+    hipEvent_t ev[kThreads * kSlots] = {};
+
+    static std::shared_ptr<HostStage> of_device(int device)
+    {
+        static std::mutex lock;
+        static std::map<int, std::weak_ptr<HostStage>> stages;
+        std::lock_guard<std::mutex> g(lock);
+        std::shared_ptr<HostStage> p = stages[device].lock();
+        if (!p) {
+            p = std::make_shared<HostStage>();
+            stages[device] = p;
+        }
+        return p;
+    }
+    hipError_t init()
+    {
+        if (ready)
+            return hipSuccess;
+        hipError_t e = pin ? hipSuccess
+                           : hipHostMalloc((void **)&pin, kThreads * kSlots * kChunk,
+                                           hipHostMallocDefault);
+        for (hipEvent_t &v : ev)
+            if (e == hipSuccess && !v)
+                e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
+        ready = e == hipSuccess;
+        return e;
+    }
+    ~HostStage()
+    {
+        for (hipEvent_t v : ev)
+            if (v)
+                (void)hipEventDestroy(v);
+        if (pin)
+            (void)hipHostFree(pin);
+    }
+    // host <-> device in stream order; complete on return
+    hipError_t copy(int device, hipStream_t s, void *host, void *dev, size_t bytes, bool to_host)
+    {
+        const size_t n = (bytes + kChunk - 1) / kChunk;
+        std::atomic<size_t> next{0};
+        std::atomic<int> error{0};
+        auto work = [&](int t) {
+            hipError_t e = hipSetDevice(device);
+            size_t at[kSlots];
+            bool used[kSlots] = {};
+            auto finish = [&](int k) { // slot k's copy has ended; its chunk to the host
+                if (!used[k])
+                    return;
+                used[k] = false;
+                const hipError_t w = hipEventSynchronize(ev[t * kSlots + k]);
+                if (e == hipSuccess)
+                    e = w;
+                if (to_host && e == hipSuccess)
+                    std::memcpy((char *)host + at[k], pin + (size_t)(t * kSlots + k) * kChunk,
+                                std::min(kChunk, bytes - at[k]));
+            };
+            int k = 0;
+            for (; e == hipSuccess && !error.load(); k = (k + 1) % kSlots) {
+                finish(k);
+                const size_t i = next.fetch_add(1);
+                if (i >= n || e != hipSuccess)
+                    break;
+                at[k] = i * kChunk;
+                const size_t len = std::min(kChunk, bytes - at[k]);
+                char *slot = pin + (size_t)(t * kSlots + k) * kChunk;
+                if (to_host) {
+                    e = hipMemcpyAsync(slot, (char *)dev + at[k], len, hipMemcpyDeviceToHost, s);
+                } else {
+                    std::memcpy(slot, (char *)host + at[k], len);
+                    e = hipMemcpyAsync((char *)dev + at[k], slot, len, hipMemcpyHostToDevice, s);
+                }
+                if (e == hipSuccess)
+                    e = hipEventRecord(ev[t * kSlots + k], s);
+                used[k] = e == hipSuccess;
+            }
+            for (int j = 0; j < kSlots; ++j)
+                finish((k + j) % kSlots);
+            if (e != hipSuccess)
+                error = (int)e;
+        };
+        std::thread threads[kThreads - 1];
+        try {
+            for (int t = 1; t < kThreads; ++t)
+                threads[t - 1] = std::thread(work, t);
+        } catch (const std::system_error &) {
+            // (as many as there are; this thread works too)
+        }
+        work(0);
+        for (std::thread &t : threads)
+            if (t.joinable())
+                t.join();
+        const hipError_t e = hipStreamSynchronize(s);
+        return error.load() ? (hipError_t)error.load() : e;
+    }
+};
+
 struct ffr_renderer {
+    std::shared_ptr<HostStage> stage;
     ffr_options opt{};
     FlameSpec spec;
     int mode = MODE_F64_U64;
@@ -378,9 +493,9 @@ struct ffr_renderer {
     BinScratch bin;
     size_t bin_pay_bytes = 0;    // bytes of bin.pay
     size_t bin_sorted_bytes = 0; // bytes of bin.pay_sorted
-    // a colour flame whose renders made at least kBinColourAtomics global
-    // atomic adds per sample: its later single renders take binned
-    // accumulation (binned -1)
+    // a colour flame whose renders missed the cell cache often enough
+    // (kBinColourRecords, kBinColourAtomics): its later single renders take
+    // binned accumulation (binned -1)
     bool bin_colour = false;
     size_t bin_hist_words = 0;
     size_t bin_tiles = 0;
@@ -634,6 +749,7 @@ int ffr_create(const char *flame_json, size_t len, const ffr_options *opt_in,
     std::unique_ptr<ffr_renderer> r(new ffr_renderer());
     r->opt = opt;
     r->device = opt.device;
+    r->stage = HostStage::of_device(opt.device);
     r->mode = opt.precision == FFR_FP64 ? MODE_F64_U64
                                         : (opt.word == FFR_WORD32 ? MODE_F32_U32 : MODE_F32_U64);
     const bool fp32 = opt.precision == FFR_FP32;
@@ -1808,8 +1924,7 @@ static int finish(ffr_renderer *r, ffr_stats *out)
         r->last_atomics = st.atomics;
         r->last_flush_atomics = st.flush_atomics;
         // a colour flame whose samples missed the LDS cache often enough
-        // renders faster binned from now on (its global atomics cost more
-        // than the records' trips through HBM)
+        // renders faster binned from now on
         if (r->spec.color_dims > 0 && !r->last_bin && !r->last_chain &&
             st.s_iter >= kBinColourMinSamples &&
             (double)(st.atomics - st.flush_atomics) >= kBinColourAtomics * (double)st.s_iter)
@@ -1904,6 +2019,28 @@ size_t ffr_buffer_bytes(const ffr_renderer *r)
 int32_t ffr_dims(const ffr_renderer *r) { return r ? r->spec.dims : 0; }
 int32_t ffr_color_dims(const ffr_renderer *r) { return r ? r->spec.color_dims : 0; }
 
+// a copy of a renderer's memory to or from the host, after its stream's work
+static hipError_t host_copy(ffr_renderer *r, void *host, void *dev, size_t bytes, bool to_host)
+{
+    // (a captured stream refuses the wait below, and takes no copies)
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (bytes >= HostStage::kMinBytes && hipStreamIsCapturing(r->stream, &cap) == hipSuccess &&
+        cap == hipStreamCaptureStatusNone) {
+        HostStage &st = *r->stage;
+        std::unique_lock<std::mutex> g(st.busy, std::try_to_lock);
+        if (g.owns_lock()) {
+            if (st.init() == hipSuccess)
+                return st.copy(r->device, r->stream, host, dev, bytes, to_host);
+            (void)hipGetLastError();
+        }
+    }
+    const hipError_t e = hipStreamSynchronize(r->stream);
+    if (e != hipSuccess)
+        return e;
+    return to_host ? hipMemcpy(host, dev, bytes, hipMemcpyDeviceToHost)
+                   : hipMemcpy(dev, host, bytes, hipMemcpyHostToDevice);
+}
+
 int ffr_read_buffer(ffr_renderer *r, void *dst, size_t bytes)
 {
     if (!r || !dst)
@@ -1911,8 +2048,7 @@ int ffr_read_buffer(ffr_renderer *r, void *dst, size_t bytes)
     if (bytes != ffr_buffer_bytes(r))
         return fail(FFR_E_SIZE, "ffr_read_buffer: size mismatch");
     HIP_TRY(hipSetDevice(r->device));
-    HIP_TRY(hipStreamSynchronize(r->stream));
-    HIP_TRY(hipMemcpy(dst, r->dbuf, bytes, hipMemcpyDeviceToHost));
+    HIP_TRY(host_copy(r, dst, r->dbuf, bytes, true));
     return FFR_OK;
 }
 
@@ -1923,8 +2059,7 @@ int ffr_write_buffer(ffr_renderer *r, const void *src, size_t bytes)
     if (bytes != ffr_buffer_bytes(r))
         return fail(FFR_E_SIZE, "ffr_write_buffer: size mismatch");
     HIP_TRY(hipSetDevice(r->device));
-    HIP_TRY(hipStreamSynchronize(r->stream));
-    HIP_TRY(hipMemcpy(r->dbuf, src, bytes, hipMemcpyHostToDevice));
+    HIP_TRY(host_copy(r, const_cast<void *>(src), r->dbuf, bytes, false));
     return FFR_OK;
 }
 
@@ -1944,8 +2079,7 @@ int ffr_add_buffer(ffr_renderer *r, const void *src, size_t bytes)
     int rc = FFR_OK;
     for (size_t off = 0; off < bytes && rc == FFR_OK; off += chunk) {
         size_t n = std::min(chunk, bytes - off);
-        hipError_t e = hipMemcpyAsync(tmp, (const char *)src + off, n, hipMemcpyHostToDevice,
-                                      r->stream);
+        hipError_t e = host_copy(r, (char *)const_cast<void *>(src) + off, tmp, n, false);
         if (e == hipSuccess)
             e = (hipError_t)launch_add_cells((char *)r->dbuf + off, tmp,
                                              n / r->word_bytes, (int)r->cell_words,
