@@ -49,13 +49,16 @@ int fail(int code, const std::string &msg)
     } while (0)
 
 // Colour flames switch to binned accumulation after a render of at least
-// kBinColourMinSamples samples made kBinColourAtomics or more global atomic
-// adds (LDS-cache misses, a count and each colour word) per sample.  Measured
-// on 64 batch flames of 2048^2 cells with three colours, 1000 samples per
-// cell, FP32: binned renders faster from 0.55-0.6 atomics per sample on
-// (1.03-1.42x at 0.6-0.9, 2-4x from 1.1 on), slower below 0.5 (0.3x for
-// flames that stay in the cache).
+// kBinColourMinSamples samples whose updates past the LDS cache (a count and
+// each colour word) reached so many words per sample.  Where those are miss
+// records: 2^30 samples of 68 batch flames of 2048^2 cells with three
+// colours, and five of them up to 5700^2, take 0.55-0.65 of the binned time
+// at 0.5-0.7 words, 0.71-0.80 (FP32) and 0.81-0.94 (FP64) at 1.1-1.5,
+// 0.86-0.92 and 0.97-1.07 at 2.0, 0.96-1.01 and 1.13-1.16 at 2.7-3.0.  Where
+// they are atomics (4-byte words): binned renders faster from 0.55-0.6 words
+// on (1.03-1.42x at 0.6-0.9, 2-4x from 1.1 on), slower below 0.5.
 constexpr uint64_t kBinColourMinSamples = 1ull << 26;
+constexpr double kBinColourRecords = 1.9;
 constexpr double kBinColourAtomics = 0.6;
 
 // the kernels take the xform record offsets as constants (XformLay<D>);
@@ -1925,9 +1928,10 @@ static int finish(ffr_renderer *r, ffr_stats *out)
         r->last_flush_atomics = st.flush_atomics;
         // a colour flame whose samples missed the LDS cache often enough
         // renders faster binned from now on
+        const double bin_from = miss_ok(r) ? kBinColourRecords : kBinColourAtomics;
         if (r->spec.color_dims > 0 && !r->last_bin && !r->last_chain &&
             st.s_iter >= kBinColourMinSamples &&
-            (double)(st.atomics - st.flush_atomics) >= kBinColourAtomics * (double)st.s_iter)
+            (double)(st.atomics - st.flush_atomics) >= bin_from * (double)st.s_iter)
             r->bin_colour = true;
         size_t nrec = (size_t)std::min<uint64_t>(st.n_bad, r->opt.bad_value_cap);
         r->bv_ids.assign(nrec, 0);

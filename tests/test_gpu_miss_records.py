@@ -113,3 +113,20 @@ def test_bad_values(ffr_mod, monkeypatch):
     assert len(a.bad_values()) == len(b.bad_values()) > 0
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("records", [True, False])
+def test_binned_later(ffr_mod, monkeypatch, records):
+    """flame_1017 (2048^2) misses 0.67 words a sample: between the 0.6 from
+    which a flame whose misses are atomics renders binned and the 1.9 of one
+    whose misses are records."""
+    print(f"binned later records={records}", flush=True)
+    text = read_flame("batch/flame_1017.json")
+    if not records:
+        monkeypatch.setenv("FFR_MISS", "0")
+    a = ffr_mod.BufferRenderer(text, seed=SEED, precision="fp32")
+    for _ in range(3):
+        assert a.render(1 << 27)
+    words = (a.last_stats.atomics - a.last_stats.flush_atomics) / (1 << 27)
+    assert a.last_stats.binned == (0 if records else 1), words
+    a.close()
