@@ -2501,7 +2501,7 @@ int render_image(ffr_renderer *r, int mode, double gamma, int bits, void *dst, s
     if (!dst)
         return FFR_OK;
     if (to_host)
-        HIP_TRY(hipMemcpy(dst, r->dimg, need, hipMemcpyDeviceToHost));
+        HIP_TRY(host_copy(r, dst, r->dimg, need, true));
     if (info) {
         float ms = 0.f;
         HIP_TRY(hipEventElapsedTime(&ms, r->ev0, r->ev1));
