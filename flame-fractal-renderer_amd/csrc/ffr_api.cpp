@@ -201,17 +201,22 @@ struct MissRounds {
 // took 216 ms with 1 GB, 195 with 2, 189 with 4 and 185 with 8; the 4K
 // colour flame (2.4 GB) 57.7, 56.7 and 55.9 ms with 1, 2 and 4
 constexpr size_t kMissBytes = (size_t)4 << 30;
-// renders of fewer samples keep their atomics, and flames that miss little:
-// at 0.14 missed words a sample (4K colour flame) records took an FP32 render
-// from 82 to 56 ms, but an FP64 one, whose longer iterations hide the
-// atomics, from 28.3 to 30.7 ms
+// renders of fewer samples keep their atomics, and flames that miss little.
+// 2^30 samples of 2048^2 flames, atomics against records (ms), by missed words
+// a sample: FP32 14.3 / 15.7 at 0.05, 15.0 / 16.6 at 0.11, 20.5 / 17.2 at
+// 0.14, 34.7 / 17.2 at 0.38; FP64, whose longer iterations hide the atomics,
+// 30.1 / 32 at 0.25, 39.7 / 32.2 at 0.36.  The 4K colour flame misses 0.12
+// to 0.14 (FP32 82 / 56 ms).  A batch's flames hide each other's: 64 of them
+// in FP64, 0.61 words in the mean, 766 / 807 ms.
 constexpr uint64_t kMissMinSamples = 1ull << 24;
-constexpr double kMissWords32 = 0.05, kMissWords64 = 0.3;
+constexpr double kMissWords32 = 0.1, kMissWords64 = 0.3, kMissWordsBatch64 = 0.75;
 
 // rate: of the last render's samples those that missed (negative: unknown)
-static bool miss_worth(double rate, int cell_words, int real_bytes)
+static bool miss_worth(double rate, int cell_words, int real_bytes, bool batch)
 {
-    return rate < 0 || rate * cell_words >= (real_bytes == 8 ? kMissWords64 : kMissWords32);
+    const double least =
+        real_bytes == 4 ? kMissWords32 : batch ? kMissWordsBatch64 : kMissWords64;
+    return rate < 0 || rate * cell_words >= least;
 }
 
 static MissRounds miss_rounds(const MissMemory &mem, uint64_t samples, uint64_t tasks, int groups,
@@ -1499,7 +1504,7 @@ static int launch_single(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchP
     MissRounds m;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (p.cache && !p.direct && r->cache_pref < 0 && miss_ok(r) &&
-        miss_worth(r->miss_rate, r->cell_words, (int)sizeof(R)) &&
+        miss_worth(r->miss_rate, (int)r->cell_words, (int)sizeof(R), false) &&
         walkers * batch >= kMissMinSamples &&
         hipStreamIsCapturing(r->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
         if (const int rc = prepare_miss_once())
