@@ -60,11 +60,32 @@ struct MissArgs {
     unsigned chunks; // 0 in the last launch
     unsigned limit;
 };
-// LDS of a workgroup (256 bytes are kept for it and the task queue): per
-// wave [chunk u32 | records in it u32]; the arguments, which are read where
-// they are used; a wave of the workgroup took a chunk past the limit
+// A wave's [chunk u32 | records in it u32], handed from the lane that moves
+// on to the others through LDS: atomic accesses only, so that no lane's copy
+// of an older value stands in for a read (a wave that went on from an older
+// place would write over records).
+struct MissSlot {
+#if defined(__HIPCC__) || defined(__HIPCC_RTC__)
+    __device__ __forceinline__ unsigned long long load() const
+    {
+        // (what the wave's other lanes stored before this point)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        return __hip_atomic_load(&at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __device__ __forceinline__ void store(unsigned long long v)
+    {
+        __hip_atomic_store(&at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+#endif
+
+private:
+    unsigned long long at;
+};
+// LDS of a workgroup (256 bytes are kept for it and the task queue): the
+// waves' chunks; the arguments, which are read where they are used; a wave
+// of the workgroup took a chunk past the limit
 struct MissLds {
-    unsigned long long wave[16];
+    MissSlot wave[16];
     MissArgs args;
     unsigned full;
 };
