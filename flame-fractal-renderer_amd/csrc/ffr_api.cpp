@@ -490,14 +490,18 @@ struct ffr_renderer {
     int bin_pref = -1;
     // split walkers: -1 chosen per render, 0 off (FFR_SPLIT)
     int split_pref = -1;
-    // miss records: -1 chosen per render, 0 off (FFR_MISS); the share of the
-    // samples expected to miss the cell cache (measured by each render)
+    // miss records: -1 chosen, 0 off, 1 wherever the flame allows them
+    // (FFR_MISS); the share of the samples expected to miss the cell cache
+    // (measured by each render)
     int miss_pref = -1;
+    int task_rounds = 1; // FFR_TASK_ROUNDS: walkers per lane in a task
     MissMemory miss_memory;
     MissTiles miss_tiles;
     double miss_rate = -1;
     bool last_cached = false; // the last render's misses count (a hashed cache)
     MissRounds miss_last; // the last render's (memory and chunks)
+    uint64_t last_records = 0; // the last render's misses that became records
+    uint32_t last_pauses = 0;  // and the pauses of its workgroups
     BinScratch bin;
     size_t bin_pay_bytes = 0;    // bytes of bin.pay
     size_t bin_sorted_bytes = 0; // bytes of bin.pay_sorted
@@ -806,8 +810,10 @@ int ffr_create(const char *flame_json, size_t len, const ffr_options *opt_in,
         if (const char *e = std::getenv("FFR_SPLIT"))
             r->split_pref = std::atoi(e) ? -1 : 0;
         if (const char *e = std::getenv("FFR_MISS"))
-            r->miss_pref = std::atoi(e) ? -1 : 0;
+            r->miss_pref = std::atoi(e) < 0 ? -1 : (std::atoi(e) ? 1 : 0);
         r->compiled_pref = opt.compiled < 0 ? -1 : (opt.compiled ? 1 : 0);
+        if (const char *e = std::getenv("FFR_TASK_ROUNDS"))
+            r->task_rounds = std::max(1, std::atoi(e));
         if (const char *e = std::getenv("FFR_CHAIN_PER_CU"))
             r->chain_per_cu = std::atoi(e);
         if (const char *e = std::getenv("FFR_COMPILED"))
@@ -1000,6 +1006,7 @@ static LaunchShape renderer_shape(const ffr_renderer *r)
     LaunchShape sh;
     sh.bin = r->bin_pref;
     sh.split = r->split_pref;
+    sh.task_rounds = r->task_rounds;
     sh.cache = r->cache_pref;
     sh.cache_kb = r->cache_kb;
     sh.block = r->block_pref;
@@ -1295,7 +1302,7 @@ constexpr uint64_t kCompiledProbeSamples = 1ull << 33;
 static bool miss_ok(const ffr_renderer *r)
 {
     const int ncol = r->spec.color_dims;
-    return r->miss_pref < 0 && ncol <= 4 && !(ncol > 0 && r->word_bytes == 4) &&
+    return r->miss_pref != 0 && ncol <= 4 && !(ncol > 0 && r->word_bytes == 4) &&
            r->cells < (ncol > 0 ? (1ull << 25) : (1ull << 28));
 }
 
@@ -1504,8 +1511,9 @@ static int launch_single(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchP
     MissRounds m;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (p.cache && !p.direct && r->cache_pref < 0 && miss_ok(r) &&
-        miss_worth(r->miss_rate, (int)r->cell_words, (int)sizeof(R), false) &&
-        walkers * batch >= kMissMinSamples &&
+        (r->miss_pref > 0 ||
+         (miss_worth(r->miss_rate, (int)r->cell_words, (int)sizeof(R), false) &&
+          walkers * batch >= kMissMinSamples)) &&
         hipStreamIsCapturing(r->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
         if (const int rc = prepare_miss_once())
             return rc;
@@ -1931,6 +1939,8 @@ static int finish(ffr_renderer *r, ffr_stats *out)
                            (double)st.s_iter;
         r->last_atomics = st.atomics;
         r->last_flush_atomics = st.flush_atomics;
+        r->last_records = st.records;
+        r->last_pauses = st.pauses;
         // a colour flame whose samples missed the LDS cache often enough
         // renders faster binned from now on
         const double bin_from = miss_ok(r) ? kBinColourRecords : kBinColourAtomics;
@@ -1989,6 +1999,17 @@ int ffr_render_async(ffr_renderer *r, uint64_t samples)
     if (samples == 0)
         return FFR_OK;
     return launch(r, samples);
+}
+
+int ffr_record_use(const ffr_renderer *r, uint64_t *records, uint32_t *pauses)
+{
+    if (!r)
+        return fail(FFR_E_ARG, "ffr_record_use: null renderer");
+    if (records)
+        *records = r->last_records;
+    if (pauses)
+        *pauses = r->last_pauses;
+    return FFR_OK;
 }
 
 int ffr_sync(ffr_renderer *r, ffr_stats *stats)

@@ -19,6 +19,8 @@ __global__ void reset_stats_kernel(DevStats *st, unsigned long long *xf_count, i
         s->flush_atomics = 0;
         s->split_fail = 0;
         s->split_again = 0;
+        s->records = 0;
+        s->pauses = 0;
         for (int i = 0; i < 3; ++i) {
             s->pmin[i] = (double)INFINITY;
             s->pmax[i] = -(double)INFINITY;
@@ -40,7 +42,9 @@ __global__ void reset_many_kernel(const ResetEntry *e, int n, unsigned *queues, 
             st->s_plot = 0;
             st->n_bad = 0;
             st->atomics = 0;
-        st->flush_atomics = 0;
+            st->flush_atomics = 0;
+            st->records = 0;
+            st->pauses = 0;
             for (int i = 0; i < 3; ++i) {
                 st->pmin[i] = (double)INFINITY;
                 st->pmax[i] = -(double)INFINITY;

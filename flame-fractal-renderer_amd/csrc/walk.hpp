@@ -22,6 +22,8 @@ struct DevStats {
     // and the segments that ran again from their neighbour's end
     unsigned split_fail;
     unsigned split_again;
+    unsigned long long records; // misses that became records
+    unsigned pauses;            // workgroups that paused for their binning
 };
 
 constexpr int kMaxSlots = 64;     // variation slots per flame

@@ -147,7 +147,7 @@ IMG_MONO, IMG_GRAY, IMG_COLOR = 0, 1, 2
 # every symbol include/ffr.h declares
 EXPORTS = [
     "ffr_default_options", "ffr_create", "ffr_destroy", "ffr_last_error",
-    "ffr_render", "ffr_render_async", "ffr_sync", "ffr_set_stream",
+    "ffr_render", "ffr_render_async", "ffr_sync", "ffr_record_use", "ffr_set_stream",
     "ffr_device_buffer", "ffr_buffer_cells", "ffr_cell_words", "ffr_word_bytes",
     "ffr_buffer_bytes", "ffr_dims", "ffr_color_dims", "ffr_read_buffer",
     "ffr_add_buffer", "ffr_add_buffer_noalloc", "ffr_write_buffer", "ffr_clear_buffer",
@@ -211,6 +211,7 @@ def lib():
     L.ffr_xform_distribution.argtypes = [P, C.POINTER(C.c_uint64), C.c_size_t]
     L.ffr_xform_id_count.restype = C.c_size_t
     L.ffr_xform_id_count.argtypes = [P]
+    L.ffr_record_use.argtypes = [P, C.POINTER(C.c_uint64), C.POINTER(C.c_uint32)]
     L.ffr_bad_values.argtypes = [P, C.POINTER(C.c_uint64), C.POINTER(C.c_double),
                                  C.c_size_t, C.POINTER(C.c_size_t)]
     L.ffr_xform_order.argtypes = [P, C.POINTER(C.c_int32), C.POINTER(C.c_double),
@@ -537,6 +538,14 @@ class BufferRenderer:
     @property
     def kernel_ms(self) -> float:
         return self.last_stats.kernel_ms
+
+    @property
+    def record_use(self) -> tuple[int, int]:
+        """Of the last render: the updates past the cell cache that became
+        records, and the pauses of workgroups that had used up their memory."""
+        n, pauses = C.c_uint64(), C.c_uint32()
+        _check(lib().ffr_record_use(self._h, C.byref(n), C.byref(pauses)))
+        return n.value, pauses.value
 
     def xform_distribution(self) -> np.ndarray:
         n = lib().ffr_xform_id_count(self._h)

@@ -159,6 +159,13 @@ int ffr_render(ffr_renderer *r, uint64_t samples, ffr_stats *stats);
 int ffr_render_async(ffr_renderer *r, uint64_t samples);
 int ffr_sync(ffr_renderer *r, ffr_stats *stats);
 
+/* Of the last finished render (batched passes and server passes too): the
+ * updates past the LDS cell cache that became records to be binned instead
+ * of atomic adds (ffr_stats.atomics counts the words of both), and how
+ * often a workgroup paused because the record memory was used up.  No
+ * counterpart in the reference.  Either pointer may be NULL. */
+int ffr_record_use(const ffr_renderer *r, uint64_t *records, uint32_t *pauses);
+
 /* launch on a caller-owned hipStream_t (NULL: the renderer's own stream) */
 int ffr_set_stream(ffr_renderer *r, void *hip_stream);
 /* device address of the buffer (cells * cell_words words) */
