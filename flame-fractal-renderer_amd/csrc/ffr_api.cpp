@@ -553,6 +553,12 @@ static int pick_variation_set(const uint32_t ts[4])
     return linear_only ? 0 : (basic ? 1 : 2);
 }
 
+// the settle iterations of a renderer's walkers
+template <typename R> static int settle_iterations(const ffr_renderer *r)
+{
+    return r->opt.settle_iters >= 0 ? (int)r->opt.settle_iters : (sizeof(R) == 4 ? 24 : 53);
+}
+
 // Split walkers: how many iterations two trajectories of the flame that draw
 // the same words take to become equal bit for bit.  A map that shrinks
 // distances by 2^-c on average takes (mantissa bits + a few) / c; the margin
@@ -648,14 +654,10 @@ static int setup_tables(ffr_renderer *r, const DeviceFlame<R> &d)
                                            " bytes exceeds the " + std::to_string(max_lds) +
                                            "-byte LDS of a workgroup");
     r->vs = pick_variation_set(d.type_set);
-    // the basic set's kernels add a zero times the mapped point where a list
-    // is short: the point is finite as long as the pre-affines cannot
-    // overflow from a point within the bad-value limit
-    if (r->vs == 1)
-        for (const XformSpec &x : r->spec.xforms)
-            for (int i = 0; i < 9; ++i)
-                if (std::fabs(x.preA[i]) > 1e15 || std::fabs(x.preb[i % 3]) > 1e15)
-                    r->vs = 2;
+    // the basic set's 2-D kernels add a zero times the mapped point where a
+    // list is short, which is nothing while the point is finite
+    if (r->vs == 1 && d.dims == 2 && !settles_in_range(d, settle_iterations<R>(r)))
+        r->vs = 3;
     r->chain_ok = r->vs == 0 /* linear only, final xform included */ && d.r <= 4 &&
                   d.slot_type.size() <= (size_t)kChainSlots;
     // every xform's post-affine is exactly the identity (entries 1.0 and
@@ -961,7 +963,7 @@ static void fill_args(ffr_renderer *r, const DeviceFlame<R> &d, WalkArgs<R> &a)
     a.n_slots = (int)d.slot_type.size();
     a.has_final = d.has_final;
     a.fin_nv = (int)d.fin_type.size();
-    a.settle = r->opt.settle_iters >= 0 ? (int)r->opt.settle_iters : (sizeof(R) == 4 ? 24 : 53);
+    a.settle = settle_iterations<R>(r);
     a.r = d.r;
     a.tab_reals = (int)d.table.size();
     a.xf0 = d.xf0;

@@ -1009,8 +1009,8 @@ template <typename R> DeviceFlame<R> compile_flame(const FlameSpec &spec)
                 basic = basic && code_of(v->type) >= 0;
         }
         if (basic) {
-            // at least three terms (linear of weight 0, which adds a zero,
-            // pads the shorter lists), whole 16 bytes
+            // at least three terms (terms of weight 0, which add a zero,
+            // pad the shorter lists), whole 16 bytes
             d.bt_nvmax = nvmax;
             d.bt_stride = (int)align4(2 * (size_t)std::max(nvmax, 3));
             T.resize(align4(T.size()), (R)0);
@@ -1025,6 +1025,8 @@ template <typename R> DeviceFlame<R> compile_flame(const FlameSpec &spec)
                     B[2 * j] = basic_code_real<R>(c);
                     B[2 * j + 1] = (R)L[j]->weight;
                 }
+                for (size_t j = L.size(); 2 * j < (size_t)d.bt_stride; ++j)
+                    B[2 * j] = basic_pad_real<R>();
             }
         }
     }
@@ -1050,6 +1052,63 @@ template <typename R> DeviceFlame<R> compile_flame(const FlameSpec &spec)
     }
     return d;
 }
+
+// the largest factor by which a 2x2 matrix (row-major) lengthens a vector
+static double norm2x2(double a, double b, double c, double d)
+{
+    const double s = a * a + b * b + c * c + d * d, det = a * d - b * c;
+    return std::sqrt(0.5 * (s + std::sqrt(std::max(0.0, s * s - 4.0 * det * det))));
+}
+
+template <typename R> bool settles_in_range(const DeviceFlame<R> &d, int settle)
+{
+    const bool f32 = sizeof(R) == 4;
+    const double eps = f32 ? 1e-10 : 1e-20, limit = f32 ? 1e10 : 1e20; // (constants.hpp:17-56)
+    const double most = f32 ? 8e37 : 4e307;   // of the mapped points
+    const double square = f32 ? 1e18 : 1e150; // ... whose square stays finite
+    // the longest image of a point of length n (it grows with n); negative:
+    // a mapped point reaches `top`
+    auto image = [&](double n, double top) {
+        double longest = 0.0;
+        for (int k = 0; k < d.nxf; ++k) {
+            const R *X = d.table.data() + d.xf0 + (size_t)k * (size_t)d.lay.stride;
+            auto affine = [&](int A, int b, double t) {
+                return (norm2x2(X[A], X[A + 1], X[A + 2], X[A + 3]) * t +
+                        std::hypot((double)X[b], (double)X[b + 1])) * (1.0 + 1e-5);
+            };
+            const double t = affine(d.lay.preA, d.lay.preb, n);
+            if (!(t < top))
+                return -1.0;
+            double v = 0.0;
+            const R *B = d.table.data() + d.bt0 + (size_t)(k * d.bt_stride);
+            for (int j = 0; 2 * j < d.bt_stride; ++j) {
+                // (linear, swirl and horseshoe lengthen no vector)
+                const R c = B[2 * j];
+                const double o = c == basic_code_real<R>(1)   ? 1.5 // sinusoidal
+                                 : c == basic_code_real<R>(2) ? 0.5 / std::sqrt(eps) // spherical
+                                 : c == basic_code_real<R>(5) ? t + 2.0 // polar
+                                                              : t;
+                v += std::fabs((double)B[2 * j + 1]) * o;
+            }
+            longest = std::max(longest, affine(d.lay.postA, d.lay.postb, v));
+        }
+        return longest;
+    };
+    if (d.bt0 < 0 || image(2.0 * limit, most) < 0.0)
+        return false;
+    double n = 1.5; // (walkers start in [-1, 1]^2)
+    for (int i = 0; i <= settle && i < 10000; ++i) {
+        const double next = image(n, square);
+        if (next < 0.0)
+            return false;
+        if (next <= n)
+            return true; // (no later point is longer)
+        n = next;
+    }
+    return settle < 10000;
+}
+template bool settles_in_range<double>(const DeviceFlame<double> &, int);
+template bool settles_in_range<float>(const DeviceFlame<float> &, int);
 
 template DeviceFlame<double> compile_flame<double>(const FlameSpec &);
 template DeviceFlame<float> compile_flame<float>(const FlameSpec &);

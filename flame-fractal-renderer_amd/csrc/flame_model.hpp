@@ -96,6 +96,9 @@ template <typename R> constexpr R basic_code_real(int code)
            : code == 5 ? (R)-2
                        : (R)0;
 }
+// ... and that of the terms that pad a list: no code, so that it counts as
+// linear, which the weight 0 takes away
+template <typename R> constexpr R basic_pad_real() { return (R)8; }
 
 template <typename R> struct DeviceFlame {
     int dims = 2, r = 0;
@@ -120,7 +123,7 @@ template <typename R> struct DeviceFlame {
     // per-xform variation lists for 2-D flames whose variations are all of
     // the basic six (linear, sinusoidal, spherical, swirl, horseshoe,
     // polar; codes 0..5): (code as a real, weight) pairs per xform in JSON
-    // order, at least three (padded with linear of weight 0), at table
+    // order, at least three (padded with terms of weight 0), at table
     // offset bt0 (-1: not built); bt_union: bit k set when some list holds
     // code k
     int bt0 = -1, bt_stride = 0, bt_nvmax = 0, bt_union = 0;
@@ -130,6 +133,11 @@ template <typename R> struct DeviceFlame {
 
 template <typename R>
 DeviceFlame<R> compile_flame(const FlameSpec &spec); // throws JsonError
+// A 2-D flame of the basic variations (bt0): whether every point that a
+// walker meets in its `settle` iterations and the first after them, none of
+// which is checked for bad values before the next, stays far inside the
+// number range when mapped, and every point within the bad-value limit too.
+template <typename R> bool settles_in_range(const DeviceFlame<R> &d, int settle);
 
 // the reference's BufferRenderer limits
 constexpr uint64_t kMaxCells = 1ull << 48;

@@ -22,12 +22,15 @@
 
 namespace ffr {
 
-enum { VS_LINEAR = 0, VS_BASIC = 1, VS_ALL = 2 };
+// (VS_EXACT: the basic six of 2-D flames whose walkers may leave the number
+// range before their bad values are seen, xform_apply)
+enum { VS_LINEAR = 0, VS_BASIC = 1, VS_ALL = 2, VS_EXACT = 3 };
 
 __host__ __device__ constexpr bool vs_has(int vs, int type)
 {
     return vs == VS_ALL || type == 0 ||
-           (vs == VS_BASIC && (type == 1 || type == 2 || type == 20 || type == 21 || type == 22));
+           ((vs == VS_BASIC || vs == VS_EXACT) &&
+            (type == 1 || type == 2 || type == 20 || type == 21 || type == 22));
 }
 
 template <typename R> __device__ __forceinline__ R dev_randnum(Stream &s)
