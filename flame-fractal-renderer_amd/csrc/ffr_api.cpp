@@ -1827,7 +1827,6 @@ static int launch(ffr_renderer *r, uint64_t samples)
     LaunchPlan p = plan_launch(r, walkers, batch, renderer_shape(r));
     LaunchPlan fb;
     r->last_split = false;
-    r->last_cached = p.cache && !p.direct && !p.bin && !p.split_log2;
     if (p.split_log2) {
         // (its scratch may be allocated here, so not while the stream is
         // captured; without the memory for it the walkers run unsplit)
@@ -1854,6 +1853,7 @@ static int launch(ffr_renderer *r, uint64_t samples)
                  : choose_cache(r, r->f32, p, r->next_walker, walkers, batch, samples);
     if (rc != FFR_OK)
         return rc;
+    r->last_cached = p.cache && !p.direct && !p.bin && !p.split_log2;
     r->last_walkers = walkers;
     r->last_batch = batch;
     r->last_cache = p.cache ? p.slots : 0;
