@@ -201,22 +201,39 @@ struct MissRounds {
 // took 216 ms with 1 GB, 195 with 2, 189 with 4 and 185 with 8; the 4K
 // colour flame (2.4 GB) 57.7, 56.7 and 55.9 ms with 1, 2 and 4
 constexpr size_t kMissBytes = (size_t)4 << 30;
-// renders of fewer samples keep their atomics, and flames that miss little.
-// 2^30 samples of 2048^2 flames, atomics against records (ms), by missed words
-// a sample: FP32 14.3 / 15.7 at 0.05, 15.0 / 16.6 at 0.11, 20.5 / 17.2 at
-// 0.14, 34.7 / 17.2 at 0.38; FP64, whose longer iterations hide the atomics,
-// 30.1 / 32 at 0.25, 39.7 / 32.2 at 0.36.  The 4K colour flame misses 0.12
-// to 0.14 (FP32 82 / 56 ms).  A batch's flames hide each other's: 64 of them
-// in FP64, 0.61 words in the mean, 766 / 807 ms.
+// Renders keep their atomics where the walkers hide them.  While the launch
+// fills the device's lanes, by missed words a sample (as atomics miss), 2^28
+// to 2^32 samples of 40 flames, atomics over records in time:
+//   FP32  0.85-0.96 below 0.09; 0.91-1.06 and once 1.6 at 0.09-0.125; 0.9-1.3
+//         at 0.13-0.135 (the 4K colour flame 1.04-1.28, compiled 1.43);
+//         1.05-1.8 at 0.16-0.25, 1.2-2.4 at 0.25-0.45
+//   FP64  (longer iterations hide more) 0.87-0.95 below 0.28, 0.97-1.02 at
+//         0.3, 1.15-1.25 at 0.34 (once 0.85), 1.1-1.4 at 0.43-0.48
+// A launch of fewer walkers than lanes takes as long as a full one and misses
+// less in it, so the line rises as the walkers fall: 2^27 samples in FP32
+// (half the lanes) cross at 0.3, 2^26 between 0.86 (0.96) and 2.4 (2.4), 2^24
+// (a sixteenth) below 2.4 (1.28); FP64 2^26 (half) between 0.84 (0.87) and
+// 2.4 (2.1).  A batch's flames hide each other's: 64 of them in FP64, 0.61
+// words in the mean, 766 / 807 ms.  A first render, which knows no rate, is
+// taken to miss 0.3 words (wrong, it costs 5 to 15 %; atomics of a flame that
+// spreads, two to five times the render).
 constexpr uint64_t kMissMinSamples = 1ull << 24;
-constexpr double kMissWords32 = 0.1, kMissWords64 = 0.3, kMissWordsBatch64 = 0.75;
+constexpr double kMissWords32 = 0.13, kMissWords64 = 0.3, kMissWordsBatch64 = 0.75;
+constexpr double kMissWordsUnknown = 0.3;
+// a single render with records seeds its caches alike (hints) and misses
+// 0.74 to 0.86 of what it misses without
+constexpr double kMissSeeded = 0.8;
 
-// rate: of the last render's samples those that missed (negative: unknown)
-static bool miss_worth(double rate, int cell_words, int real_bytes, bool batch)
+// rate: of the last render's samples those that missed (negative: unknown),
+// with seeded caches or without
+static bool miss_worth(double rate, bool seeded, int cell_words, int real_bytes, bool batch,
+                       uint64_t walkers, uint64_t lanes)
 {
     const double least =
-        real_bytes == 4 ? kMissWords32 : batch ? kMissWordsBatch64 : kMissWords64;
-    return rate < 0 || rate * cell_words >= least;
+        real_bytes == 4 ? kMissWords32 : batch && rate >= 0 ? kMissWordsBatch64 : kMissWords64;
+    const double words =
+        rate < 0 ? kMissWordsUnknown : rate * cell_words / (seeded ? kMissSeeded : 1.0);
+    return words >= least * std::max(1.0, (double)lanes / (double)std::max<uint64_t>(walkers, 1));
 }
 
 static MissRounds miss_rounds(const MissMemory &mem, uint64_t samples, uint64_t tasks, int groups,
@@ -498,6 +515,9 @@ struct ffr_renderer {
     MissMemory miss_memory;
     MissTiles miss_tiles;
     double miss_rate = -1;
+    bool rate_seeded = false; // ... by one with seeded caches
+    bool miss_seeded = false; // the last render's caches were seeded
+    unsigned hot_tag = 0;     // of the hints that single renders left
     bool last_cached = false; // the last render's misses count (a hashed cache)
     MissRounds miss_last; // the last render's (memory and chunks)
     uint64_t last_records = 0; // the last render's misses that became records
@@ -1298,6 +1318,13 @@ static int launch_compiled_kernel(ffr_renderer *r, const LaunchPlan &p, void *fn
 // compile (about half a second) pays off only over repeated renders.
 constexpr uint64_t kCompiledProbeSamples = 1ull << 33;
 
+// the lanes of a cached plan that the device holds at a time
+static uint64_t cached_lanes(const ffr_renderer *r, const LaunchPlan &p)
+{
+    const uint64_t groups = std::max<uint64_t>(1, r->lds_per_cu / std::max<size_t>(p.lds, 1));
+    return (uint64_t)r->cu_count * groups * (uint64_t)p.block;
+}
+
 // Miss records apply to a cached launch of a flame whose cells (and colour
 // sums) the binning kernels hold: not colour flames with 4-byte words, whose
 // float sums keep the per-sample float adds
@@ -1514,7 +1541,8 @@ static int launch_single(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchP
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (p.cache && !p.direct && r->cache_pref < 0 && miss_ok(r) &&
         (r->miss_pref > 0 ||
-         (miss_worth(r->miss_rate, (int)r->cell_words, (int)sizeof(R), false) &&
+         (miss_worth(r->miss_rate, r->rate_seeded, (int)r->cell_words, (int)sizeof(R), false,
+                     walkers, cached_lanes(r, p)) &&
           walkers * batch >= kMissMinSamples)) &&
         hipStreamIsCapturing(r->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
         if (const int rc = prepare_miss_once())
@@ -1551,6 +1579,11 @@ static int launch_single(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchP
             a[0].hot_tag = 0x40000000u | ((unsigned)p.log2s << 8) | (unsigned)p.ways;
         }
     }
+    // (hints of an earlier render, or of this one's own earlier tasks)
+    r->miss_seeded = m.rounds && (r->hot_tag == a[0].hot_tag ||
+                                  walkers >= 2 * (uint64_t)p.grid * p.task_walkers);
+    if (m.rounds)
+        r->hot_tag = a[0].hot_tag;
     a[1] = a[0];
     a[1].miss.chunks = 0;
     r->hargs.resize(sizeof a);
@@ -1936,9 +1969,11 @@ static int finish(ffr_renderer *r, ffr_stats *out)
             r->last_split = false;
         }
         r->last_bad = st.n_bad;
-        if (r->last_cached && st.s_iter)
+        if (r->last_cached && st.s_iter) {
+            r->rate_seeded = r->miss_seeded;
             r->miss_rate = (double)(st.atomics - st.flush_atomics) / (double)r->cell_words /
                            (double)st.s_iter;
+        }
         r->last_atomics = st.atomics;
         r->last_flush_atomics = st.flush_atomics;
         r->last_records = st.records;

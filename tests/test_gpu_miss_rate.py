@@ -1,7 +1,8 @@
 """What a render learns about its misses comes from renders through the LDS
-cell cache alone: an uncached batch, whose every sample goes past the cache, does not make the next cached one take records.  (FP64 renders of a
-flame that misses 0.12 words a sample keep their atomics; the first render of
-a renderer, which knows nothing, takes records.)"""
+cell cache alone: an uncached batch, whose every sample goes past the cache, does
+not make the next cached one take records.  (FP64 renders of a flame that
+misses 0.12 words a sample keep their atomics; the first render of a renderer,
+which knows nothing, takes records.)"""
 
 import pytest
 

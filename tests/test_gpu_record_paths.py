@@ -157,8 +157,11 @@ def test_batch(ffr_mod, monkeypatch, small, rounds):
             assert all(batch.render(samples))
             for a, b, n in zip(rs, alone, samples):
                 assert b.render(n)
-                assert 0 < a.record_use[0] <= missed(a)
+                # (in the small memory one flame's misses may all come when
+                # it is used up)
+                assert int(not small) <= a.record_use[0] <= missed(a)
                 same_buffers(a, b)
+            assert sum(a.record_use[0] for a in rs) > 0
             assert (sum(a.record_use[1] for a in rs) > 0) == small
     for r in rs + alone:
         r.close()
