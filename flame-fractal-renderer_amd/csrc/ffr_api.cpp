@@ -519,7 +519,6 @@ struct ffr_renderer {
     bool miss_seeded = false; // the last render's caches were seeded
     unsigned hot_tag = 0;     // of the hints that single renders left
     bool last_cached = false; // the last render's misses count (a hashed cache)
-    MissRounds miss_last; // the last render's (memory and chunks)
     uint64_t last_records = 0; // the last render's misses that became records
     uint32_t last_pauses = 0;  // and the pauses of its workgroups
     BinScratch bin;
@@ -1335,25 +1334,114 @@ static bool miss_ok(const ffr_renderer *r)
            r->cells < (ncol > 0 ? (1ull << 25) : (1ull << 28));
 }
 
-// ... and a kernel probe takes them as the last render did, where that
-// render's memory holds this launch's workgroups
-static bool miss_ready(const ffr_renderer *r, const LaunchPlan &p, int real_bytes, MissScratch &x)
+// ... and are taken by a launch of enough walkers and samples that miss
+// enough (not where the cache is forced, or indexed directly, so that
+// nothing misses; their memory may be allocated, so not while the stream is
+// captured)
+static bool records_wanted(const ffr_renderer *r, const LaunchPlan &p, uint64_t walkers,
+                           uint64_t batch, int real_bytes)
 {
-    const size_t pause = real_bytes == 8 ? sizeof(WalkerPause<double>) : sizeof(WalkerPause<float>);
-    if (!r->miss_last.rounds || !p.cache || p.direct ||
-        r->miss_memory.ctrl_bytes < (size_t)(p.grid + 1) * sizeof(MissCtrl) ||
-        r->miss_memory.state_bytes < (size_t)p.grid * (size_t)p.block * pause)
-        return false;
-    x = miss_scratch(r->miss_memory, r->miss_tiles, r->miss_last.chunks, p.grid,
-                     record_words(walk_nc(r), real_bytes), real_bytes, r->cu_count);
-    return true;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return p.cache && !p.direct && r->cache_pref < 0 && miss_ok(r) &&
+           (r->miss_pref > 0 ||
+            (miss_worth(r->miss_rate, r->rate_seeded, (int)r->cell_words, real_bytes, false,
+                        walkers, cached_lanes(r, p)) &&
+             walkers * batch >= kMissMinSamples)) &&
+           hipStreamIsCapturing(r->stream, &cap) == hipSuccess &&
+           cap == hipStreamCaptureStatusNone;
+}
+
+// The memory for the records of a launch into `buf`, and its rounds: none
+// without the memory (the misses then stay atomics).
+static int reserve_records(ffr_renderer *r, const LaunchPlan &p, uint64_t walkers, uint64_t batch,
+                           int real_bytes, void *buf, MissTiles &tiles, MissRounds &m)
+{
+    m = MissRounds();
+    if (const int rc = prepare_miss_once())
+        return rc;
+    const int words = record_words(walk_nc(r), real_bytes);
+    MissRounds want =
+        miss_rounds(r->miss_memory, walkers * batch,
+                    (walkers + p.task_walkers - 1) / p.task_walkers, p.grid, p.block, words,
+                    r->miss_rate);
+    if (!want.rounds)
+        return 0;
+    hipError_t e = r->miss_memory.ensure(p.grid, p.block, want.chunks, words, real_bytes);
+    if (e == hipSuccess) {
+        MissFlame f{};
+        f.buf = buf;
+        f.cells = r->cells;
+        f.r = r->spec.color_dims;
+        e = tiles.set({f}, f.r > 0 ? kBinTileBitsColour : kBinTileBits, r->stream);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        r->miss_memory.free_all();
+        return 0;
+    }
+    m = want;
+    return 0;
+}
+
+static MissScratch records_scratch(const ffr_renderer *r, const LaunchPlan &p,
+                                   const MissTiles &tiles, const MissRounds &m, int real_bytes)
+{
+    return miss_scratch(r->miss_memory, tiles, m.chunks, p.grid,
+                        record_words(walk_nc(r), real_bytes), real_bytes, r->cu_count);
+}
+
+// the arguments of a lane-per-walker render: its walker launches', and those
+// of the last one, which has no record memory
+template <typename R>
+static void records_args(const ffr_renderer *r, const LaunchPlan &p, const MissTiles &tiles,
+                         const MissRounds &m, WalkArgs<R> (&a)[2])
+{
+    if (m.rounds) {
+        a[0].miss = miss_args(records_scratch(r, p, tiles, m, (int)sizeof(R)), m.limit);
+        // hints: with records, workgroups seeded alike have no atomics to
+        // queue on (the headline flame misses 3.0 instead of 3.5 %)
+        if (r->dhot && p.slots <= kHotSlots) {
+            a[0].hot = r->dhot;
+            a[0].hot_tag = 0x40000000u | ((unsigned)p.log2s << 8) | (unsigned)p.ways;
+        }
+    }
+    a[1] = a[0];
+    a[1].miss.chunks = 0;
+}
+
+// the launches of such a render, by the flame's compiled kernel fn or the
+// table-driven one (nullptr); the arguments are at r->dargs
+template <typename R>
+static int launch_rounds(ffr_renderer *r, const LaunchPlan &p, void *fn, int nslots,
+                         const MissTiles &tiles, const MissRounds &m)
+{
+    // (a compiled flame's kernel reads only the launch part, WalkDyn, at the
+    // start of WalkArgs; its flame fields are constants)
+    auto walk = [&](int k) {
+        const void *args = (const unsigned char *)r->dargs + (size_t)k * sizeof(WalkArgs<R>);
+        return fn ? launch_compiled_kernel(r, p, fn, args)
+                  : launch_table_kernel(r, p, nslots, args);
+    };
+    if (!m.rounds)
+        return walk(0);
+    const MissScratch x = records_scratch(r, p, tiles, m, (int)sizeof(R));
+    int rc = launch_miss_init(x, p.task_walkers, r->stream);
+    for (int k = 0; k < m.rounds && !rc; ++k) {
+        rc = walk(0);
+        if (!rc)
+            rc = launch_miss_round(x, (int)r->word_bytes, r->stream);
+    }
+    if (!rc && m.last)
+        rc = walk(1);
+    return rc;
 }
 
 // Time kernels for the coming render: n launch plans, each with the flame's
 // compiled kernel fns[k] or the table-driven one (nullptr), on the render's
 // walkers with at most 1024 samples each, into a scratch buffer: the
 // renderer's buffer and stream positions are untouched, and the statistics
-// the runs leave are reset before the render.  ms[k]: the better of two
+// the runs leave are reset before the render.  Misses become records where
+// the render's would, and their binning is timed with the walkers.  ms[k]: the better of two
 // runs (one, when after the first every other kernel took more than
 // stop_ratio times kernel 0's time; 0: always two).
 template <typename R>
@@ -1365,19 +1453,30 @@ static int time_kernels(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchPl
     void *scratch = nullptr;
     HIP_TRY(hipMalloc(&scratch, ffr_buffer_bytes(r)));
     std::vector<std::vector<unsigned char>> h((size_t)n);
-    MissScratch miss;
+    std::vector<MissRounds> rounds((size_t)n);
+    MissTiles tiles;
     for (int k = 0; k < n; ++k) {
-        WalkArgs<R> a;
-        walk_args(r, d, plans[k], walker0, walkers, pb, pb, a);
-        a.buf = scratch;
-        // (records of the last render's memory, which nothing bins; a
-        // workgroup that pauses ends its run there)
-        if (miss_ready(r, plans[k], (int)sizeof(R), miss))
-            a.miss = miss_args(miss, r->miss_last.limit);
-        a.bv_limit = ~0ull; // the runs never stop at the bad-value limit
-        h[(size_t)k].resize(sizeof a);
-        std::memcpy(h[(size_t)k].data(), &a, sizeof a);
         ms[k] = 1e30f;
+        int rc = 0;
+        if (records_wanted(r, plans[k], walkers, batch, (int)sizeof(R)))
+            rc = reserve_records(r, plans[k], walkers, pb, (int)sizeof(R), scratch, tiles,
+                                 rounds[(size_t)k]);
+        if (rc) {
+            tiles.free_all();
+            (void)hipFree(scratch);
+            return fail(FFR_E_DEVICE, std::string("kernel probe: ") +
+                                          hipGetErrorString((hipError_t)rc));
+        }
+    }
+    // (the record memory stands now)
+    for (int k = 0; k < n; ++k) {
+        WalkArgs<R> a[2];
+        walk_args(r, d, plans[k], walker0, walkers, pb, pb, a[0]);
+        a[0].buf = scratch;
+        a[0].bv_limit = ~0ull; // the runs never stop at the bad-value limit
+        records_args(r, plans[k], tiles, rounds[(size_t)k], a);
+        h[(size_t)k].resize(sizeof a);
+        std::memcpy(h[(size_t)k].data(), a, sizeof a);
     }
     hipError_t e = hipSuccess;
     for (int round = 0; round < 2 && e == hipSuccess; ++round) {
@@ -1395,15 +1494,11 @@ static int time_kernels(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchPl
                 e = launch_reset_stats(r->dstats, r->dxf, r->nxf, r->stream)
                         ? hipErrorLaunchFailure
                         : hipSuccess;
-            if (e == hipSuccess && miss_ready(r, plans[k], (int)sizeof(R), miss))
-                e = (hipError_t)launch_miss_init(miss, plans[k].task_walkers, r->stream);
             if (e == hipSuccess)
                 e = hipEventRecord(r->ev0, r->stream);
             if (e == hipSuccess)
-                e = (hipError_t)(fns[k] ? launch_compiled_kernel(r, plans[k], fns[k], r->dargs)
-                                        : launch_table_kernel(r, plans[k],
-                                                              (int)d.slot_type.size(),
-                                                              r->dargs));
+                e = (hipError_t)launch_rounds<R>(r, plans[k], fns[k], (int)d.slot_type.size(),
+                                                 tiles, rounds[(size_t)k]);
             if (e == hipSuccess)
                 e = hipEventRecord(r->ev1, r->stream);
             if (e == hipSuccess)
@@ -1416,6 +1511,7 @@ static int time_kernels(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchPl
         }
     }
     const hipError_t ef = hipFree(scratch);
+    tiles.free_all();
     if (e == hipSuccess)
         e = ef;
     if (e != hipSuccess)
@@ -1531,85 +1627,27 @@ template <typename R>
 static int launch_single(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchPlan &p,
                          uint64_t walker0, uint64_t walkers, uint64_t batch, uint64_t last)
 {
+    MissRounds m;
+    if (records_wanted(r, p, walkers, batch, (int)sizeof(R)))
+        if (const int rc = reserve_records(r, p, walkers, batch, (int)sizeof(R), r->dbuf,
+                                           r->miss_tiles, m))
+            return rc;
     WalkArgs<R> a[2];
     walk_args(r, d, p, walker0, walkers, batch, last, a[0]);
-    // miss records (unless the cache is forced, or indexed directly, where
-    // nothing misses; their memory may be allocated here, so not while the
-    // stream is captured; without it the misses stay atomics)
-    const int words = record_words(walk_nc(r), (int)sizeof(R));
-    MissRounds m;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (p.cache && !p.direct && r->cache_pref < 0 && miss_ok(r) &&
-        (r->miss_pref > 0 ||
-         (miss_worth(r->miss_rate, r->rate_seeded, (int)r->cell_words, (int)sizeof(R), false,
-                     walkers, cached_lanes(r, p)) &&
-          walkers * batch >= kMissMinSamples)) &&
-        hipStreamIsCapturing(r->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
-        if (const int rc = prepare_miss_once())
-            return rc;
-        m = miss_rounds(r->miss_memory, walkers * batch,
-                        (walkers + p.task_walkers - 1) / p.task_walkers, p.grid, p.block, words,
-                        r->miss_rate);
-        hipError_t e = hipSuccess;
-        if (m.rounds)
-            e = r->miss_memory.ensure(p.grid, p.block, m.chunks, words, (int)sizeof(R));
-        if (m.rounds && e == hipSuccess) {
-            MissFlame f{};
-            f.buf = r->dbuf;
-            f.cells = r->cells;
-            f.r = r->spec.color_dims;
-            e = r->miss_tiles.set({f}, f.r > 0 ? kBinTileBitsColour : kBinTileBits, r->stream);
-        }
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            r->miss_memory.free_all();
-            m = MissRounds();
-        }
-    }
-    r->miss_last = m;
-    MissScratch x;
-    if (m.rounds) {
-        x = miss_scratch(r->miss_memory, r->miss_tiles, m.chunks, p.grid, words, (int)sizeof(R),
-                         r->cu_count);
-        a[0].miss = miss_args(x, m.limit);
-        // hints: with records, workgroups seeded alike have no atomics to
-        // queue on (the headline flame misses 3.0 instead of 3.5 %)
-        if (r->dhot && p.slots <= kHotSlots) {
-            a[0].hot = r->dhot;
-            a[0].hot_tag = 0x40000000u | ((unsigned)p.log2s << 8) | (unsigned)p.ways;
-        }
-    }
+    records_args(r, p, r->miss_tiles, m, a);
     // (hints of an earlier render, or of this one's own earlier tasks)
     r->miss_seeded = m.rounds && (r->hot_tag == a[0].hot_tag ||
                                   walkers >= 2 * (uint64_t)p.grid * p.task_walkers);
     if (m.rounds)
         r->hot_tag = a[0].hot_tag;
-    a[1] = a[0];
-    a[1].miss.chunks = 0;
     r->hargs.resize(sizeof a);
     std::memcpy(r->hargs.data(), a, sizeof a);
-    hipError_t e = hipMemcpyAsync(r->dargs, r->hargs.data(), m.last ? sizeof a : sizeof a[0],
-                                  hipMemcpyHostToDevice, r->stream);
+    const hipError_t e = hipMemcpyAsync(r->dargs, r->hargs.data(),
+                                        m.last ? sizeof a : sizeof a[0], hipMemcpyHostToDevice,
+                                        r->stream);
     if (e != hipSuccess)
         return (int)e;
-    // (a compiled flame's kernel reads only the launch part, WalkDyn, at the
-    // start of WalkArgs; its flame fields are constants)
-    auto walk = [&](int k) {
-        const void *args = (const unsigned char *)r->dargs + (size_t)k * sizeof a[0];
-        return r->rtc_fn ? launch_compiled_kernel(r, p, r->rtc_fn, args)
-                         : launch_table_kernel(r, p, (int)d.slot_type.size(), args);
-    };
-    if (!m.rounds)
-        return walk(0);
-    int rc = launch_miss_init(x, p.task_walkers, r->stream);
-    for (int k = 0; k < m.rounds && !rc; ++k) {
-        rc = walk(0);
-        if (!rc)
-            rc = launch_miss_round(x, (int)r->word_bytes, r->stream);
-    }
-    if (!rc && m.last)
-        rc = walk(1);
-    return rc;
+    return launch_rounds<R>(r, p, r->rtc_fn, (int)d.slot_type.size(), r->miss_tiles, m);
 }
 
 // walkers and samples per walker of a render of `samples`
