@@ -83,6 +83,20 @@ struct DevTables {
     int tab_reals = 0;
 };
 
+bool free_idle_records(); // (of the current device, below)
+
+// device memory that a call cannot do without: idle record memory makes way
+template <typename T> hipError_t device_malloc(T **p, size_t bytes)
+{
+    hipError_t e = hipMalloc((void **)p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        if (free_idle_records())
+            e = hipMalloc((void **)p, bytes);
+    }
+    return e;
+}
+
 // grow a device allocation to at least `bytes` (contents not kept)
 hipError_t ensure_device(void **p, size_t &have, size_t bytes)
 {
@@ -91,7 +105,7 @@ hipError_t ensure_device(void **p, size_t &have, size_t bytes)
     (void)hipFree(*p);
     *p = nullptr;
     have = 0;
-    hipError_t e = hipMalloc(p, bytes);
+    hipError_t e = device_malloc(p, bytes);
     if (e == hipSuccess)
         have = bytes;
     return e;
@@ -99,8 +113,8 @@ hipError_t ensure_device(void **p, size_t &have, size_t bytes)
 
 } // namespace
 
-// Miss records: the memory of a renderer's launches (or a batch's: its
-// kinds run one after another)
+// Miss records: the memory of a render's launches (or of a batch's kinds,
+// which run one after another)
 struct MissMemory {
     void *rec = nullptr, *sorted = nullptr, *info = nullptr, *ctrl = nullptr, *state = nullptr;
     size_t rec_bytes = 0, sorted_bytes = 0, info_bytes = 0, ctrl_bytes = 0, state_bytes = 0;
@@ -128,9 +142,176 @@ struct MissMemory {
             (void)hipFree(p);
         *this = MissMemory();
     }
+    size_t bytes() const
+    {
+        return rec_bytes + sorted_bytes + info_bytes + ctrl_bytes + state_bytes;
+    }
 };
 
-// ... and the tiles of its flames
+// The scratch of binned accumulation: of a renderer's binned renders, or of a
+// split one's
+struct BinMemory {
+    BinScratch b;
+    size_t rec = 0, sorted = 0, hist = 0, total = 0, start = 0, pay = 0, pay_sorted = 0; // bytes
+
+    // what the arrays take for `cap` records of ncol colours
+    static BinMemory sizes(uint64_t cells, int ncol, uint64_t cap, int real_bytes)
+    {
+        const int tile_bits = ncol > 0 ? kBinTileBitsColour : kBinTileBits;
+        const size_t ntiles = (size_t)((cells + (1ull << tile_bits) - 1) >> tile_bits);
+        BinMemory n;
+        n.rec = (size_t)cap * 4;
+        n.hist = bin_scratch_hist_words(cap, (int)ntiles) * 4;
+        // per tile: records, then the first accumulation work item; the regions
+        n.total = n.start = 2 * (ntiles + 1) * 4;
+        if (ncol == 0) {
+            n.sorted = n.rec;
+        } else {
+            // the records' colours, component i at i * capacity, and the
+            // whole records in tile order
+            n.pay = (size_t)ncol * (size_t)cap * (size_t)real_bytes;
+            n.pay_sorted = (size_t)cap * (size_t)(4 * record_words(ncol, real_bytes));
+        }
+        return n;
+    }
+    size_t bytes() const { return rec + sorted + hist + total + start + pay + pay_sorted; }
+    // the bytes that ensure(n) would allocate
+    size_t growth(const BinMemory &n) const
+    {
+        auto more = [](size_t have, size_t need) { return need > have ? need : 0; };
+        return more(rec, n.rec) + more(sorted, n.sorted) + more(hist, n.hist) +
+               more(total, n.total) + more(start, n.start) + more(pay, n.pay) +
+               more(pay_sorted, n.pay_sorted);
+    }
+    // grown as needed
+    hipError_t ensure(const BinMemory &n, uint64_t cap)
+    {
+        b.capacity = 0;
+        hipError_t e = ensure_device((void **)&b.rec, rec, n.rec);
+        if (e == hipSuccess)
+            e = ensure_device((void **)&b.sorted, sorted, n.sorted);
+        if (e == hipSuccess)
+            e = ensure_device((void **)&b.hist, hist, n.hist);
+        if (e == hipSuccess)
+            e = ensure_device((void **)&b.total, total, n.total);
+        if (e == hipSuccess)
+            e = ensure_device((void **)&b.start, start, n.start);
+        if (e == hipSuccess)
+            e = ensure_device(&b.pay, pay, n.pay);
+        if (e == hipSuccess)
+            e = ensure_device(&b.pay_sorted, pay_sorted, n.pay_sorted);
+        if (e == hipSuccess)
+            b.capacity = cap;
+        return e;
+    }
+    void free_all()
+    {
+        for (void *p : {(void *)b.rec, (void *)b.sorted, (void *)b.hist, (void *)b.total,
+                        (void *)b.start, b.pay, b.pay_sorted})
+            (void)hipFree(p);
+        *this = BinMemory();
+    }
+};
+
+// Record memory that a render (or a batch's pass) can do without, lent for
+// the time from its launch to the wait for it.  A device's renderers share
+// what lies idle, and it makes way for any other allocation of the library
+// (device_malloc).
+struct RecordMemory {
+    MissMemory miss;
+    BinMemory split; // split walkers
+    ~RecordMemory()
+    {
+        miss.free_all();
+        split.free_all();
+    }
+    size_t bytes() const { return miss.bytes() + split.bytes(); }
+};
+
+struct RecordPool {
+    // idle memories kept, the last one whatever its size (as many programs
+    // render on several threads as have a memory each)
+    static constexpr size_t kIdle = 4, kIdleBytes = (size_t)16 << 30;
+    std::mutex lock;
+    std::deque<std::unique_ptr<RecordMemory>> idle; // oldest first
+
+    static std::shared_ptr<RecordPool> of_device(int device, bool make = true)
+    {
+        static std::mutex m;
+        static std::map<int, std::weak_ptr<RecordPool>> pools;
+        std::lock_guard<std::mutex> g(m);
+        std::shared_ptr<RecordPool> p = pools[device].lock();
+        if (!p && make) {
+            p = std::make_shared<RecordPool>();
+            pools[device] = p;
+        }
+        return p;
+    }
+    std::unique_ptr<RecordMemory> take()
+    {
+        std::lock_guard<std::mutex> g(lock);
+        if (idle.empty())
+            return std::make_unique<RecordMemory>();
+        std::unique_ptr<RecordMemory> m = std::move(idle.back());
+        idle.pop_back();
+        return m;
+    }
+    void give(std::unique_ptr<RecordMemory> m)
+    {
+        std::deque<std::unique_ptr<RecordMemory>> out; // (freed outside the lock)
+        std::lock_guard<std::mutex> g(lock);
+        size_t bytes = m->bytes();
+        for (const auto &i : idle)
+            bytes += i->bytes();
+        idle.push_back(std::move(m));
+        while (idle.size() > 1 && (idle.size() > kIdle || bytes > kIdleBytes)) {
+            bytes -= idle.front()->bytes();
+            out.push_back(std::move(idle.front()));
+            idle.pop_front();
+        }
+    }
+    bool free_idle()
+    {
+        std::deque<std::unique_ptr<RecordMemory>> out;
+        std::lock_guard<std::mutex> g(lock);
+        out.swap(idle);
+        return !out.empty();
+    }
+};
+
+// a renderer's (or a batch's) loan
+struct RecordLoan {
+    std::shared_ptr<RecordPool> pool;
+    std::unique_ptr<RecordMemory> mem;
+
+    RecordMemory &get()
+    {
+        if (!mem)
+            mem = pool->take();
+        return *mem;
+    }
+    // (nothing that uses the memory runs any more)
+    void give_back()
+    {
+        if (mem)
+            pool->give(std::move(mem));
+    }
+};
+
+namespace {
+
+bool free_idle_records()
+{
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess)
+        return false;
+    const std::shared_ptr<RecordPool> p = RecordPool::of_device(device, false);
+    return p && p->free_idle();
+}
+
+} // namespace
+
+// The tiles of the flames of a launch with miss records
 struct MissTiles {
     void *words = nullptr, *flames = nullptr;
     size_t words_bytes = 0, flames_bytes = 0;
@@ -196,8 +377,8 @@ struct MissRounds {
     bool last = false;
 };
 
-// The record memory (as much again holds the sorted records); at most a
-// sixteenth of the free memory.  The batch of 24 flames (32 GB of records)
+// The record memory (as much again holds the sorted records): at most an
+// eighth of the free memory in all.  The batch of 24 flames (32 GB of records)
 // took 216 ms with 1 GB, 195 with 2, 189 with 4 and 185 with 8; the 4K
 // colour flame (2.4 GB) 57.7, 56.7 and 55.9 ms with 1, 2 and 4
 constexpr size_t kMissBytes = (size_t)4 << 30;
@@ -512,7 +693,7 @@ struct ffr_renderer {
     // (measured by each render)
     int miss_pref = -1;
     int task_rounds = 1; // FFR_TASK_ROUNDS: walkers per lane in a task
-    MissMemory miss_memory;
+    RecordLoan records;
     MissTiles miss_tiles;
     double miss_rate = -1;
     bool rate_seeded = false; // ... by one with seeded caches
@@ -521,15 +702,11 @@ struct ffr_renderer {
     bool last_cached = false; // the last render's misses count (a hashed cache)
     uint64_t last_records = 0; // the last render's misses that became records
     uint32_t last_pauses = 0;  // and the pauses of its workgroups
-    BinScratch bin;
-    size_t bin_pay_bytes = 0;    // bytes of bin.pay
-    size_t bin_sorted_bytes = 0; // bytes of bin.pay_sorted
+    BinMemory bin;
     // a colour flame whose renders missed the cell cache often enough
     // (kBinColourRecords, kBinColourAtomics): its later single renders take
     // binned accumulation (binned -1)
     bool bin_colour = false;
-    size_t bin_hist_words = 0;
-    size_t bin_tiles = 0;
     void *wstate = nullptr;
     size_t wstate_bytes = 0;
     void *dargs_bin = nullptr;
@@ -783,6 +960,7 @@ int ffr_create(const char *flame_json, size_t len, const ffr_options *opt_in,
     r->opt = opt;
     r->device = opt.device;
     r->stage = HostStage::of_device(opt.device);
+    r->records.pool = RecordPool::of_device(opt.device);
     r->mode = opt.precision == FFR_FP64 ? MODE_F64_U64
                                         : (opt.word == FFR_WORD32 ? MODE_F32_U32 : MODE_F32_U64);
     const bool fp32 = opt.precision == FFR_FP32;
@@ -849,7 +1027,7 @@ int ffr_create(const char *flame_json, size_t len, const ffr_options *opt_in,
     r->cell_words = 1u + (uint32_t)r->spec.color_dims;
     r->word_bytes = r->mode == MODE_F32_U32 ? 4u : 8u;
     const size_t bytes = (size_t)r->cells * r->cell_words * r->word_bytes;
-    hipError_t e = hipMalloc(&r->dbuf, bytes);
+    hipError_t e = device_malloc(&r->dbuf, bytes);
     if (e != hipSuccess) {
         ffr_destroy(r.release());
         return fail(FFR_E_DEVICE, "hipMalloc of the " + std::to_string(bytes) +
@@ -913,16 +1091,10 @@ void ffr_destroy(ffr_renderer *r)
     (void)hipFree(r->dargs);
     (void)hipFree(r->dimg);
     (void)hipFree(r->dhot);
-    (void)hipFree(r->bin.rec);
-    (void)hipFree(r->bin.sorted);
-    (void)hipFree(r->bin.hist);
-    (void)hipFree(r->bin.total);
-    (void)hipFree(r->bin.start);
-    (void)hipFree(r->bin.pay);
-    (void)hipFree(r->bin.pay_sorted);
+    r->bin.free_all();
     (void)hipFree(r->wstate);
     (void)hipFree(r->dargs_bin);
-    r->miss_memory.free_all();
+    r->records.give_back();
     r->miss_tiles.free_all();
     for (int k = 0; k < 2; ++k) {
         if (r->pin[k])
@@ -1360,13 +1532,14 @@ static int reserve_records(ffr_renderer *r, const LaunchPlan &p, uint64_t walker
     if (const int rc = prepare_miss_once())
         return rc;
     const int words = record_words(walk_nc(r), real_bytes);
+    MissMemory &mem = r->records.get().miss;
     MissRounds want =
-        miss_rounds(r->miss_memory, walkers * batch,
+        miss_rounds(mem, walkers * batch,
                     (walkers + p.task_walkers - 1) / p.task_walkers, p.grid, p.block, words,
                     r->miss_rate);
     if (!want.rounds)
         return 0;
-    hipError_t e = r->miss_memory.ensure(p.grid, p.block, want.chunks, words, real_bytes);
+    hipError_t e = mem.ensure(p.grid, p.block, want.chunks, words, real_bytes);
     if (e == hipSuccess) {
         MissFlame f{};
         f.buf = buf;
@@ -1376,7 +1549,7 @@ static int reserve_records(ffr_renderer *r, const LaunchPlan &p, uint64_t walker
     }
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        r->miss_memory.free_all();
+        mem.free_all();
         return 0;
     }
     m = want;
@@ -1386,7 +1559,7 @@ static int reserve_records(ffr_renderer *r, const LaunchPlan &p, uint64_t walker
 static MissScratch records_scratch(const ffr_renderer *r, const LaunchPlan &p,
                                    const MissTiles &tiles, const MissRounds &m, int real_bytes)
 {
-    return miss_scratch(r->miss_memory, tiles, m.chunks, p.grid,
+    return miss_scratch(r->records.mem->miss, tiles, m.chunks, p.grid,
                         record_words(walk_nc(r), real_bytes), real_bytes, r->cu_count);
 }
 
@@ -1451,7 +1624,7 @@ static int time_kernels(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchPl
 {
     const uint64_t pb = std::min<uint64_t>(batch, 1024);
     void *scratch = nullptr;
-    HIP_TRY(hipMalloc(&scratch, ffr_buffer_bytes(r)));
+    HIP_TRY(device_malloc(&scratch, ffr_buffer_bytes(r)));
     std::vector<std::vector<unsigned char>> h((size_t)n);
     std::vector<MissRounds> rounds((size_t)n);
     MissTiles tiles;
@@ -1659,48 +1832,6 @@ static void split_samples(const ffr_renderer *r, uint64_t samples, uint64_t &bat
     last = samples - (walkers - 1) * batch;
 }
 
-// the scratch of binned accumulation for `cap` records: grown as needed and
-// kept to ffr_destroy
-static hipError_t ensure_bin_scratch(ffr_renderer *r, uint64_t cap, int real_bytes)
-{
-    const int ncol = r->spec.color_dims;
-    const int tile_bits = ncol > 0 ? kBinTileBitsColour : kBinTileBits;
-    const size_t ntiles = (size_t)((r->cells + (1ull << tile_bits) - 1) >> tile_bits);
-    hipError_t e = hipSuccess;
-    size_t have_rec = (size_t)r->bin.capacity * 4, have_sorted = have_rec;
-    if (have_rec < cap * 4) {
-        e = ensure_device((void **)&r->bin.rec, have_rec, (size_t)cap * 4);
-        if (e == hipSuccess && ncol == 0)
-            e = ensure_device((void **)&r->bin.sorted, have_sorted, (size_t)cap * 4);
-        r->bin.capacity = e == hipSuccess ? cap : 0;
-    }
-    // colour flames: the records' colours, component i at i * capacity, and
-    // the whole records in tile order
-    if (e == hipSuccess && ncol > 0) {
-        const size_t need = (size_t)ncol * (size_t)r->bin.capacity * (size_t)real_bytes;
-        e = ensure_device(&r->bin.pay, r->bin_pay_bytes, need);
-        if (e == hipSuccess)
-            e = ensure_device(&r->bin.pay_sorted, r->bin_sorted_bytes,
-                              (size_t)r->bin.capacity *
-                                  (size_t)(4 * record_words(ncol, real_bytes)));
-    }
-    size_t hist_bytes = r->bin_hist_words * 4;
-    if (e == hipSuccess)
-        e = ensure_device((void **)&r->bin.hist, hist_bytes,
-                          bin_scratch_hist_words(cap, (int)ntiles) * 4);
-    r->bin_hist_words = hist_bytes / 4;
-    // per tile: records, then the first accumulation work item; the regions
-    size_t tile_bytes = r->bin_tiles * 4;
-    if (e == hipSuccess && tile_bytes < 2 * (ntiles + 1) * 4) {
-        size_t t2 = tile_bytes;
-        e = ensure_device((void **)&r->bin.total, tile_bytes, 2 * (ntiles + 1) * 4);
-        if (e == hipSuccess)
-            e = ensure_device((void **)&r->bin.start, t2, 2 * (ntiles + 1) * 4);
-    }
-    r->bin_tiles = e == hipSuccess ? std::max(r->bin_tiles, 2 * (ntiles + 1)) : 0;
-    return e;
-}
-
 // Binned accumulation of one render: passes of `span` iterations of every
 // walker (the walkers' points and stream positions carry over in wstate),
 // each pass writing at most kBinPassRecords records, sorted by tile and
@@ -1723,7 +1854,8 @@ static int launch_binned(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchP
     const uint64_t npass = (batch + span - 1) / span;
     const uint64_t cap = slots * span;
     const int ncol = r->spec.color_dims; // colour components of each record
-    hipError_t e = ensure_bin_scratch(r, cap, (int)sizeof(R));
+    hipError_t e =
+        r->bin.ensure(BinMemory::sizes(r->cells, ncol, cap, (int)sizeof(R)), cap);
     if (e == hipSuccess && npass > 1)
         e = ensure_device(&r->wstate, r->wstate_bytes, (size_t)slots * sizeof(WalkerState<R>));
     size_t args_bytes = r->dargs_bin_n * sizeof(WalkArgs<R>);
@@ -1738,10 +1870,10 @@ static int launch_binned(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchP
     for (uint64_t k = 0; k < npass; ++k) {
         WalkArgs<R> a;
         walk_args(r, d, p, walker0, walkers, batch, last, a);
-        a.rec = r->bin.rec;
+        a.rec = r->bin.b.rec;
         a.wstate = r->wstate;
-        a.pay = r->bin.pay;
-        a.pay_stride = r->bin.capacity;
+        a.pay = r->bin.b.pay;
+        a.pay_stride = r->bin.b.capacity;
         a.it0 = k * span;
         a.it1 = std::min<uint64_t>(batch, a.it0 + span);
         std::memcpy(r->hargs.data() + k * sizeof a, &a, sizeof a);
@@ -1829,7 +1961,7 @@ static int launch_binned(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchP
             use = faster ? fn : nullptr;
             ab = false;
         }
-        rc = launch_bin_accumulate(r->bin, n_rec, r->cells, r->dbuf, (int)r->word_bytes, ncol,
+        rc = launch_bin_accumulate(r->bin.b, n_rec, r->cells, r->dbuf, (int)r->word_bytes, ncol,
                                    (int)sizeof(R), r->stream);
         if (rc)
             return rc;
@@ -1842,6 +1974,22 @@ static int launch_binned(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchP
 static uint64_t split_records(const LaunchPlan &p)
 {
     return (uint64_t)p.grid * kSplitBlock * p.split_len;
+}
+
+// the scratch of a split render: at most an eighth of the free memory
+static hipError_t reserve_split(ffr_renderer *r, const LaunchPlan &p)
+{
+    const BinMemory n = BinMemory::sizes(r->cells, r->spec.color_dims, split_records(p),
+                                         r->mode == MODE_F64_U64 ? 8 : 4);
+    BinMemory &mem = r->records.get().split;
+    const size_t more = mem.growth(n);
+    size_t free_b = 0, total_b = 0;
+    if (more && (hipMemGetInfo(&free_b, &total_b) != hipSuccess || more > free_b / 8))
+        return hipErrorOutOfMemory;
+    const hipError_t e = mem.ensure(n, split_records(p));
+    if (e != hipSuccess)
+        mem.free_all();
+    return e;
 }
 
 // A split render: the split walkers write their records, which are binned
@@ -1862,9 +2010,10 @@ static int launch_split_render(ffr_renderer *r, const DeviceFlame<R> &d, const L
     a[1].split_len = p.split_len;
     a[1].split_log2 = p.split_log2;
     a[1].split_warm = r->split_warm;
-    a[1].rec = r->bin.rec;
-    a[1].pay = r->bin.pay;
-    a[1].pay_stride = r->bin.capacity;
+    const BinScratch &bin = r->records.mem->split.b;
+    a[1].rec = bin.rec;
+    a[1].pay = bin.pay;
+    a[1].pay_stride = bin.capacity;
     r->hargs.resize(sizeof a);
     std::memcpy(r->hargs.data(), a, sizeof a);
     hipError_t e = hipMemcpyAsync(r->dargs, r->hargs.data(), sizeof a, hipMemcpyHostToDevice,
@@ -1883,7 +2032,7 @@ static int launch_split_render(ffr_renderer *r, const DeviceFlame<R> &d, const L
     int rc = launch_walk_any(r->mode, r->spec.dims, L);
     if (rc)
         return rc;
-    rc = launch_bin_accumulate(r->bin, split_records(p), r->cells, r->dbuf, (int)r->word_bytes,
+    rc = launch_bin_accumulate(bin, split_records(p), r->cells, r->dbuf, (int)r->word_bytes,
                                r->spec.color_dims, (int)sizeof(R), r->stream,
                                &r->dstats->split_fail);
     if (rc)
@@ -1906,8 +2055,7 @@ static int launch(ffr_renderer *r, uint64_t samples)
                               cap != hipStreamCaptureStatusNone;
         LaunchShape sh = renderer_shape(r);
         sh.split = 0;
-        if (!captured &&
-            ensure_bin_scratch(r, split_records(p), r->mode == MODE_F64_U64 ? 8 : 4) == hipSuccess) {
+        if (!captured && reserve_split(r, p) == hipSuccess) {
             r->last_split = true;
             r->last_split_segments = walkers << p.split_log2;
             sh.bin = 0;
@@ -1977,6 +2125,7 @@ static int finish(ffr_renderer *r, ffr_stats *out)
     if (r->pending) {
         HIP_TRY(hipStreamSynchronize(r->stream));
         r->pending = false;
+        r->records.give_back();
         DevStats st;
         HIP_TRY(hipMemcpy(&st, r->dstats, sizeof st, hipMemcpyDeviceToHost));
         std::vector<unsigned long long> xf((size_t)std::max(r->nxf, 1));
@@ -2109,6 +2258,11 @@ int ffr_set_stream(ffr_renderer *r, void *hip_stream)
         return fail(FFR_E_ARG, "ffr_set_stream: null renderer");
     if (r->pending)
         return fail(FFR_E_ARG, "ffr_set_stream: a render is pending");
+    if (r->records.mem) { // (of a launch that failed half way)
+        HIP_TRY(hipSetDevice(r->device));
+        HIP_TRY(hipStreamSynchronize(r->stream));
+        r->records.give_back();
+    }
     r->stream = hip_stream ? (hipStream_t)hip_stream : r->own_stream;
     return FFR_OK;
 }
@@ -2180,7 +2334,7 @@ int ffr_add_buffer(ffr_renderer *r, const void *src, size_t bytes)
     const size_t chunk_cells = std::max<size_t>(1, (size_t)(256u << 20) / cell_bytes);
     const size_t chunk = std::min(bytes, chunk_cells * cell_bytes);
     void *tmp = nullptr;
-    HIP_TRY(hipMalloc(&tmp, chunk));
+    HIP_TRY(device_malloc(&tmp, chunk));
     int rc = FFR_OK;
     for (size_t off = 0; off < bytes && rc == FFR_OK; off += chunk) {
         size_t n = std::min(chunk, bytes - off);
@@ -2235,7 +2389,7 @@ int io_init(ffr_renderer *r)
                                           cell_bytes);
     for (int k = 0; k < 2; ++k) {
         HIP_TRY(hipHostMalloc(&r->pin[k], chunk, hipHostMallocDefault));
-        HIP_TRY(hipMalloc(&r->dchunk[k], chunk));
+        HIP_TRY(device_malloc(&r->dchunk[k], chunk));
         HIP_TRY(hipEventCreateWithFlags(&r->io_ev[k], hipEventDisableTiming));
     }
     r->io_chunk = chunk;
@@ -2486,7 +2640,7 @@ int ffr_atomic_rate(int32_t device, uint64_t cells, uint32_t cell_words, uint32_
                                         hipGetErrorString(e));
         return rc == FFR_OK;
     };
-    if (step(hipMalloc(&buf, bytes), "hipMalloc") &&
+    if (step(device_malloc(&buf, bytes), "hipMalloc") &&
         step(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "stream") &&
         step(hipEventCreate(&e0), "event") && step(hipEventCreate(&e1), "event") &&
         step((hipError_t)launch_fill_zero(buf, bytes, s), "clear") &&
@@ -2557,7 +2711,7 @@ int render_image(ffr_renderer *r, int mode, double gamma, int bits, void *dst, s
                 HIP_TRY(hipFree(r->dimg));
                 r->dimg = nullptr;
                 r->dimg_bytes = 0;
-                HIP_TRY(hipMalloc(&r->dimg, need));
+                HIP_TRY(device_malloc(&r->dimg, need));
                 r->dimg_bytes = need;
             }
             out = r->dimg;

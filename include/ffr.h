@@ -65,9 +65,18 @@ typedef struct ffr_options {
      * (under 64 per CU) of a flame whose variations draw no random words,
      * of at most 2^28 samples, split each walker's iterations over many
      * lanes (not colour flames with 4-byte words).  The result is the
-     * unsplit one; scratch memory is allocated as for binned accumulation,
-     * and without it, or while the stream is captured, the walkers run
-     * unsplit. */
+     * unsplit one; without memory for their records, or while the stream
+     * is captured, the walkers run unsplit.
+     * Renders and batched passes of 2^24 samples or more whose samples
+     * often miss the cell cache keep the misses as records that are binned
+     * (not when cell_cache is 0 or 1, nor colour flames with 4-byte words;
+     * the counts are the same, colour sums differ by the rounding of their
+     * order of addition).
+     * The memory of these records (at most an eighth of what is free, 8 GiB
+     * for misses) is lent from the launch to the wait for it.  Up to four
+     * idle loans, 16 GiB in all or the last one, are kept for the device's
+     * renderers, batches and servers together, until the last of them is
+     * destroyed or another allocation of the library needs the room. */
     int32_t cell_cache;
     int32_t cache_kib;
     int32_t block;
@@ -372,7 +381,8 @@ typedef struct ffr_server ffr_server;
 enum { FFR_JOB_QUEUED = 0, FFR_JOB_RUNNING = 1, FFR_JOB_DONE = 2, FFR_JOB_FAILED = 3 };
 
 typedef struct ffr_server_options {
-    uint64_t hbm_budget;   /* bytes of job buffers held at once (0: 200e9)          */
+    uint64_t hbm_budget;   /* bytes of job buffers held at once (0: 200e9); record
+                              memory (ffr_options.cell_cache) is not counted      */
     double pass_ms;        /* target device time of one pass, ms (0: 100)           */
     int32_t device;        /* HIP device ordinal                                    */
     int32_t reserved;
