@@ -500,13 +500,23 @@ static int prepare_miss_once()
 // the link moves others: 1.9 ms for 66 MB either way (8 threads of 2 MB
 // chunks; 2.3 with 6 or 12 of 1 MB, 3.2 of 0.5 MB).  One per device, shared by its
 // renderers and given back with the last of them; a copy that finds it in
-// use takes the runtime's.
+// use takes the runtime's.  By size, the runtime's copy against this one
+// (ms): reads 0.46 / 0.37 of 8 MiB, 0.9-1.3 / 0.6 of 16, 3.1 / 1.2 of 32, 4.8
+// / 1.5 of 48; writes 0.24 / 0.33, 0.45 / 0.54, 0.98 / 0.94, 1.7 / 1.4.  The
+// first copy also pays 1 to 2.5 ms for the pinned memory, so it is made
+// for a copy that wins them back, or once earlier ones would have.  Memory
+// that the caller pinned takes the link by itself (0.16 / 0.36 ms of 8 MiB,
+// 2.3 / 3.4 of 128).
 struct HostStage {
     static constexpr int kThreads = 8, kSlots = 2;
     static constexpr size_t kChunk = (size_t)2 << 20;
-    static constexpr size_t kMinBytes = (size_t)8 << 20; // (smaller: the threads' start)
+    static constexpr size_t kReadBytes = (size_t)8 << 20;
+    static constexpr size_t kWriteBytes = (size_t)48 << 20;
+    // bytes of copies beyond kReadBytes each from which on it is made
+    static constexpr size_t kFirstBytes = (size_t)40 << 20;
     std::mutex busy;
     bool ready = false;
+    size_t asked = 0; // bytes of the copies so far beyond kReadBytes each
     char *pin = nullptr;
     hipEvent_t ev[kThreads * kSlots] = {};
 
@@ -521,6 +531,13 @@ struct HostStage {
             stages[device] = p;
         }
         return p;
+    }
+    // made, or worth it with this copy
+    bool wanted(size_t bytes)
+    {
+        if (!ready)
+            asked += bytes - kReadBytes;
+        return ready || asked >= kFirstBytes;
     }
     hipError_t init()
     {
@@ -2278,16 +2295,27 @@ size_t ffr_buffer_bytes(const ffr_renderer *r)
 int32_t ffr_dims(const ffr_renderer *r) { return r ? r->spec.dims : 0; }
 int32_t ffr_color_dims(const ffr_renderer *r) { return r ? r->spec.color_dims : 0; }
 
+// memory that the caller pinned
+static bool host_pinned(const void *p)
+{
+    hipPointerAttribute_t at{};
+    const bool known = hipPointerGetAttributes(&at, p) == hipSuccess;
+    if (!known)
+        (void)hipGetLastError();
+    return known && at.type != hipMemoryTypeUnregistered;
+}
+
 // a copy of a renderer's memory to or from the host, after its stream's work
 static hipError_t host_copy(ffr_renderer *r, void *host, void *dev, size_t bytes, bool to_host)
 {
     // (a captured stream refuses the wait below, and takes no copies)
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (bytes >= HostStage::kMinBytes && hipStreamIsCapturing(r->stream, &cap) == hipSuccess &&
-        cap == hipStreamCaptureStatusNone) {
+    if (bytes >= (to_host ? HostStage::kReadBytes : HostStage::kWriteBytes) &&
+        hipStreamIsCapturing(r->stream, &cap) == hipSuccess &&
+        cap == hipStreamCaptureStatusNone && !host_pinned(host)) {
         HostStage &st = *r->stage;
         std::unique_lock<std::mutex> g(st.busy, std::try_to_lock);
-        if (g.owns_lock()) {
+        if (g.owns_lock() && st.wanted(bytes)) {
             if (st.init() == hipSuccess)
                 return st.copy(r->device, r->stream, host, dev, bytes, to_host);
             (void)hipGetLastError();
