@@ -336,7 +336,8 @@ typedef struct ffr_batch_stats {
     double kernel_ms;    /* device time of the batch (HIP events around it)      */
     uint64_t samples;    /* samples rendered                                     */
     uint64_t tasks;      /* workgroup tasks                                      */
-    uint32_t launches;   /* walker-kernel launches (kernel kinds)                */
+    uint32_t launches;   /* walker-kernel launches: one per kernel kind, more
+                            where its misses are binned between them          */
     uint32_t graph;      /* 1 when the launches ran as a replayed HIP graph      */
 } ffr_batch_stats;
 

@@ -48,3 +48,24 @@ def test_colour_counts_share_a_kind(ffr_mod, precision, colours, kinds):
             assert np.all(np.abs(ca - cb) <= n * 2.0 ** -52 * np.abs(cb))
         a.close()
         b.close()
+
+
+def test_launches_are_counted(ffr_mod, monkeypatch):
+    """one per kind, and those of the rounds of miss records"""
+    print("batch launches", flush=True)
+    monkeypatch.setenv("FFR_MISS", "0")
+    rs = [ffr_mod.BufferRenderer(flame(1069, c, 1000), precision="fp32", seed=1, batch_size=256)
+          for c in (0, 3)]
+    n = 30000 * 256
+    with ffr_mod.Batch(rs) as batch:
+        assert all(batch.render([n, n])) and batch.last_stats.launches == 2
+    monkeypatch.setenv("FFR_MISS", "1")
+    with_records = [ffr_mod.BufferRenderer(flame(1069, c, 1000), precision="fp32", seed=1,
+                                           batch_size=256) for c in (0, 3)]
+    with ffr_mod.Batch(with_records) as batch:
+        assert all(batch.render([n, n])) and batch.last_stats.launches == 2  # a round each
+        monkeypatch.setenv("FFR_MISS_BYTES", str(1 << 22))
+        assert all(batch.render([n, n]))
+        assert any(r.record_use[1] for r in with_records) and batch.last_stats.launches > 4
+    for r in rs + with_records:
+        r.close()
