@@ -422,8 +422,9 @@ static MissRounds miss_rounds(const MissMemory &mem, uint64_t samples, uint64_t 
 {
     const uint64_t chunk = miss_chunk(words), chunk_bytes = chunk * (uint64_t)words * 4;
     const uint64_t waves = ((uint64_t)lanes + 63) / 64;
-    // a wave ends each task, and each launch, with a chunk that is partly filled
-    const uint64_t all = samples / chunk + (tasks + (uint64_t)groups) * waves + 1;
+    // (a wave begins a chunk in each task; a launch whose chunks were used up
+    // would leave walkers paused)
+    const uint64_t all = miss_chunks_most(samples, (tasks + (uint64_t)groups) * waves, words);
     uint64_t bytes = kMissBytes;
     if (const char *e = std::getenv("FFR_MISS_BYTES"))
         bytes = std::max<uint64_t>((uint64_t)std::atoll(e), 2 * chunk_bytes);

@@ -89,6 +89,14 @@ struct MissFlame {
     int r;
     int pad;
 };
+// The most chunks that waves fill with `records` records in `runs` runs, each
+// of which begins a chunk: a wave takes the next one when an iteration's
+// records (64 at most) have no room, so that a chunk it leaves holds all but
+// 63 of its records or more, or is its run's last.
+constexpr uint64_t miss_chunks_most(uint64_t records, uint64_t runs, int words)
+{
+    return records / (miss_chunk(words) - 63u) + runs;
+}
 // the device arrays of a launch's miss records
 struct MissScratch {
     unsigned *rec = nullptr;    // [chunks][miss_chunk] records of `words` words
