@@ -82,32 +82,32 @@ C5_3D_SAMPLES = 1 << 30
 C5_CHUNKS = 4
 C5_BUDGET = 200_000_000_000
 HBM_PEAK_GBS = 8000.0
-# walker kernel HBM bytes per launch on the headline workload, from two
-# counter runs (FETCH_SIZE, then WRITE_SIZE, KiB per dispatch, the timed
-# step's dispatch): FP32 (native trajectories, table-driven kernel) FETCH
-# 901.125 x 2.0 + WRITE 18719063.3125 x 1.0; FP64 (the flame's compiled
-# kernel, which the probe keeps) FETCH 1001.1875 x 2.0 + WRITE
-# 18871357.5625 x 1.0.  The factors come from kernels of known traffic on
-# the same buffer (the add reads 2 x 265420800 B and reports 259236 KiB of
-# FETCH_SIZE, the histogram pass reads the buffer once and reports half of
-# it; the clear and the add each write 265420800 B and report exactly
-# 259200 KiB of WRITE_SIZE).  Global atomics count 32 B each in WRITE_SIZE.
-# The raw values are in profiles/walk_kernel_random_color_3840x2160_hbm.md.
-C2_FP32_TRAFFIC_BYTES = 901.125 * 1024 * 2.0 + 18719063.3125 * 1024 * 1.0
-C2_FP64_TRAFFIC_BYTES = 1001.1875 * 1024 * 2.0 + 18871357.5625 * 1024 * 1.0
+# HBM bytes per render on the headline workload, walker launches and the
+# binning of their miss records together, from two counter runs (FETCH_SIZE,
+# then WRITE_SIZE, KiB, summed over the dispatches of a renderer's third
+# render; the flame's compiled kernels, which the probes keep): FP32 FETCH
+# 4364729.375 x 2.0 + WRITE 7428390.5 x 1.0 (records); FP64, whose misses stay
+# atomics, FETCH 1031.9375 x 2.0 + WRITE 18882665.15625 x 1.0.  The factors
+# come from kernels of known traffic on the same buffer (the add reads 2 x
+# 265420800 B and reports 259236 KiB of FETCH_SIZE, the histogram pass reads
+# the buffer once and reports half of it; the clear and the add each write
+# 265420800 B and report exactly 259200 KiB of WRITE_SIZE).  Global atomics
+# count 32 B each in WRITE_SIZE.  The raw values are in
+# profiles/walk_kernel_random_color_3840x2160_records.md.
+C2_FP32_TRAFFIC_BYTES = 4364729.375 * 1024 * 2.0 + 7428390.5 * 1024 * 1.0
+C2_FP64_TRAFFIC_BYTES = 1031.9375 * 1024 * 2.0 + 18882665.15625 * 1024 * 1.0
 # HBM bytes of one binned tetrahedron render (32 passes of 2^28 records):
 # per pass walker 1.10 GB, tile histogram 1.09, column scan 0.03, scatter
 # 2.53, tile accumulation 1.11 (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0)
 C3_BINNED_TRAFFIC_BYTES = 32 * 5.86e9
-# VALU instructions (SQ_INSTS_VALU, wave64) per headline launch of 2^32
+# VALU instructions (SQ_INSTS_VALU, wave64) per headline render of 2^32
 # samples, by precision and kernel (table-driven or the flame's compiled
-# one), from counter runs of the same launches
-# (profiles/walk_kernel_random_color_3840x2160_valu.md); the compiled FP32
-# kernel was counted only on 2^29-sample runs (x 8 here).  The VALU peak is
+# one), from counter runs of the same renders, their binning included
+# (profiles/walk_kernel_random_color_3840x2160_records.md).  The VALU peak is
 # one wave64 instruction per 4 cycles per SIMD (16 lanes a cycle, FP32 and
 # FP64 alike on this device): 256 CUs x 4 SIMDs x 2.4 GHz / 4.
-C2_VALU_PER_LAUNCH = {("fp32", False): 35077692829, ("fp32", True): 4069185530 * 8,
-                      ("fp64", False): 51868535255, ("fp64", True): 46629032406}
+C2_VALU_PER_LAUNCH = {("fp32", False): 33001778736, ("fp32", True): 29631699561,
+                      ("fp64", False): 43810419448, ("fp64", True): 40724111981}
 VALU_PEAK_G = 256 * 4 * 2.4 / 4
 
 
@@ -185,11 +185,19 @@ def image_leg(ffr, r, words, cpu):
 _atomic_peak = {}
 
 
-def atomic_roofline(ffr, atomics, kernel_ms, cells, cell_words, word_bytes, flush_atomics=None):
+def atomic_adds(r):
+    """the last render's global atomic adds: the words of updates past the
+    cell cache, without those that became records"""
+    return int(r.last_stats.atomics) - r.record_use[0] * r.cell_words
+
+
+def atomic_roofline(ffr, atomics, kernel_ms, cells, cell_words, word_bytes, flush_atomics=None,
+                    records=0):
     """The walker kernel's global atomic adds per second (counted by the
-    kernel: misses of the LDS cell cache and its flushes) against the rate
-    the device sustains for cell updates scattered uniformly over a buffer
-    of the same shape (ffr_atomic_rate, 2^28 cell updates)."""
+    kernel: misses of the LDS cell cache and its flushes; not the misses
+    that became records) against the rate the device sustains for cell
+    updates scattered uniformly over a buffer of the same shape
+    (ffr_atomic_rate, 2^28 cell updates)."""
     key = (cells, cell_words, word_bytes)
     if key not in _atomic_peak:
         _atomic_peak[key] = ffr.atomic_rate(cells, cell_words, word_bytes, 1 << 28)
@@ -197,6 +205,7 @@ def atomic_roofline(ffr, atomics, kernel_ms, cells, cell_words, word_bytes, flus
     achieved = atomics / (kernel_ms * 1e-3) / 1e9
     out = {"achieved": achieved, "peak": peak, "unit": "G atomics/s",
            "frac": achieved / peak if peak > 0 else None, "atomics_per_launch": atomics,
+           "records_per_launch": records,
            "peak_buffer": f"{cells} cells x {cell_words} words of {word_bytes} B"}
     if flush_atomics is not None:
         # the LDS cache's flushes, reported apart: one 32-B atomic per word
@@ -222,7 +231,7 @@ def run_gpu(ffr, text, *, precision, samples, steps, warmup, bytes_per_plot, see
         kms.append(r.kernel_ms)
     t1 = time.perf_counter()
     plotted = (r.samples_plotted - plot0) / steps
-    atomics = int(r.last_stats.atomics)
+    atomics, records = atomic_adds(r), r.record_use[0]
     flush_atomics = int(r.last_stats.flush_atomics)
     wall = t1 - t0
     kavg = sum(kms) / len(kms)
@@ -245,7 +254,7 @@ def run_gpu(ffr, text, *, precision, samples, steps, warmup, bytes_per_plot, see
             "traffic": None,
         },
         "atomic_roofline": atomic_roofline(ffr, atomics, kavg, r.cells, r.cell_words,
-                                           r.word_bytes, flush_atomics),
+                                           r.word_bytes, flush_atomics, records),
     }
     hist = None
     if keep:
@@ -305,7 +314,8 @@ def run_batch(ffr, texts, samples, precision, keep, seed0=C4_SEED):
         raise RuntimeError("a batched flame stopped at the bad-value limit")
     st = b.last_stats
     plotted = sum(r.samples_plotted for r in rs)
-    atomics = sum(int(r.last_stats.atomics) for r in rs)
+    atomics = sum(atomic_adds(r) for r in rs)
+    records = sum(r.record_use[0] for r in rs)
     flush_atomics = sum(int(r.last_stats.flush_atomics) for r in rs)
     big = max(rs, key=lambda r: r.cells)
     hists = None
@@ -335,7 +345,8 @@ def run_batch(ffr, texts, samples, precision, keep, seed0=C4_SEED):
         },
         # priced at the largest flame's buffer shape (most of the samples)
         "atomic_roofline": atomic_roofline(ffr, atomics, st.kernel_ms, big.cells,
-                                           big.cell_words, big.word_bytes, flush_atomics),
+                                           big.cell_words, big.word_bytes, flush_atomics,
+                                           records),
     }
     b.close()
     for r in rs:
