@@ -47,3 +47,22 @@ def test_the_choice_is_kept(ffr_mod, flame, kept):
 def test_launches_that_do_not_fill_the_device(ffr_mod, precision, flame, samples, records):
     print(f"miss line {precision} {flame} {samples}", flush=True)
     assert uses(ffr_mod, flame, samples, len(records), precision=precision) == records
+
+
+def test_a_tuned_batch_knows_its_misses(ffr_mod):
+    """two flames of 0.44 and 0.48 words in FP64, where a batch takes records
+    from 0.75 on: a first pass that knows nothing takes them"""
+    print("miss line of a tuned batch", flush=True)
+    for tuned in (False, True):
+        rs = [ffr_mod.BufferRenderer(read_flame("batch/flame_%d.json" % k), precision="fp64",
+                                     seed=k) for k in (1048, 1040)]
+        samples = [1 << 27] * 2
+        with ffr_mod.Batch(rs) as batch:
+            if tuned:
+                batch.tune(samples, 1.0 / 8)
+            assert all(batch.render(samples))
+            assert all((r.record_use[0] == 0) == tuned for r in rs)
+            assert all(batch.render(samples))
+            assert all(r.record_use[0] == 0 for r in rs)
+        for r in rs:
+            r.close()
