@@ -229,11 +229,11 @@ struct RecordMemory {
 };
 
 struct RecordPool {
-    // idle memories kept, the last one whatever its size (as many programs
-    // render on several threads as have a memory each)
+    // idle memories kept, the last one whatever its size (several for
+    // programs that render on several threads)
     static constexpr size_t kIdle = 4, kIdleBytes = (size_t)16 << 30;
     std::mutex lock;
-    std::deque<std::unique_ptr<RecordMemory>> idle; // oldest first
+    std::vector<std::unique_ptr<RecordMemory>> idle; // oldest first
 
     static std::shared_ptr<RecordPool> of_device(int device, bool make = true)
     {
@@ -258,7 +258,7 @@ struct RecordPool {
     }
     void give(std::unique_ptr<RecordMemory> m)
     {
-        std::deque<std::unique_ptr<RecordMemory>> out; // (freed outside the lock)
+        std::vector<std::unique_ptr<RecordMemory>> out; // (freed outside the lock)
         std::lock_guard<std::mutex> g(lock);
         size_t bytes = m->bytes();
         for (const auto &i : idle)
@@ -267,12 +267,12 @@ struct RecordPool {
         while (idle.size() > 1 && (idle.size() > kIdle || bytes > kIdleBytes)) {
             bytes -= idle.front()->bytes();
             out.push_back(std::move(idle.front()));
-            idle.pop_front();
+            idle.erase(idle.begin());
         }
     }
     bool free_idle()
     {
-        std::deque<std::unique_ptr<RecordMemory>> out;
+        std::vector<std::unique_ptr<RecordMemory>> out;
         std::lock_guard<std::mutex> g(lock);
         out.swap(idle);
         return !out.empty();
