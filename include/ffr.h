@@ -87,12 +87,14 @@ typedef struct ffr_options {
      * for flames without colour whose buffer has at least 2^22 and under
      * 2^28 cells when the lane-per-walker kernel runs, and for a colour
      * flame once a render of 2^26 samples or more had 1.9 words per sample
-     * of updates past the cell cache (0.6 with 4-byte words); 0 off; 1 on where the flame allows it: under
-     * 2^28 cells without colour, under 2^25 with up to four colours).
+     * of updates past the cell cache (0.6 with 4-byte words); 0 off; 1 on
+     * where the flame allows it: under 2^28 cells without colour, under
+     * 2^25 with up to four colours).
      * Counts are the same either way; colour sums differ by the rounding
      * of their order of addition.  The first binned render allocates the
      * pass scratch, kept to ffr_destroy: up to 2 GiB of records, and for
-     * colour flames up to 6 GiB (three FP32 colours) or 12 GiB (FP64). */
+     * colour flames up to 8 GiB (three FP32 colours), 15 GiB (FP64) or
+     * 21 GiB (four FP64 colours). */
     int32_t binned;
     /* the flame compiled into its own kernel (no counterpart in the
      * reference, whose flame is objects with virtual calls): the walker code
@@ -103,7 +105,9 @@ typedef struct ffr_options {
      * renders again after its renders have asked for 2^33 samples in all,
      * on a scratch buffer for the lane kernel, on the render's first two
      * passes for the binned walker; 0 off; 1 on).  Results equal the
-     * table-driven kernel's bit for bit. */
+     * table-driven kernel's bit for bit, but for FP32 flames with some
+     * trigonometric variations (handkerchief, julian, blob), whose run-time
+     * compiled functions round otherwise in places. */
     int32_t compiled;
     int32_t reserved;
 } ffr_options;
