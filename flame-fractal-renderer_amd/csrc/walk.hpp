@@ -302,10 +302,10 @@ __host__ __device__ constexpr bool chain_build_sh(bool shared, bool post_id, int
 }
 
 // the colour registers a walker kernel is built for: none; exactly three
-// (2-D flames of the basic variations, set 1); up to four; more
+// (2-D flames of the basic variations, sets 1 and 3); up to four; more
 constexpr int nc_class(int r, int vs)
 {
-    return r == 0 ? 0 : r == 3 && vs == 1 ? 3 : r <= 4 ? 4 : 128;
+    return r == 0 ? 0 : r == 3 && (vs == 1 || vs == 3) ? 3 : r <= 4 ? 4 : 128;
 }
 
 #ifndef __HIPCC_RTC__
