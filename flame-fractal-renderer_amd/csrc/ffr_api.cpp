@@ -216,7 +216,10 @@ struct BinMemory {
 // Record memory that a render (or a batch's pass) can do without, lent for
 // the time from its launch to the wait for it.  A device's renderers share
 // what lies idle, and it makes way for any other allocation of the library
-// (device_malloc).
+// (device_malloc).  One idle memory outlives the last of them (kKeepBytes):
+// the driver wipes freed memory in the background, and a program that makes
+// a renderer per flame, frees gigabytes with each and has gone through the
+// device's memory once waits 0.1 to 1 s in an allocation for that.
 struct RecordMemory {
     MissMemory miss;
     BinMemory split; // split walkers
@@ -229,22 +232,24 @@ struct RecordMemory {
 };
 
 struct RecordPool {
-    // idle memories kept, the last one whatever its size (several for
-    // programs that render on several threads)
+    // idle memories kept while there are renderers, the last one whatever its
+    // size (several for programs that render on several threads)
     static constexpr size_t kIdle = 4, kIdleBytes = (size_t)16 << 30;
+    // the largest that is kept after them (miss records take 8 GiB)
+    static constexpr size_t kKeepBytes = (size_t)10 << 30;
+    using Idle = std::vector<std::unique_ptr<RecordMemory>>; // oldest first
     std::mutex lock;
-    std::vector<std::unique_ptr<RecordMemory>> idle; // oldest first
+    Idle idle;
 
-    static std::shared_ptr<RecordPool> of_device(int device, bool make = true)
+    // a device's, for the life of the process
+    static RecordPool *of_device(int device)
     {
-        static std::mutex m;
-        static std::map<int, std::weak_ptr<RecordPool>> pools;
-        std::lock_guard<std::mutex> g(m);
-        std::shared_ptr<RecordPool> p = pools[device].lock();
-        if (!p && make) {
-            p = std::make_shared<RecordPool>();
-            pools[device] = p;
-        }
+        static std::mutex *m = new std::mutex;
+        static std::map<int, RecordPool *> *pools = new std::map<int, RecordPool *>;
+        std::lock_guard<std::mutex> g(*m);
+        RecordPool *&p = (*pools)[device];
+        if (!p)
+            p = new RecordPool;
         return p;
     }
     std::unique_ptr<RecordMemory> take()
@@ -258,7 +263,7 @@ struct RecordPool {
     }
     void give(std::unique_ptr<RecordMemory> m)
     {
-        std::vector<std::unique_ptr<RecordMemory>> out; // (freed outside the lock)
+        Idle out; // (freed outside the lock)
         std::lock_guard<std::mutex> g(lock);
         size_t bytes = m->bytes();
         for (const auto &i : idle)
@@ -270,9 +275,20 @@ struct RecordPool {
             idle.erase(idle.begin());
         }
     }
+    // the last renderer, batch and server are gone
+    void rest()
+    {
+        Idle out;
+        std::lock_guard<std::mutex> g(lock);
+        out.swap(idle);
+        if (!out.empty() && out.back()->bytes() <= kKeepBytes) {
+            idle.push_back(std::move(out.back()));
+            out.pop_back();
+        }
+    }
     bool free_idle()
     {
-        std::vector<std::unique_ptr<RecordMemory>> out;
+        Idle out;
         std::lock_guard<std::mutex> g(lock);
         out.swap(idle);
         return !out.empty();
@@ -281,20 +297,36 @@ struct RecordPool {
 
 // a renderer's (or a batch's) loan
 struct RecordLoan {
-    std::shared_ptr<RecordPool> pool;
+    // held by every renderer and batch of a device
+    struct Users {
+        RecordPool *pool;
+        ~Users() { pool->rest(); }
+    };
+    std::shared_ptr<Users> users;
     std::unique_ptr<RecordMemory> mem;
 
+    void open(int device)
+    {
+        static std::mutex *m = new std::mutex;
+        static std::map<int, std::weak_ptr<Users>> *all = new std::map<int, std::weak_ptr<Users>>;
+        std::lock_guard<std::mutex> g(*m);
+        users = (*all)[device].lock();
+        if (!users) {
+            users.reset(new Users{RecordPool::of_device(device)});
+            (*all)[device] = users;
+        }
+    }
     RecordMemory &get()
     {
         if (!mem)
-            mem = pool->take();
+            mem = users->pool->take();
         return *mem;
     }
     // (nothing that uses the memory runs any more)
     void give_back()
     {
         if (mem)
-            pool->give(std::move(mem));
+            users->pool->give(std::move(mem));
     }
 };
 
@@ -303,10 +335,7 @@ namespace {
 bool free_idle_records()
 {
     int device = 0;
-    if (hipGetDevice(&device) != hipSuccess)
-        return false;
-    const std::shared_ptr<RecordPool> p = RecordPool::of_device(device, false);
-    return p && p->free_idle();
+    return hipGetDevice(&device) == hipSuccess && RecordPool::of_device(device)->free_idle();
 }
 
 } // namespace
@@ -978,7 +1007,7 @@ int ffr_create(const char *flame_json, size_t len, const ffr_options *opt_in,
     r->opt = opt;
     r->device = opt.device;
     r->stage = HostStage::of_device(opt.device);
-    r->records.pool = RecordPool::of_device(opt.device);
+    r->records.open(opt.device);
     r->mode = opt.precision == FFR_FP64 ? MODE_F64_U64
                                         : (opt.word == FFR_WORD32 ? MODE_F32_U32 : MODE_F32_U64);
     const bool fp32 = opt.precision == FFR_FP32;
@@ -2251,6 +2280,13 @@ int ffr_record_use(const ffr_renderer *r, uint64_t *records, uint32_t *pauses)
         *records = r->last_records;
     if (pauses)
         *pauses = r->last_pauses;
+    return FFR_OK;
+}
+
+int ffr_free_idle(int32_t device)
+{
+    HIP_TRY(hipSetDevice(device));
+    (void)RecordPool::of_device(device)->free_idle();
     return FFR_OK;
 }
 

@@ -147,7 +147,8 @@ IMG_MONO, IMG_GRAY, IMG_COLOR = 0, 1, 2
 # every symbol include/ffr.h declares
 EXPORTS = [
     "ffr_default_options", "ffr_create", "ffr_destroy", "ffr_last_error",
-    "ffr_render", "ffr_render_async", "ffr_sync", "ffr_record_use", "ffr_set_stream",
+    "ffr_render", "ffr_render_async", "ffr_sync", "ffr_record_use", "ffr_free_idle",
+    "ffr_set_stream",
     "ffr_device_buffer", "ffr_buffer_cells", "ffr_cell_words", "ffr_word_bytes",
     "ffr_buffer_bytes", "ffr_dims", "ffr_color_dims", "ffr_read_buffer",
     "ffr_add_buffer", "ffr_add_buffer_noalloc", "ffr_write_buffer", "ffr_clear_buffer",
@@ -211,6 +212,7 @@ def lib():
     L.ffr_xform_distribution.argtypes = [P, C.POINTER(C.c_uint64), C.c_size_t]
     L.ffr_xform_id_count.restype = C.c_size_t
     L.ffr_xform_id_count.argtypes = [P]
+    L.ffr_free_idle.argtypes = [C.c_int32]
     L.ffr_record_use.argtypes = [P, C.POINTER(C.c_uint64), C.POINTER(C.c_uint32)]
     L.ffr_bad_values.argtypes = [P, C.POINTER(C.c_uint64), C.POINTER(C.c_double),
                                  C.c_size_t, C.POINTER(C.c_size_t)]
@@ -283,6 +285,12 @@ def check_flame(text: str, precision: str = "fp64"):
     prec = FFR_FP32 if precision == "fp32" else FFR_FP64
     _check(L.ffr_check_flame(b, len(b), prec, ids, cw, cap, C.byref(n)))
     return [ids[i] for i in range(n.value)], [cw[i] for i in range(n.value)]
+
+
+def free_idle(device: int = 0):
+    """Free the device's idle record memory (what renders with miss records or
+    split walkers borrow)."""
+    _check(lib().ffr_free_idle(device))
 
 
 def atomic_rate(cells: int, cell_words: int = 4, word_bytes: int = 8,

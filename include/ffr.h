@@ -75,8 +75,9 @@ typedef struct ffr_options {
      * The memory of these records (at most an eighth of what is free, 8 GiB
      * for misses) is lent from the launch to the wait for it.  Up to four
      * idle loans, 16 GiB in all or the last one, are kept for the device's
-     * renderers, batches and servers together, until the last of them is
-     * destroyed or another allocation of the library needs the room. */
+     * renderers, batches and servers together, and one of at most 10 GiB
+     * after the last of them is destroyed; an allocation of the library
+     * that needs the room frees them, and so does ffr_free_idle. */
     int32_t cell_cache;
     int32_t cache_kib;
     int32_t block;
@@ -178,6 +179,10 @@ int ffr_sync(ffr_renderer *r, ffr_stats *stats);
  * often a workgroup paused because the record memory was used up.  No
  * counterpart in the reference.  Either pointer may be NULL. */
 int ffr_record_use(const ffr_renderer *r, uint64_t *records, uint32_t *pauses);
+
+/* free the idle record memory of a device (ffr_options.cell_cache), for a
+ * program that wants it for something else */
+int ffr_free_idle(int32_t device);
 
 /* launch on a caller-owned hipStream_t (NULL: the renderer's own stream) */
 int ffr_set_stream(ffr_renderer *r, void *hip_stream);

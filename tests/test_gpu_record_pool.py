@@ -1,7 +1,7 @@
 """Record memory that renders can do without (miss records, split walkers) is
 lent for a render: a device's renderers, batches and servers share it, it
-makes way for an allocation that a call needs, and goes with the last of
-them."""
+makes way for an allocation that a call needs, one of at most 10 GiB stays
+after the last of them, and free_idle frees it."""
 
 import ctypes as C
 import json
@@ -45,6 +45,7 @@ def test_renderers_share_it(ffr_mod, render):
     print(f"record pool {render.__name__}", flush=True)
     after = []
     for _ in range(3):
+        ffr_mod.free_idle()
         free, rs, held = free_memory(ffr_mod), [], []
         for k in range(5):
             rs.append(render(ffr_mod, k))
@@ -53,9 +54,27 @@ def test_renderers_share_it(ffr_mod, render):
         assert held[0] > GB and held[-1] < 1.1 * held[0], held
         for r in rs:
             r.close()
+        assert free - free_memory(ffr_mod) < 10 * GB + (256 << 20)
+        ffr_mod.free_idle()
         after.append(free_memory(ffr_mod))
     # (the runtime keeps a few MB per stream from the first time on)
     assert after[1] - after[2] < 64 << 20, after
+
+
+def test_it_outlives_the_last_renderer(ffr_mod):
+    """a program that makes one renderer after another does not allocate and
+    free gigabytes with each"""
+    print("record pool of renderers in turn", flush=True)
+    for _ in range(2):
+        with_records(ffr_mod, 0).close()
+    idle = free_memory(ffr_mod)
+    for k in range(3):
+        r = with_records(ffr_mod, k)
+        assert idle - free_memory(ffr_mod) < r.cells * r.cell_words * r.word_bytes + (64 << 20)
+        r.close()
+        assert abs(idle - free_memory(ffr_mod)) < 64 << 20
+    ffr_mod.free_idle()
+    assert free_memory(ffr_mod) - idle > 4 * GB
 
 
 def test_batches_share_it(ffr_mod):
