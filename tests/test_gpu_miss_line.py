@@ -35,12 +35,15 @@ def test_the_choice_is_kept(ffr_mod, flame, kept):
 
 
 @pytest.mark.parametrize("precision, flame, samples, records", [
-    ("fp32", 1069, 1 << 26, [False, True, True]),    # 2.4 words, a quarter of the lanes
+    ("fp32", 1069, 1 << 26, [True, True, True]),     # 2.4 words, a quarter of the lanes
+    ("fp32", 1082, 1 << 26, [True, False, False]),   # 0.43
+    ("fp32", 1069, 1 << 25, [False, True, True]),    # 2.4, an eighth
     ("fp32", 1017, 1 << 25, [False, False, False]),  # 0.86, an eighth
     ("fp32", 1082, 1 << 27, [True, True, True]),     # 0.44, half
     ("fp32", 1000, 1 << 27, [True, False, False]),   # 0.22, half
     ("fp64", 1017, 1 << 25, [False, False, False]),  # 0.84, a quarter
-    ("fp64", 1069, 1 << 26, [False, True, True]),    # 2.4, half
+    ("fp64", 1069, 1 << 26, [True, True, True]),     # 2.4, half
+    ("fp64", 1069, 1 << 25, [False, True, True]),    # 2.4, a quarter
     ("fp64", 1241, 1 << 27, [True, True, True]),     # 0.34, all
     ("fp64", 1166, 1 << 27, [True, False, False]),   # 0.16, all
 ])
