@@ -182,3 +182,22 @@ def test_bad_value_limit_with_records_waiting(ffr_mod, monkeypatch, small):
     assert r.last_stats.n_bad > 300 and r.record_use[0] > 0
     assert r.histogram_stats()[0] == r.samples_plotted
     r.close()
+
+
+@pytest.mark.parametrize("compiled", [0, 1])
+@pytest.mark.parametrize("mode", ["fp32", "fp64"])
+@pytest.mark.parametrize("name", ["basic_c3", "basic_c1", "basic_c4", "basic_many_xforms"])
+def test_binned_records(ffr_mod, monkeypatch, name, mode, compiled):
+    """binned accumulation of the basic variations, in passes of 2^20 records"""
+    print(f"binned records {name} {mode} compiled={compiled}", flush=True)
+    text = FLAMES[name]()
+    b = make(ffr_mod, monkeypatch, text, False, compiled=0, **MODES[mode])
+    monkeypatch.setenv("FFR_BIN_PASS_RECORDS", str(1 << 20))
+    a = ffr_mod.BufferRenderer(text, seed=SEED, batch_size=BATCH, binned=1, compiled=compiled,
+                               **MODES[mode])
+    for _ in range(2):
+        assert a.render(SAMPLES) and b.render(SAMPLES)
+        assert a.last_stats.binned == 1 and a.last_stats.compiled == compiled
+        same_buffers(a, b)
+    a.close()
+    b.close()
