@@ -433,19 +433,14 @@ constexpr size_t kMissBytes = (size_t)4 << 30;
 constexpr uint64_t kMissMinSamples = 1ull << 24;
 constexpr double kMissWords32 = 0.13, kMissWords64 = 0.3, kMissWordsBatch64 = 0.75;
 constexpr double kMissWordsUnknown = 0.6;
-// a single render with records seeds its caches alike (hints) and misses
-// 0.74 to 0.86 of what it misses without
-constexpr double kMissSeeded = 0.8;
 
-// rate: of the last render's samples those that missed (negative: unknown),
-// with seeded caches or without
-static bool miss_worth(double rate, bool seeded, int cell_words, int real_bytes, bool batch,
+// rate: the share of the samples that missed (negative: unknown)
+static bool miss_worth(double rate, int cell_words, int real_bytes, bool batch,
                        uint64_t walkers, uint64_t lanes)
 {
     const double least =
         real_bytes == 4 ? kMissWords32 : batch && rate >= 0 ? kMissWordsBatch64 : kMissWords64;
-    const double words =
-        rate < 0 ? kMissWordsUnknown : rate * cell_words / (seeded ? kMissSeeded : 1.0);
+    const double words = rate < 0 ? kMissWordsUnknown : rate * cell_words;
     return words >= least * std::max(1.0, (double)lanes / (double)std::max<uint64_t>(walkers, 1));
 }
 
@@ -746,9 +741,13 @@ struct ffr_renderer {
     RecordLoan records;
     MissTiles miss_tiles;
     double miss_rate = -1;
-    bool rate_seeded = false; // ... by one with seeded caches
-    bool miss_seeded = false; // the last render's caches were seeded
-    unsigned hot_tag = 0;     // of the hints that single renders left
+    // ... without hints (records_args), by log2 of the render's samples
+    // (negative: not measured), and of the latest such render; seeded caches
+    // miss 0.75 to 0.9 of that, by flame and by run (the 4K colour flame 0.75
+    // to 0.88), too wide a range to judge one by the other
+    std::vector<double> plain_rates = std::vector<double>(64, -1.0);
+    double plain_last = -1;
+    int plain_class = -1; // of a render without hints that runs: its log2
     bool last_cached = false; // the last render's misses count (a hashed cache)
     uint64_t last_records = 0; // the last render's misses that became records
     uint32_t last_pauses = 0;  // and the pauses of its workgroups
@@ -1556,6 +1555,19 @@ static bool miss_ok(const ffr_renderer *r)
            r->cells < (ncol > 0 ? (1ull << 25) : (1ull << 28));
 }
 
+// The share of a render's samples that its launch would miss without hints,
+// as far as earlier renders tell
+static int rate_class(uint64_t samples)
+{
+    return 63 - __builtin_clzll(samples | 1);
+}
+
+static double plain_rate(const ffr_renderer *r, uint64_t samples)
+{
+    const double known = r->plain_rates[rate_class(samples)];
+    return known >= 0 ? known : r->plain_last;
+}
+
 // ... and are taken by a launch of enough walkers and samples that miss
 // enough (not where the cache is forced, or indexed directly, so that
 // nothing misses; their memory may be allocated, so not while the stream is
@@ -1566,7 +1578,7 @@ static bool records_wanted(const ffr_renderer *r, const LaunchPlan &p, uint64_t 
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     return p.cache && !p.direct && r->cache_pref < 0 && miss_ok(r) &&
            (r->miss_pref > 0 ||
-            (miss_worth(r->miss_rate, r->rate_seeded, (int)r->cell_words, real_bytes, false,
+            (miss_worth(plain_rate(r, walkers * batch), (int)r->cell_words, real_bytes, false,
                         walkers, cached_lanes(r, p)) &&
              walkers * batch >= kMissMinSamples)) &&
            hipStreamIsCapturing(r->stream, &cap) == hipSuccess &&
@@ -1613,17 +1625,19 @@ static MissScratch records_scratch(const ffr_renderer *r, const LaunchPlan &p,
                         record_words(walk_nc(r), real_bytes), real_bytes, r->cu_count);
 }
 
-// the arguments of a lane-per-walker render: its walker launches', and those
-// of the last one, which has no record memory
+// the arguments of a lane-per-walker render of `samples`: its walker
+// launches', and those of the last one, which has no record memory
 template <typename R>
 static void records_args(const ffr_renderer *r, const LaunchPlan &p, const MissTiles &tiles,
-                         const MissRounds &m, WalkArgs<R> (&a)[2])
+                         const MissRounds &m, uint64_t samples, WalkArgs<R> (&a)[2])
 {
     if (m.rounds) {
         a[0].miss = miss_args(records_scratch(r, p, tiles, m, (int)sizeof(R)), m.limit);
         // hints: with records, workgroups seeded alike have no atomics to
-        // queue on (the headline flame misses 3.0 instead of 3.5 %)
-        if (r->dhot && p.slots <= kHotSlots) {
+        // queue on (the headline flame misses 3.0 instead of 3.5 %), once a
+        // render of this size went without (55.9 instead of 55.2 ms) and
+        // left the rate that its records are judged by
+        if (r->dhot && p.slots <= kHotSlots && r->plain_rates[rate_class(samples)] >= 0) {
             a[0].hot = r->dhot;
             a[0].hot_tag = 0x40000000u | ((unsigned)p.log2s << 8) | (unsigned)p.ways;
         }
@@ -1697,7 +1711,7 @@ static int time_kernels(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchPl
         walk_args(r, d, plans[k], walker0, walkers, pb, pb, a[0]);
         a[0].buf = scratch;
         a[0].bv_limit = ~0ull; // the runs never stop at the bad-value limit
-        records_args(r, plans[k], tiles, rounds[(size_t)k], a);
+        records_args(r, plans[k], tiles, rounds[(size_t)k], walkers * batch, a);
         h[(size_t)k].resize(sizeof a);
         std::memcpy(h[(size_t)k].data(), a, sizeof a);
     }
@@ -1857,12 +1871,8 @@ static int launch_single(ffr_renderer *r, const DeviceFlame<R> &d, const LaunchP
             return rc;
     WalkArgs<R> a[2];
     walk_args(r, d, p, walker0, walkers, batch, last, a[0]);
-    records_args(r, p, r->miss_tiles, m, a);
-    // (hints of an earlier render, or of this one's own earlier tasks)
-    r->miss_seeded = m.rounds && (r->hot_tag == a[0].hot_tag ||
-                                  walkers >= 2 * (uint64_t)p.grid * p.task_walkers);
-    if (m.rounds)
-        r->hot_tag = a[0].hot_tag;
+    records_args(r, p, r->miss_tiles, m, walkers * batch, a);
+    r->plain_class = a[0].hot ? -1 : rate_class(walkers * batch);
     r->hargs.resize(sizeof a);
     std::memcpy(r->hargs.data(), a, sizeof a);
     const hipError_t e = hipMemcpyAsync(r->dargs, r->hargs.data(),
@@ -2207,9 +2217,10 @@ static int finish(ffr_renderer *r, ffr_stats *out)
         }
         r->last_bad = st.n_bad;
         if (r->last_cached && st.s_iter) {
-            r->rate_seeded = r->miss_seeded;
             r->miss_rate = (double)(st.atomics - st.flush_atomics) / (double)r->cell_words /
                            (double)st.s_iter;
+            if (r->plain_class >= 0)
+                r->plain_last = r->plain_rates[r->plain_class] = r->miss_rate;
         }
         r->last_atomics = st.atomics;
         r->last_flush_atomics = st.flush_atomics;
